@@ -67,23 +67,22 @@ OCC_BYTES = 1  # shadow query result
 # pcg32 state (8), sample index (4), film position (8), scene byte (1) and
 # a queue entry (4); the first-hit stage reads the queue
 # entry, hit and direction and writes radiance and a material-queue entry;
-# a shading vertex reads its queue entry, hit, direction, throughput,
-# aux, pcg32 state and sample index (a path's first vertex: not
-# throughput and aux, which are implied) and writes the shadow ray's
-# direction and its NEE term, the continuation ray (whose origin the shadow
-# ray shares), throughput,
-# pcg32 state, aux and two queue entries (radiance only when an emitter
-# sample that casts no shadow ray adds to it); its post-processing
-# reads aux, radiance, NEE term, occlusion byte, throughput, hit, direction,
-# pcg32 state and sample index and writes radiance, aux, throughput, pcg32
-# state and a queue entry; the film gather reads each sample's position and
-# radiance once and writes a pixel per 64 samples.
+# a shading vertex reads its queue entry, hit, direction, throughput, pcg32
+# state and sample index (a path's first vertex: not the throughput, which
+# is implied) and writes the shadow ray's direction and its NEE term, the
+# continuation ray (whose origin the shadow ray shares), throughput, pcg32
+# state, aux and two queue entries (radiance only when an emitter sample
+# that casts no shadow ray adds to it); its post-processing reads its queue
+# entry and hit and writes a queue entry (misses, emitter hits and Russian
+# roulette touch more, and an unoccluded shadow ray adds its NEE term to the
+# radiance: not counted, so the sum is a lower bound); the film gather reads
+# each sample's position and radiance once and writes a pixel per 64 samples.
 PATH_STATE_BYTES = {"raygen": 2 * 16 + 8 + 4 + 8 + 1 + 4,                     # 57
                     "first_hit": 4 + 2 * 16 + 16 + 4,                          # 56
-                    "shade": (4 + 4 * 16 + 8 + 4) + (6 * 16 + 8 + 2 * 4),      # 80 read + 112 written
-                    "post": (4 + 6 * 16 + 1 + 8 + 4) + (3 * 16 + 8 + 4),       # 113 read + 60 written
+                    "shade": (4 + 3 * 16 + 8 + 4) + (5 * 16 + 8 + 8 + 2 * 4),  # 64 read + 104 written
+                    "post": (4 + 16) + 4,                                      # 20 read + 4 written
                     "film": 8 + 16 + 16 / 64.0,
-                    "first_vertex_skip": 2 * 16}                               # per path: an undercount
+                    "first_vertex_skip": 16}                                   # per path: an undercount
 TRACE_KERNEL = "k_trace_queue<false>"
 COPY_KERNEL = "k_copy"
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_trace_queue_%s_traffic.json" % WORKLOAD)
@@ -156,7 +155,7 @@ def path_bytes(agg, bytes_closest, bytes_shadow):
     paths = agg["paths"]
     vertices = agg["closest_rays"] - paths
     trav = (agg["closest_rays"] * (bytes_closest + 4) + agg["shadow_rays"] * (bytes_shadow + 4)) / paths
-    # the throughput and aux a first shading vertex does not read are taken
+    # the throughput a first shading vertex does not read is taken
     # off once per path, also for paths that never reach one (so the sum is
     # a lower bound)
     state = (paths * (PATH_STATE_BYTES["raygen"] + PATH_STATE_BYTES["first_hit"] + PATH_STATE_BYTES["film"] -

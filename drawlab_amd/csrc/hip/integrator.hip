@@ -37,9 +37,10 @@ namespace dl {
 constexpr int kStageBlock = 256;
 constexpr int kTypes = 8;  // material queue segments (DL_BSDF_COUNT rounded up)
 
+// kFlagDiffuse: the vertex the continuation left has a non-delta BSDF.
 // kFlagCamera: the continuation is still the camera ray (it passed through
 // a hidden light), so its next hit or miss is treated as the first one.
-enum : uint32_t { kFlagDiffuse = 1u, kFlagNee = 2u, kFlagCont = 4u, kFlagCamera = 8u };
+enum : uint32_t { kFlagDiffuse = 1u, kFlagCamera = 2u };
 // Material-queue segment of paths that pass straight through a hidden
 // light's surface (after the BSDF types).
 constexpr int kPassQ = DL_BSDF_COUNT;
@@ -49,10 +50,8 @@ struct Counters {
     uint32_t mat[2][kTypes];
     uint32_t ray;     // continuation rays queued (block_append index 0)
     uint32_t shadow;  // shadow rays queued (block_append index 1)
-    uint32_t work_ray;     // rays claimed by the closest-hit traversal
-    uint32_t work_shadow;  // rays claimed by the shadow traversal
-    uint32_t emit;         // continuations that hit an emitter (k_post -> k_post_emit)
-    uint32_t pad[11];
+    uint32_t emit;    // continuations that hit an emitter (k_post -> k_post_emit)
+    uint32_t pad[13];
     unsigned long long nodes;
     unsigned long long tris;
     unsigned long long invalid;
@@ -64,16 +63,19 @@ struct Counters {
 struct RenderBufs {
     float4 *ray_o, *ray_d, *hit, *sh_d;  // a shadow ray starts at ray_o
     float4 *thr, *rad, *nee;
-    int4* aux;
+    uint2* aux;    // the previous vertex's sampling pdf (bits) and flags
+    int2* depth;   // depth and 1 + training record slot: passes whose paths differ in depth (hidden
+                   // lights let them pass through) or that record; elsewhere every path of a bounce
+                   // has the bounce's depth and the array is not touched
     uint64_t* rng;
     uint32_t* seq;  // sample index of the path (its pcg32 stream selector)
     float2* pos;
-    uint8_t* occ;
     uint32_t* matq[2];
     uint32_t* rayq;
     uint32_t* shq;
     uint32_t* emq;  // paths whose continuation hit an emitter (MIS-weighted emission pending)
     Counters* cnt;
+    uint32_t* work;  // work counters of the closest-hit, then of the shadow traversal (trace.h)
     float4* film;
     float* rgb;
     float* gmix;  // guided rendering: mixture (40 floats) per entry of the queue being shaded
@@ -161,30 +163,6 @@ __device__ __forceinline__ void block_append(uint32_t* counters, const uint32_t 
 __device__ __forceinline__ vec3 f3(const float4& a) { return v3(a.x, a.y, a.z); }
 __device__ __forceinline__ float4 f4(vec3 a, float w) { return make_float4(a.x, a.y, a.z, w); }
 
-// Locate entry i of the concatenated per-type queues.
-__device__ __forceinline__ bool queue_entry(const uint32_t* counts, const uint32_t* q, uint32_t cap, uint32_t i,
-                                            uint32_t& path, int& type) {
-    uint32_t base = 0;
-#pragma unroll
-    for (int t = 0; t < kTypes; t++) {
-        const uint32_t c = counts[t];
-        if (i < base + c) {
-            path = q[(size_t)t * cap + (i - base)];
-            type = t;
-            return true;
-        }
-        base += c;
-    }
-    return false;
-}
-
-__device__ __forceinline__ uint32_t queue_total(const uint32_t* counts) {
-    uint32_t s = 0;
-#pragma unroll
-    for (int t = 0; t < kTypes; t++) s += counts[t];
-    return s;
-}
-
 // Learned proposal during a pass: mixtures of the queue being shaded,
 // training records (nullptr: not training) and the scene bounds.
 struct GuideView {
@@ -211,16 +189,16 @@ struct PassParams {
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kStageBlock) void k_reset(Counters* cnt, int next) {
+__global__ __launch_bounds__(kStageBlock) void k_reset(Counters* cnt, uint32_t* work, int next) {
     const int t = threadIdx.x;
     if (t < kTypes) cnt->mat[next][t] = 0;
     if (t == 0) {
         cnt->ray = 0;
         cnt->shadow = 0;
-        cnt->work_ray = 0;
-        cnt->work_shadow = 0;
         cnt->emit = 0;
     }
+    static_assert(2 * kWorkGroups <= kStageBlock, "a thread per work counter");
+    if (t < 2 * (int)kWorkGroups) work[t * kWorkStride] = 0;
 }
 
 __global__ __launch_bounds__(kStageBlock) void k_reset_all(Counters* cnt) {
@@ -320,7 +298,8 @@ struct QueueIO {
     const float4* __restrict__ ro;
     const float4* __restrict__ rd;
     float4* __restrict__ hit;
-    uint8_t* __restrict__ occ;
+    const float4* __restrict__ nee;
+    float4* __restrict__ rad;
     const uint8_t* __restrict__ sid;
     const int32_t* __restrict__ roots;
     // a refill loads the queue entry and then the ray it names (8 measured
@@ -341,18 +320,29 @@ struct QueueIO {
                                               uint32_t) const {
         hit[p] = make_float4(__uint_as_float(prim), t, u, v);
     }
-    __device__ __forceinline__ void store_occ(uint32_t p, bool o, uint32_t, uint32_t) const { occ[p] = o ? 1 : 0; }
+    // an unoccluded shadow ray adds its emitter sample to the path's radiance
+    // (one shadow ray per path and bounce, and nothing else touches the
+    // radiance meanwhile)
+    static constexpr bool kResolve = true;
+    __device__ __forceinline__ void resolve_load(uint32_t p, float4& c, float4& r) const {
+        c = nee[p];
+        r = rad[p];
+    }
+    __device__ __forceinline__ void resolve_store(uint32_t p, const float4& c, const float4& r) const {
+        rad[p] = f4(add(f3(r), f3(c)), 0.f);
+    }
+    __device__ __forceinline__ void store_occ(uint32_t, bool, uint32_t, uint32_t) const {}
 };
 
 template <bool COUNT>
-__global__ __launch_bounds__(kTraceBlock) void k_trace_queue(BvhView bvh, RenderBufs rs, int* __restrict__ ovf) {
+__global__ __launch_bounds__(kTraceBlock, COUNT ? 4 : 8) void k_trace_queue(BvhView bvh, RenderBufs rs, int* __restrict__ ovf) {
     __shared__ int lds[kLdsStack * kTraceBlock];
     const uint32_t n = rs.cnt->ray;
     const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x, G = gridDim.x * kTraceBlock;
     LaneStack stk{lds, (int)threadIdx.x, kTraceBlock, ovf + g, G};
-    QueueIO io{rs.rayq, rs.ray_o, rs.ray_d, rs.hit, nullptr, rs.sid, rs.roots};
+    QueueIO io{rs.rayq, rs.ray_o, rs.ray_d, rs.hit, nullptr, nullptr, rs.sid, rs.roots};
     TraceCounters cnt;
-    traverse_persistent<false, COUNT>(bvh, n, &rs.cnt->work_ray, stk, io, cnt);
+    traverse_persistent<false, COUNT>(bvh, trace_work(rs.work, n), stk, io, cnt);
     if (COUNT) {
         wave_add(&rs.cnt->nodes, cnt.nodes);
         wave_add(&rs.cnt->tris, cnt.tris);
@@ -360,14 +350,14 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_queue(BvhView bvh, Render
 }
 
 template <bool COUNT>
-__global__ __launch_bounds__(kTraceBlock) void k_shadow_queue(BvhView bvh, RenderBufs rs, int* __restrict__ ovf) {
+__global__ __launch_bounds__(kTraceBlock, COUNT ? 4 : 8) void k_shadow_queue(BvhView bvh, RenderBufs rs, int* __restrict__ ovf) {
     __shared__ int lds[kLdsStack * kTraceBlock];
     const uint32_t n = rs.cnt->shadow;
     const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x, G = gridDim.x * kTraceBlock;
     LaneStack stk{lds, (int)threadIdx.x, kTraceBlock, ovf + g, G};
-    QueueIO io{rs.shq, rs.ray_o, rs.sh_d, nullptr, rs.occ, rs.sid, rs.roots};
+    QueueIO io{rs.shq, rs.ray_o, rs.sh_d, nullptr, rs.nee, rs.rad, rs.sid, rs.roots};
     TraceCounters cnt;
-    traverse_persistent<true, COUNT>(bvh, n, &rs.cnt->work_shadow, stk, io, cnt);
+    traverse_persistent<true, COUNT>(bvh, trace_work(rs.work + kWorkGroups * kWorkStride, n), stk, io, cnt);
     if (COUNT) {
         wave_add(&rs.cnt->nodes_sh, cnt.nodes);
         wave_add(&rs.cnt->tris_sh, cnt.tris);
@@ -430,7 +420,8 @@ __global__ __launch_bounds__(kStageBlock) void k_post_camera(PassParams pp, Scen
                     const uint32_t info = prim_info(s, prim);
                     if (HIDE && info_light(info)) {
                         rs.thr[p] = make_float4(1.f, 1.f, 1.f, 1.f);
-                        rs.aux[p] = make_int4(0, (int)(kFlagCont | kFlagCamera), 0, 0);
+                        rs.aux[p] = make_uint2(0u, kFlagCamera);
+                        rs.depth[p] = make_int2(0, 0);
                         alive = true;
                         type = kPassQ;
                     } else {
@@ -484,9 +475,6 @@ __global__ __launch_bounds__(kStageBlock) void k_pass(PassParams pp, SceneView s
                 const float4 h = rs.hit[p];
                 Its its;
                 make_its(s, __float_as_uint(h.x), h.z, h.w, false, its);
-                int4 aux = rs.aux[p];
-                aux.y = (int)(((uint32_t)aux.y & (kFlagDiffuse | kFlagCamera)) | kFlagCont);
-                rs.aux[p] = aux;
                 rs.ray_o[p] = f4(its.p, pp.eps);
                 rs.ray_d[p] = f4(f3(rs.ray_d[p]), INFINITY);
             }
@@ -527,7 +515,7 @@ __global__ __launch_bounds__(kStageBlock) void k_normals(SceneView s, RenderBufs
 // type), so each carries only its own BSDF's code and registers.
 template <int TYPE, bool GUIDED>
 __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView s, RenderBufs rs, int cur,
-                                                       GuideView gv, bool first) {
+                                                       GuideView gv, bool first, bool track) {
     const uint32_t n = rs.cnt->mat[cur][TYPE];
     const uint32_t* __restrict__ queue = rs.matq[cur] + (size_t)TYPE * pp.cap;
     constexpr int type = TYPE;
@@ -548,13 +536,11 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
                 const uint32_t prim = __float_as_uint(h.x);
                 const vec3 d = f3(rs.ray_d[p]);
                 // the first shading vertex of a camera path: throughput 1,
-                // eta 1, aux 0 (not stored by k_raygen)
+                // eta 1, depth 0 (not stored by k_raygen)
                 float4 th4 = make_float4(1.f, 1.f, 1.f, 1.f);
-                int4 aux = make_int4(0, 0, 0, 0);
-                if (!first) {
-                    th4 = rs.thr[p];
-                    aux = rs.aux[p];
-                }
+                if (!first) th4 = rs.thr[p];
+                int2 dep = make_int2(0, 0);
+                if (track && !first) dep = rs.depth[p];
                 vec3 thr = f3(th4);
                 float eta = th4.w;
                 Pcg32 rng;
@@ -604,7 +590,6 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
                     if (csum(spectrum) > 0) {
                         rs.nee[p] = f4(contrib, 0.f);
                         rs.sh_d[p] = f4(ds.d, ds.dist - pp.eps);  // from ray_o, written below
-                        flags |= kFlagNee;
                         want_shadow = true;
                     } else {
                         // (the path's radiance is read and written only here:
@@ -659,14 +644,13 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
                 if (want_shadow || !is_zero(thr)) rs.ray_o[p] = f4(its.p, pp.eps);
                 if (!is_zero(thr)) {
                     rs.ray_d[p] = f4(to_world(its.sh, br.wo), INFINITY);
-                    flags |= kFlagCont;
                     want_cont = true;
                 }
-                aux.w = 0;
+                dep.y = 0;
                 if (GUIDED && gv.rec && want_cont && guide_material(type, prm)) {
                     // training record of this vertex (its radiance before the
                     // continuation is completed by k_post)
-                    const uint32_t depth = (uint32_t)aux.z;
+                    const uint32_t depth = (uint32_t)dep.x;
                     const uint32_t slot = (p / gv.rec_stride) * kGRecDepth + depth;
                     if (depth < (uint32_t)kGRecDepth && p % gv.rec_stride == 0 && slot < gv.rec_cap) {
                         float* r = gv.rec + (size_t)slot * kGRecFloats;
@@ -690,14 +674,13 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
                         r[kRecThr + 2] = thr.z;
                         r[kRecPath] = __uint_as_float(p);
                         r[kRecValid] = 1.0f;
-                        aux.w = (int)slot + 1;
+                        dep.y = (int)slot + 1;
                     }
                 }
                 rs.thr[p] = f4(thr, eta);
                 rs.rng[p] = rng.state;
-                aux.x = __float_as_int(prev_pdf);
-                aux.y = (int)flags;
-                rs.aux[p] = aux;
+                rs.aux[p] = make_uint2(__float_as_uint(prev_pdf), flags);
+                if (track) rs.depth[p] = dep;
             }
             s_p[u][threadIdx.x] = p;
             s_b[u][threadIdx.x] = (want_cont ? 1u : 0u) | (want_shadow ? 2u : 0u);
@@ -728,8 +711,8 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
 // The lanes of a wave that call it together take consecutive queue slots
 // with one atomic (the queue's order does not matter: each entry is one
 // path's own emission).
-__device__ __forceinline__ void defer_emission(const RenderBufs& rs, uint32_t p, vec3 thr, int light) {
-    rs.nee[p] = f4(thr, __int_as_float(light));
+__device__ __forceinline__ void defer_emission(const RenderBufs& rs, uint32_t p, vec3 thr) {
+    rs.nee[p] = f4(thr, 0.f);
     const unsigned long long mask = __ballot(1);
     const int lane = __lane_id();
     const int leader = __ffsll((long long)mask) - 1;
@@ -748,10 +731,10 @@ __global__ __launch_bounds__(kStageBlock) void k_post_emit(SceneView s, RenderBu
         const float4 h = rs.hit[p];
         const uint32_t prim = __float_as_uint(h.x);
         const float4 t4 = rs.nee[p];
-        const int light = __float_as_int(t4.w);
-        const int4 aux = rs.aux[p];
-        const float prev_pdf = __int_as_float(aux.x);
-        const bool diffuse = ((uint32_t)aux.y & kFlagDiffuse) != 0;
+        const int light = light_of(s, prim);
+        const uint2 aux = rs.aux[p];
+        const float prev_pdf = __uint_as_float(aux.x);
+        const bool diffuse = (aux.y & kFlagDiffuse) != 0;
         const vec3 o = f3(rs.ray_o[p]);
         const vec3 d = f3(rs.ray_d[p]);
         vec3 hp, hn;
@@ -765,114 +748,126 @@ __global__ __launch_bounds__(kStageBlock) void k_post_emit(SceneView s, RenderBu
     }
 }
 
+// What a traced continuation leads to, for every entry of the ray queue: a
+// miss adds the environment, an emitter hit is queued for k_post_emit,
+// Russian roulette and the depth cap end paths, and the survivors are sorted
+// into the material queues of the next bounce.  (The radiance already holds
+// the bounce's emitter sample: the shadow traversal added it.)  `depth`: the
+// depth of every path of the bounce (HIDE: each path's own).
+// It is bound by memory traffic (176 bytes read per vertex when it resolved
+// the emitter samples itself and went through every shaded path's state:
+// 3.2 ms of a 512x512x64 Cornell box): a block first fetches the path index, hit primitive
+// and primitive class of all its items in three rounds of independent loads,
+// and only misses, emitter hits and roulette touch the path's other state.
 // HIDE: light surfaces are hidden (hitgroup_pgs.cu:55-64): a path ray that
 // hits one collects its emission as usual, unless it is still the camera
 // ray, and passes through (queue kPassQ) without a bounce; a camera ray that
 // passed through is treated as the camera ray at its next hit or miss.
 template <bool HIDE>
-__global__ __launch_bounds__(kStageBlock) void k_post(PassParams pp, SceneView s, RenderBufs rs, int cur,
+__global__ __launch_bounds__(kStageBlock) void k_post(PassParams pp, SceneView s, RenderBufs rs, int next, int depth,
                                                       float* __restrict__ grec) {
-    // the lengths of the queues being read, loaded once: the counters'
-    // cache line takes every block's appends to the next queues meanwhile
-    uint32_t counts[kTypes];
-#pragma unroll
-    for (int t = 0; t < kTypes; t++) counts[t] = rs.cnt->mat[cur][t];
-    const uint32_t n = queue_total(counts);
-    const int next = cur ^ 1;
+    // read once: the counters' cache line takes every block's appends to the
+    // next queues meanwhile
+    const uint32_t n = rs.cnt->ray;
+    constexpr uint32_t kMiss = 0x100u;  // an item's class: prim_info, or a miss, or no item
+    constexpr uint32_t kNone = 0x200u;
     __shared__ uint32_t s_p[kStageItems][kStageBlock];
     __shared__ uint32_t s_b[kStageItems][kStageBlock];
     const uint32_t items = stage_items(n);
     for (uint32_t i0 = blockIdx.x * items * kStageBlock; i0 < n; i0 += gridDim.x * items * kStageBlock) {
-        // items are staged in LDS (each thread reads back only its own) so the
-        // per-item body is not unrolled
+        {
+            uint32_t p[kStageItems], prim[kStageItems];
+#pragma unroll
+            for (int u = 0; u < kStageItems; u++) {
+                const uint32_t i = (uint32_t)u < items ? i0 + (uint32_t)u * kStageBlock + threadIdx.x : n;
+                p[u] = i < n ? rs.rayq[i] : 0xffffffffu;
+            }
+#pragma unroll
+            for (int u = 0; u < kStageItems; u++)
+                prim[u] = p[u] != 0xffffffffu ? __float_as_uint(rs.hit[p[u]].x) : 0xffffffffu;
+#pragma unroll
+            for (int u = 0; u < kStageItems; u++) {
+                s_p[u][threadIdx.x] = p[u];
+                s_b[u][threadIdx.x] = prim[u] != 0xffffffffu ? prim_info(s, prim[u])
+                                      : p[u] != 0xffffffffu  ? kMiss
+                                                             : kNone;
+            }
+        }
+        // the class of each item (each thread's own in LDS, so that the
+        // per-item body is not unrolled) becomes the bit of its next queue
 #pragma unroll 1
         for (int u = 0; u < kStageItems; u++) {
-            const uint32_t i = (uint32_t)u < items ? i0 + (uint32_t)u * kStageBlock + threadIdx.x : n;
+            const uint32_t info = s_b[u][threadIdx.x];
+            const uint32_t p = s_p[u][threadIdx.x];
             bool alive = false;
             int ntype = 0;
-            uint32_t p = 0;
-            if (i < n) {
-                int type;
-                queue_entry(counts, rs.matq[cur], pp.cap, i, p, type);
-                int4 aux = rs.aux[p];
-                const uint32_t flags = (uint32_t)aux.y;
-                vec3 rad = f3(rs.rad[p]);
-                if ((flags & kFlagNee) && rs.occ[p] == 0) rad = add(rad, f3(rs.nee[p]));
-                if (grec && aux.w > 0) {
-                    // radiance before the continuation of a recorded vertex
-                    float* r = grec + (size_t)(aux.w - 1) * kGRecFloats;
-                    r[kRecRad] = rad.x;
-                    r[kRecRad + 1] = rad.y;
-                    r[kRecRad + 2] = rad.z;
-                }
-                if (flags & kFlagCont) {
-                    const float4 th4 = rs.thr[p];
-                    vec3 thr = f3(th4);
-                    const float eta = th4.w;
-                    const float prev_pdf = __int_as_float(aux.x);
-                    const bool diffuse = (flags & kFlagDiffuse) != 0;
-                    const float4 h = rs.hit[p];
-                    const uint32_t prim = __float_as_uint(h.x);
-                    const vec3 d = f3(rs.ray_d[p]);
-                    const bool cam = HIDE && (flags & kFlagCamera) != 0;
-                    if (prim == 0xffffffffu) {
-                        const SceneRec sc = path_scene(s, p);
-                        if (sc.env_light >= 0) {
-                            const LightRec& e = s.lights[sc.env_light];
-                            if (cam) {
-                                rad = add(rad,
-                                          mul(thr, e.env_visual ? env_eval(s, e, d) : v3(sc.bg[0], sc.bg[1], sc.bg[2])));
-                            } else {
-                                float epdf;
-                                const vec3 ev = env_eval_pdf(s, e, sc.num_lights, d, epdf);
-                                const float mis = diffuse ? mis_weight(prev_pdf, epdf) : 1.f;
-                                rad = add(rad, mul(scale(thr, mis), ev));
-                            }
-                        }
-                    } else {
-                        const uint32_t info = prim_info(s, prim);
-                        if (HIDE && (cam || info_light(info))) {
-                            if (info_light(info)) {
-                                if (!cam) defer_emission(rs, p, thr, light_of(s, prim));
-                                aux.w = 0;  // the record's radiance before its continuation is already kept
-                                rs.aux[p] = aux;
-                                alive = true;
-                                ntype = kPassQ;
-                            } else {
-                                // the camera ray's first visible surface (as k_post_camera)
-                                alive = !(pp.max_depth >= 0 && 0 + 2 > pp.max_depth);
-                                ntype = info_type(info);
-                            }
-                        } else {
-                            if (info_light(info)) defer_emission(rs, p, thr, light_of(s, prim));
-                            alive = true;
-                            const int depth = aux.z;
-                            if (depth >= pp.rr_depth) {
-                                Pcg32 rng;
-                                rng.state = rs.rng[p];
-                                rng.inc = ((uint64_t)rs.seq[p] << 1u) | 1u;
-                                const float pr = fmin0(cmax(scale(scale(thr, eta), eta)), 0.99f);
-                                if (rng.next_float() > pr) {
-                                    alive = false;
-                                } else {
-                                    thr = divs(thr, pr);
-                                    rs.thr[p] = f4(thr, eta);
-                                }
-                                rs.rng[p] = rng.state;
-                            }
-                            if (alive) {
-                                const int nd = depth + 1;
-                                if (pp.max_depth >= 0 && nd + 2 > pp.max_depth) alive = false;
-                                aux.z = nd;
-                                rs.aux[p] = aux;
-                                ntype = info_type(info);
-                            }
-                        }
+            if (info != kNone) {
+                if (grec) {
+                    const int rec = rs.depth[p].y;
+                    if (rec > 0) {
+                        // radiance before the continuation of a recorded vertex
+                        const float4 rad = rs.rad[p];
+                        float* r = grec + (size_t)(rec - 1) * kGRecFloats;
+                        r[kRecRad] = rad.x;
+                        r[kRecRad + 1] = rad.y;
+                        r[kRecRad + 2] = rad.z;
                     }
                 }
-                rs.rad[p] = f4(rad, 0.f);
+                const bool cam = HIDE && (rs.aux[p].y & kFlagCamera) != 0;
+                if (info == kMiss) {
+                    const SceneRec sc = path_scene(s, p);
+                    if (sc.env_light >= 0) {
+                        const uint2 aux = rs.aux[p];
+                        const vec3 d = f3(rs.ray_d[p]);
+                        const vec3 thr = f3(rs.thr[p]);
+                        vec3 rad = f3(rs.rad[p]);
+                        const LightRec& e = s.lights[sc.env_light];
+                        if (cam) {
+                            rad = add(rad,
+                                      mul(thr, e.env_visual ? env_eval(s, e, d) : v3(sc.bg[0], sc.bg[1], sc.bg[2])));
+                        } else {
+                            float epdf;
+                            const vec3 ev = env_eval_pdf(s, e, sc.num_lights, d, epdf);
+                            const float mis =
+                                (aux.y & kFlagDiffuse) != 0 ? mis_weight(__uint_as_float(aux.x), epdf) : 1.f;
+                            rad = add(rad, mul(scale(thr, mis), ev));
+                        }
+                        rs.rad[p] = f4(rad, 0.f);
+                    }
+                } else if (HIDE && (cam || info_light(info))) {
+                    if (info_light(info)) {
+                        if (!cam) defer_emission(rs, p, f3(rs.thr[p]));
+                        rs.depth[p].y = 0;  // the record's radiance before its continuation is already kept
+                        alive = true;
+                        ntype = kPassQ;
+                    } else {
+                        // the camera ray's first visible surface (as k_post_camera)
+                        alive = !(pp.max_depth >= 0 && 0 + 2 > pp.max_depth);
+                        ntype = info_type(info);
+                    }
+                } else {
+                    if (info_light(info)) defer_emission(rs, p, f3(rs.thr[p]));
+                    const int at = HIDE ? rs.depth[p].x : depth;
+                    // (at the cap no path survives, so no roulette is drawn)
+                    alive = !(pp.max_depth >= 0 && at + 1 + 2 > pp.max_depth);
+                    ntype = info_type(info);
+                    if (alive && at >= pp.rr_depth) {
+                        const float4 th4 = rs.thr[p];
+                        const float eta = th4.w;
+                        Pcg32 rng;
+                        rng.state = rs.rng[p];
+                        rng.inc = ((uint64_t)rs.seq[p] << 1u) | 1u;
+                        const float pr = fmin0(cmax(scale(scale(f3(th4), eta), eta)), 0.99f);
+                        if (rng.next_float() > pr) {
+                            alive = false;
+                        } else {
+                            rs.thr[p] = f4(divs(f3(th4), pr), eta);
+                            rs.rng[p] = rng.state;
+                        }
+                    }
+                    if (HIDE && alive) rs.depth[p].x = at + 1;
+                }
             }
-            s_p[u][threadIdx.x] = p;
             s_b[u][threadIdx.x] = alive ? 1u << ntype : 0u;
         }
         uint32_t pv[kStageItems], bv[kStageItems];
@@ -1202,10 +1197,10 @@ dl_status ensure_state(Ctx* c, uint32_t P, uint32_t pixels) {
     DL_TRY(alloc(c, rs, &rs->b.rad, P));
     DL_TRY(alloc(c, rs, &rs->b.nee, P));
     DL_TRY(alloc(c, rs, &rs->b.aux, P));
+    DL_TRY(alloc(c, rs, &rs->b.depth, P));
     DL_TRY(alloc(c, rs, &rs->b.rng, P));
     DL_TRY(alloc(c, rs, &rs->b.seq, P));
     DL_TRY(alloc(c, rs, &rs->b.pos, P));
-    DL_TRY(alloc(c, rs, &rs->b.occ, P));
     DL_TRY(alloc(c, rs, &rs->b.sid, P));
     DL_TRY(alloc(c, rs, &rs->b.matq[0], (size_t)P * kTypes));
     DL_TRY(alloc(c, rs, &rs->b.matq[1], (size_t)P * kTypes));
@@ -1213,6 +1208,7 @@ dl_status ensure_state(Ctx* c, uint32_t P, uint32_t pixels) {
     DL_TRY(alloc(c, rs, &rs->b.shq, P));
     DL_TRY(alloc(c, rs, &rs->b.emq, P));
     DL_TRY(alloc(c, rs, &rs->b.cnt, 1));
+    DL_TRY(alloc(c, rs, &rs->b.work, 2 * kWorkGroups * kWorkStride));
     DL_TRY(alloc(c, rs, &rs->b.film, pixels));
     DL_TRY(alloc(c, rs, &rs->b.rgb, (size_t)pixels * 3));
     DL_HIP_CHECK(c, hipHostMalloc((void**)&rs->cnt_host, sizeof(Counters), hipHostMallocDefault));
@@ -1223,7 +1219,7 @@ constexpr uint32_t kGuideRecords = dl_sizes::kGuideRecordSlots;  // training rec
 static_assert(kGRecFloats == dl_sizes::kGuideRecordFloats && kGMix == dl_sizes::kGuideMixFloats,
               "guided buffer sizes the render service reserves");
 // the per-path bytes ensure_state allocates, as the render service reserves them
-static_assert(8 * sizeof(float4) + sizeof(uint64_t) + sizeof(uint32_t) + sizeof(float2) + 2 * sizeof(uint8_t) +
+static_assert(7 * sizeof(float4) + sizeof(uint2) + sizeof(int2) + sizeof(uint64_t) + sizeof(uint32_t) + sizeof(float2) + sizeof(uint8_t) +
                       2 * kTypes * sizeof(uint32_t) + 3 * sizeof(uint32_t) ==
                   dl_sizes::kStateBytesPerPath &&
               kTypes == dl_sizes::kMatQueueSegs && sizeof(float4) + 3 * sizeof(float) == dl_sizes::kFilmBytesPerPixel,
@@ -1325,14 +1321,17 @@ dl_status run_bounces(Ctx* c, RenderState* rs, const PassParams& pp, const Scene
     DL_TRY(tm.stop());
     DL_HIP_CHECK(c, hipGetLastError());
     if (normals) return DL_OK;  // no bounces
-    // One bounce: shading of the paths in queue `cur` (whose lengths per
-    // material type are `len`; `first`: the camera paths' first shading
+    // Bounce k: shading of the paths in queue k & 1 (whose lengths per
+    // material type are `len`; k = 0: the camera paths' first shading
     // vertices), their continuation and shadow traces, and post (which
-    // queues the survivors in cur ^ 1).  Every kernel reads its
+    // queues the survivors in the other one).  Every kernel reads its
     // queue length from the device counters; the host skips the shading
     // kernels of empty queues.
-    auto bounce = [&](int cur, const uint32_t* len, bool first) -> dl_status {
-        k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, cur ^ 1);
+    const bool track = hide || gv.rec != nullptr;
+    auto bounce = [&](int k, const uint32_t* len) -> dl_status {
+        const int cur = k & 1;
+        const bool first = k == 0;
+        k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, rs->b.work, cur ^ 1);
         DL_TRY(tm.start(kTagShade));
         if (hide && len[kPassQ] > 0) k_pass<<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur);
         for (int t = 0; t < DL_BSDF_COUNT; t++) {
@@ -1349,20 +1348,20 @@ dl_status run_bounces(Ctx* c, RenderState* rs, const PassParams& pp, const Scene
                 DL_TRY(tm.stop());
                 DL_TRY(tm.start(kTagShade));
                 switch (t) {
-                    case DL_BSDF_DIFFUSE: k_shade<DL_BSDF_DIFFUSE, true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first); break;
-                    case DL_BSDF_MICROFACET: k_shade<DL_BSDF_MICROFACET, true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first); break;
-                    case DL_BSDF_ANISO_GGX: k_shade<DL_BSDF_ANISO_GGX, true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first); break;
-                    case DL_BSDF_CONDUCTOR: k_shade<DL_BSDF_CONDUCTOR, true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first); break;
+                    case DL_BSDF_DIFFUSE: k_shade<DL_BSDF_DIFFUSE, true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first, track); break;
+                    case DL_BSDF_MICROFACET: k_shade<DL_BSDF_MICROFACET, true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first, track); break;
+                    case DL_BSDF_ANISO_GGX: k_shade<DL_BSDF_ANISO_GGX, true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first, track); break;
+                    case DL_BSDF_CONDUCTOR: k_shade<DL_BSDF_CONDUCTOR, true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first, track); break;
                 }
                 continue;
             }
             switch (t) {
-                case DL_BSDF_DIFFUSE: k_shade<DL_BSDF_DIFFUSE, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first); break;
-                case DL_BSDF_MIRROR: k_shade<DL_BSDF_MIRROR, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first); break;
-                case DL_BSDF_DIELECTRIC: k_shade<DL_BSDF_DIELECTRIC, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first); break;
-                case DL_BSDF_MICROFACET: k_shade<DL_BSDF_MICROFACET, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first); break;
-                case DL_BSDF_ANISO_GGX: k_shade<DL_BSDF_ANISO_GGX, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first); break;
-                case DL_BSDF_CONDUCTOR: k_shade<DL_BSDF_CONDUCTOR, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first); break;
+                case DL_BSDF_DIFFUSE: k_shade<DL_BSDF_DIFFUSE, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first, track); break;
+                case DL_BSDF_MIRROR: k_shade<DL_BSDF_MIRROR, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first, track); break;
+                case DL_BSDF_DIELECTRIC: k_shade<DL_BSDF_DIELECTRIC, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first, track); break;
+                case DL_BSDF_MICROFACET: k_shade<DL_BSDF_MICROFACET, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first, track); break;
+                case DL_BSDF_ANISO_GGX: k_shade<DL_BSDF_ANISO_GGX, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first, track); break;
+                case DL_BSDF_CONDUCTOR: k_shade<DL_BSDF_CONDUCTOR, false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv, first, track); break;
             }
         }
         DL_TRY(tm.stop());
@@ -1380,9 +1379,9 @@ dl_status run_bounces(Ctx* c, RenderState* rs, const PassParams& pp, const Scene
         DL_TRY(tm.stop());
         DL_TRY(tm.start(kTagShade));
         if (hide)
-            k_post<true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv.rec);
+            k_post<true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur ^ 1, k, gv.rec);
         else
-            k_post<false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur, gv.rec);
+            k_post<false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur ^ 1, k, gv.rec);
         k_post_emit<<<stage_grid, kStageBlock, 0, c->stream>>>(sv, rs->b);
         DL_TRY(tm.stop());
         DL_HIP_CHECK(c, hipGetLastError());
@@ -1409,7 +1408,7 @@ dl_status run_bounces(Ctx* c, RenderState* rs, const PassParams& pp, const Scene
         if (live == 0) break;
         uint32_t len[kTypes];
         for (int t = 0; t < kTypes; t++) len[t] = s.mat[cur][t];
-        DL_TRY(bounce(cur, len, k == 0));
+        DL_TRY(bounce(k, len));
     }
     return DL_OK;
 }
@@ -1513,8 +1512,8 @@ dl_status render(Ctx* c, const dl_render_params* prm, float* rgb_host, dl_render
                                                               kGuideRecords));
             k_clear_records<<<std::max(1, c->num_cus) * 4, 256, 0, c->stream>>>(rs->b.grec, kGuideRecords);
         }
-        k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, 0);
-        k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, 1);
+        k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, rs->b.work, 0);
+        k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, rs->b.work, 1);
         DL_TRY(tm.start(kTagOther));
         k_raygen<<<stage_grid, kStageBlock, 0, c->stream>>>(pp, c->cam, rs->b, 0u, pp.P);
         DL_TRY(tm.stop());
@@ -1699,8 +1698,8 @@ dl_status render_batch(Ctx* c, const dl_render_params* prm, const dl_batch_item*
     std::vector<uint32_t> base(n);
     DL_HIP_CHECK(c, hipEventRecord(c->ev0, c->stream));
     k_reset_all<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt);
-    k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, 0);
-    k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, 1);
+    k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, rs->b.work, 0);
+    k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, rs->b.work, 1);
     DL_TRY(tm.start(kTagOther));
     uint32_t off = 0;
     for (uint32_t i = 0; i < n; i++) {

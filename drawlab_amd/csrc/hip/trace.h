@@ -42,16 +42,33 @@ struct LaneStack {
     int lane, stride;
     int* __restrict__ ovf;
     uint32_t ostride;
-    // No tree is deeper than kMaxStack, so the last branch is never taken;
-    // it keeps every access in bounds regardless.
-    __device__ __forceinline__ void push(int& sp, int v) {
-        if (sp < kLdsStack)
-            lds[sp * stride + lane] = v;
-        else if (sp < kMaxStack)
-            ovf[(size_t)(sp - kLdsStack) * ostride] = v;
-        else
-            return;
-        ++sp;
+    // Pushes a, b, c in this order, each only if its flag is set.  While the
+    // three cannot reach the overflow they are stored without a branch (a
+    // store whose flag is clear leaves the entry to the next one).  No tree is
+    // deeper than kMaxStack, so the last test never fails; it keeps every
+    // access in bounds regardless.
+    __device__ __forceinline__ void push3(int& sp, int a, bool pa, int b, bool pb, int c, bool pc) {
+        if (sp <= kLdsStack - 3) {
+            lds[sp * stride + lane] = a;
+            sp += pa ? 1 : 0;
+            lds[sp * stride + lane] = b;
+            sp += pb ? 1 : 0;
+            lds[sp * stride + lane] = c;
+            sp += pc ? 1 : 0;
+        } else {
+#pragma unroll 1
+            for (int k = 0; k < 3; k++) {
+                const int v = k == 0 ? a : k == 1 ? b : c;
+                if (!(k == 0 ? pa : k == 1 ? pb : pc)) continue;
+                if (sp < kLdsStack)
+                    lds[sp * stride + lane] = v;
+                else if (sp < kMaxStack)
+                    ovf[(size_t)(sp - kLdsStack) * ostride] = v;
+                else
+                    break;
+                ++sp;
+            }
+        }
     }
     __device__ __forceinline__ int pop(int& sp) {
         --sp;
@@ -70,31 +87,28 @@ __device__ __forceinline__ void cswap(float& ka, int& ra, float& kb, int& rb) {
     ra = r;
 }
 
-// Slab test of one child box (lo, hi per axis): entry distance n and
-// whether [n, far] meets [tmin, tmax] (far widened by kFarSlack).
-__device__ __forceinline__ bool slab1(float lx, float hx, float ly, float hy, float lz, float hz, const vec3& o,
-                                      const vec3& rcp, float tmin, float tmax, float& n) {
-    const float a0 = (lx - o.x) * rcp.x, b0 = (hx - o.x) * rcp.x;
-    const float a1 = (ly - o.y) * rcp.y, b1 = (hy - o.y) * rcp.y;
-    const float a2 = (lz - o.z) * rcp.z, b2 = (hz - o.z) * rcp.z;
-    n = fmaxf(fmaxf(fminf(a0, b0), fminf(a1, b1)), fmaxf(fminf(a2, b2), tmin));
-    const float f = fminf(fminf(fmaxf(a0, b0), fmaxf(a1, b1)), fminf(fmaxf(a2, b2), tmax));
-    return n <= f * kFarSlack;
-}
-
-// Slab test of the child whose quantised planes sit at bit `sh` of the
-// node's records r1, r2: each plane is origin + q * step.  q * step is
-// exact (an 8-bit integer times a power of two), so the fused
-// multiply-add rounds once, exactly like the separate product and sum the
-// quantiser checked.
+// One plane of a child box: its byte of `word` (children 0..3 in bytes 0..3)
+// as origin + q * step.  q * step is exact (an 8-bit integer times a power of
+// two), so the fused multiply-add rounds once, exactly like the separate
+// product and sum the quantiser checked.
 __device__ __forceinline__ float qplane(uint32_t word, int sh, float step, float origin) {
     return __builtin_fmaf((float)((word >> sh) & 0xffu), step, origin);
 }
-__device__ __forceinline__ bool slab_q(const float4& r0, const uint4& r1, const uint4& r2, int sh, float sx, float sy,
-                                       float sz, const vec3& o, const vec3& rcp, float tmin, float tmax, float& n) {
-    return slab1(qplane(r1.x, sh, sx, r0.x), qplane(r1.y, sh, sx, r0.x), qplane(r1.z, sh, sy, r0.y),
-                 qplane(r1.w, sh, sy, r0.y), qplane(r2.x, sh, sz, r0.z), qplane(r2.y, sh, sz, r0.z), o, rcp, tmin,
-                 tmax, n);
+// Slab test of the child at bit `sh` of the words of its near and far planes
+// (per axis the lo planes are the near ones for a direction whose reciprocal
+// is positive, else the hi planes: chosen once per node as whole words, which
+// takes 6 selects instead of 24 minima and maxima of plane distances): entry
+// distance n, and whether [n, far] meets [tmin, tmax] (far widened by
+// kFarSlack).
+__device__ __forceinline__ bool slab_q(const uint32_t (&nw)[3], const uint32_t (&fw)[3], int sh, const vec3& step,
+                                       const vec3& org, const vec3& o, const vec3& rcp, float tmin, float tmax,
+                                       float& n) {
+    const float n0 = (qplane(nw[0], sh, step.x, org.x) - o.x) * rcp.x, f0 = (qplane(fw[0], sh, step.x, org.x) - o.x) * rcp.x;
+    const float n1 = (qplane(nw[1], sh, step.y, org.y) - o.y) * rcp.y, f1 = (qplane(fw[1], sh, step.y, org.y) - o.y) * rcp.y;
+    const float n2 = (qplane(nw[2], sh, step.z, org.z) - o.z) * rcp.z, f2 = (qplane(fw[2], sh, step.z, org.z) - o.z) * rcp.z;
+    n = fmaxf(fmaxf(n0, n1), fmaxf(n2, tmin));
+    const float f = fminf(fminf(f0, f1), fminf(f2, tmax));
+    return n <= f * kFarSlack;
 }
 
 // Moller-Trumbore on a pre-gathered triangle; returns false on a miss.
@@ -137,11 +151,56 @@ __device__ __forceinline__ void wave_add(unsigned long long* dst, uint32_t v) {
 // 4 : 5 measure within 0.5% of it).
 constexpr uint32_t kTriCost = 2, kNodeCost = 5;
 
+// How a persistent grid's waves share n work slots: slots [0, base) are
+// spread evenly over them, the others handed out in chunks of `unit` slots.
+// The chunks are dealt in turn to kWorkGroups groups of blocks, and a wave
+// claims its group's next chunk with one atomic on the group's counter (zero
+// at launch).  One counter for all waves would serialise: its atomics pass at
+// about 55 per microsecond (measured), so the 8192 waves of a full grid
+// claiming once each would already take 150 us.  The blocks of a group run on
+// one XCD (block b runs on XCD b mod 8), whose L2 holds their counter.
+constexpr uint32_t kWorkGroups = kWorkGroupsHost;
+struct TraceWork {
+    uint32_t* counter;  // of this wave's group
+    uint32_t n;         // slots in all
+    uint32_t first;     // this wave's first slots: [first, first + count)
+    uint32_t count;
+    uint32_t base;
+    uint32_t unit;
+    uint32_t group;
+};
+__device__ __forceinline__ TraceWork trace_work(uint32_t* counters, uint32_t n) {
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+    const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+    // (n is at most 2^31 and a grid has at most 2^13 waves)
+    const uint32_t share = (n + waves - 1) / waves;
+    // Few slots: a few lanes of every wave rather than all lanes of some, as
+    // a wave takes as long as the slowest of its lanes.  From 16 per wave on
+    // half of them, at most 64, are given out at once, the rest in chunks of
+    // a sixteenth of a wave's share, 8 to 64 slots, so the waves end together.
+    const uint32_t per = share < 16u ? share : min(64u, share / 2u);
+    TraceWork w;
+    w.group = blockIdx.x % kWorkGroups;
+    w.counter = counters + w.group * kWorkStride;
+    w.n = n;
+    w.base = min(n, per * waves);
+    w.first = min(wave * per, w.base);
+    w.count = min(per, w.base - w.first);
+    w.unit = share >= 1024u ? 64u : share >= 512u ? 32u : share >= 256u ? 16u : 8u;
+    return w;
+}
+
 // Persistent traversal with per-lane ray refill.  Every lane of a wave stays
-// in the loop until the whole wave has run out of rays; lanes whose rays
-// finished start their next rays as soon as enough of them wait (lane g
-// takes rays g, g + G, g + 2G, ...: no atomic round trip on the refill
-// path), so a wave never idles behind its slowest ray.
+// in the loop until the wave has run out of rays; lanes whose rays finished
+// start the wave's next rays as soon as enough of them wait, so a wave never
+// idles behind its slowest ray.  A wave holds a chunk of up to 64 consecutive
+// slots, their entries loaded together (one per lane); while it works on it,
+// the claim of the next chunk is already on its way.  (With lane g taking
+// rays g, g + G, g + 2G, ... of the queue instead, a launch waited for the
+// waves that chance gave the longest rays, CUs idle a quarter of the time,
+// and the rays a wave had in flight lay far apart: 4.19M diffuse-bounce rays
+// against 2M triangles took 1.36 ms, now 0.81 ms, of which the branch-free
+// near / far planes, triangle indices and pushes are the smaller part.)
 //
 // A step visits one node, or tests the next one or two of the triangles of
 // the leaves the lane's last node visit hit.  A node visit decides the next
@@ -162,42 +221,71 @@ constexpr uint32_t kTriCost = 2, kNodeCost = 5;
 // entry(slot) (the ray of work slot `slot`), load(e, o, d,
 // tmin, tmax), root(e) (the node traversal starts from), store_hit(e, prim,
 // t, u, v, nodes, tris) for closest hits and store_occ(e, occluded, nodes,
-// tris) for any-hit queries, e being an entry.
+// tris) for any-hit queries, e being an entry.  With kResolve an any-hit
+// query has no occlusion store: for every ray that finished unoccluded the
+// lane calls resolve_load(e, a, b) and resolve_store(e, a, b) at the wave's
+// next refill, so those loads wait together with the next rays'.
 template <bool ANY, bool COUNT, class IO>
-__device__ __forceinline__ void traverse_persistent(const BvhView& bvh, uint32_t n, uint32_t* work, LaneStack& stk,
-                                                    IO& io, TraceCounters& total) {
-    (void)work;  // a claim counter the static-stride refill does not need (callers still zero it)
-    const uint32_t G = gridDim.x * blockDim.x;
-    uint32_t next = blockIdx.x * blockDim.x + threadIdx.x;
-    // the IO entry of the lane's next slot, fetched one refill ahead (a
-    // queue's entry is a load the ray's own loads depend on)
-    uint32_t pnext = next < n ? io.entry(next) : 0u;
+__device__ __forceinline__ void traverse_persistent(const BvhView& bvh, const TraceWork& work, LaneStack& stk, IO& io,
+                                                    TraceCounters& total) {
+    const uint32_t lane = __lane_id();
+    const uint32_t n = work.n;
+    // the wave's chunk: slots pos .. len - 1 of its entries are still to start
+    uint32_t pos = 0, len = work.count;
+    uint32_t ent = lane < len ? io.entry(work.first + lane) : 0u;
+    bool more = work.base < n;  // slots may be left to claim
+    uint32_t claim = 0;
+    auto claim_next = [&]() {
+        if (lane == 0) claim = atomicAdd(work.counter, 1u);
+    };
+    if (more) claim_next();
     uint32_t ray = 0;
-    bool active = false, exhausted = false;
+    bool active = false;
     vec3 o = v3(0, 0, 0), d = v3(0, 0, 0), rcp = v3(0, 0, 0);
     float tmin = 0.f, best_t = 0.f, bu = 0.f, bv = 0.f;
     uint32_t best = 0xffffffffu;
     int sp = 0, cur = 0;
-    // triangles of the last visited node's hit leaves: leaf references, the
-    // triangle count of each hit leaf child packed one byte each (0 for the
-    // others; a leaf holds at most kMaxLeafCount = 255), their total and the
-    // next one to test; `last`: no node left to visit once they are tested
-    int4 lref = make_int4(0, 0, 0, 0);
-    uint32_t lcnt = 0;
+    // triangles of the last visited node's hit leaves: triangle j lies at
+    // j + lb[c], c the first slot whose running total of triangles exceeds j
+    // (totals of slots 0, 0-1 and 0-2 packed in lend, 10 bits each: a leaf
+    // holds at most kMaxLeafCount = 255), their number and the next one to
+    // test; `last`: no node left to visit once they are tested
+    int4 lb = make_int4(0, 0, 0, 0);
+    uint32_t lend = 0;
     int ltri = 0, lj = 0;
     bool last = false;
+    bool pend = false;  // (kResolve) the lane's finished ray is unoccluded and not yet resolved
     TraceCounters cnt;
     for (;;) {
-        const bool need = !active && !exhausted;
+        if (pos == len && more) {
+            const uint32_t chunk = (uint32_t)__builtin_amdgcn_readfirstlane((int)claim) * kWorkGroups + work.group;
+            const uint32_t b = work.base + chunk * work.unit;
+            if (b < n) {
+                pos = 0;
+                len = min(work.unit, n - b);
+                ent = lane < len ? io.entry(b + lane) : 0u;
+                claim_next();
+            } else {
+                more = false;
+            }
+        }
+        const unsigned long long busy = __ballot(active);
         const uint32_t refill_min = ANY ? IO::kRefillMinAny : IO::kRefillMin;
-        const bool refill = (uint32_t)__popcll(__ballot(need)) >= refill_min || !__ballot(active);
-        if (need && refill) {
-            const uint32_t slot = next;
-            next += G;
-            {
-                if (slot < n) {
-                    ray = pnext;
-                    if (next < n) pnext = io.entry(next);
+        const uint32_t idle = 64u - (uint32_t)__popcll(busy);
+        if (pos < len && idle >= refill_min) {
+            const uint32_t at = pos + (uint32_t)__builtin_amdgcn_mbcnt_hi(
+                                          ~(uint32_t)(busy >> 32), __builtin_amdgcn_mbcnt_lo(~(uint32_t)busy, 0));
+            const uint32_t e = (uint32_t)__shfl((int)ent, (int)(at & 63u));
+            if (!active) {
+                const uint32_t fin = ray;
+                const bool resolve = ANY && IO::kResolve && pend;
+                float4 ra, rb;
+                if (resolve) {
+                    io.resolve_load(fin, ra, rb);
+                    pend = false;
+                }
+                if (at < len) {
+                    ray = e;
                     float tmax;
                     io.load(ray, o, d, tmin, tmax);
                     rcp = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
@@ -206,7 +294,6 @@ __device__ __forceinline__ void traverse_persistent(const BvhView& bvh, uint32_t
                     bu = bv = 0.0f;
                     sp = 0;
                     cur = io.root(ray);
-                    lcnt = 0;
                     ltri = lj = 0;
                     last = false;
                     cnt = TraceCounters();
@@ -215,19 +302,22 @@ __device__ __forceinline__ void traverse_persistent(const BvhView& bvh, uint32_t
                     // test: finish it at once as a miss.
                     if (isnan(o.x) || isnan(o.y) || isnan(o.z) || isnan(d.x) || isnan(d.y) || isnan(d.z) || isnan(tmin) ||
                         isnan(tmax)) {
-                        if (ANY)
+                        if (ANY && IO::kResolve)
+                            pend = true;
+                        else if (ANY)
                             io.store_occ(ray, false, 0, 0);
                         else
                             io.store_hit(ray, best, best_t, 0.0f, 0.0f, 0, 0);
                     } else {
                         active = true;
                     }
-                } else {
-                    exhausted = true;
                 }
+                if (resolve) io.resolve_store(fin, ra, rb);
             }
+            pos = min(len, pos + idle);
+        } else if (idle == 64u && pos == len && !more) {
+            break;
         }
-        if (!__ballot(active)) break;
         // One kind of step per wave and iteration: the lanes whose next
         // step is a triangle test and those whose next step is a node visit
         // would otherwise run both branches every iteration under partial
@@ -242,21 +332,22 @@ __device__ __forceinline__ void traverse_persistent(const BvhView& bvh, uint32_t
         if (!active || tri_step != tri_mode) continue;
 
         bool done = false, hit_any = false;
-        if (tri_step) {
+        if (tri_mode) {
             // the next one or two triangles of the last visit's hit leaves, in
             // slot order: both fetched before the first is tested, so a pair
             // costs one dependent wait; the second is accepted against the
             // best t the first left, as a sequential loop would
-            const int ls0 = (int)(lcnt & 0xffu);
-            const int ls1 = ls0 + (int)((lcnt >> 8) & 0xffu);
-            const int ls2 = ls1 + (int)((lcnt >> 16) & 0xffu);
+            const int e0 = (int)(lend & 0x3ffu), e1 = (int)((lend >> 10) & 0x3ffu), e2 = (int)(lend >> 20);
             const int j = lj;
             const bool two = j + 1 < ltri;
-            const int k0 = j < ls0 ? ~lref.x + j : j < ls1 ? ~lref.y + (j - ls0) : j < ls2 ? ~lref.z + (j - ls1)
-                                                                                     : ~lref.w + (j - ls2);
             const int j1 = two ? j + 1 : j;
-            const int k1 = j1 < ls0 ? ~lref.x + j1 : j1 < ls1 ? ~lref.y + (j1 - ls0) : j1 < ls2 ? ~lref.z + (j1 - ls1)
-                                                                                          : ~lref.w + (j1 - ls2);
+            int k0 = lb.w, k1 = lb.w;
+            k0 = j < e2 ? lb.z : k0;
+            k1 = j1 < e2 ? lb.z : k1;
+            k0 = j < e1 ? lb.y : k0;
+            k1 = j1 < e1 ? lb.y : k1;
+            k0 = (j < e0 ? lb.x : k0) + j;
+            k1 = (j1 < e0 ? lb.x : k1) + j1;
             const float4* tp0 = bvh.tris + 3 * k0;
             const float4* tp1 = bvh.tris + 3 * k1;
             const float4 ta = tp0[0], tb = tp0[1], tc = tp0[2];
@@ -306,20 +397,28 @@ __device__ __forceinline__ void traverse_persistent(const BvhView& bvh, uint32_t
             if (COUNT) cnt.nodes++;
             // child boxes: origin + q * step (q * step exact, one rounding)
             const uint32_t eb = __float_as_uint(r0.w);
-            const float sx = __uint_as_float((eb & 0xffu) << 23), sy = __uint_as_float(((eb >> 8) & 0xffu) << 23),
-                        sz = __uint_as_float(((eb >> 16) & 0xffu) << 23);
+            const vec3 step = v3(__uint_as_float((eb & 0xffu) << 23), __uint_as_float(((eb >> 8) & 0xffu) << 23),
+                                 __uint_as_float(((eb >> 16) & 0xffu) << 23));
+            const vec3 org = v3(r0.x, r0.y, r0.z);
+            const bool px = rcp.x >= 0.0f, py = rcp.y >= 0.0f, pz = rcp.z >= 0.0f;
+            const uint32_t nw[3] = {px ? r1.x : r1.y, py ? r1.z : r1.w, pz ? r2.x : r2.y};
+            const uint32_t fw[3] = {px ? r1.y : r1.x, py ? r1.w : r1.z, pz ? r2.y : r2.x};
             float n0, n1, n2, n3;
-            const bool h0 = slab_q(r0, r1, r2, 0, sx, sy, sz, o, rcp, tmin, best_t, n0);
-            const bool h1 = slab_q(r0, r1, r2, 8, sx, sy, sz, o, rcp, tmin, best_t, n1);
-            const bool h2 = slab_q(r0, r1, r2, 16, sx, sy, sz, o, rcp, tmin, best_t, n2);
-            const bool h3 = slab_q(r0, r1, r2, 24, sx, sy, sz, o, rcp, tmin, best_t, n3);
+            const bool h0 = slab_q(nw, fw, 0, step, org, o, rcp, tmin, best_t, n0);
+            const bool h1 = slab_q(nw, fw, 8, step, org, o, rcp, tmin, best_t, n1);
+            const bool h2 = slab_q(nw, fw, 16, step, org, o, rcp, tmin, best_t, n2);
+            const bool h3 = slab_q(nw, fw, 24, step, org, o, rcp, tmin, best_t, n3);
             // triangles of the hit leaf children, tested in the next
             // iterations (the closest hit is the minimum over (t, id), so
             // their order does not change it)
-            lref = ref;
-            lcnt = r2.z & (((h0 && ref.x < 0) ? 0xffu : 0u) | ((h1 && ref.y < 0) ? 0xff00u : 0u) |
-                           ((h2 && ref.z < 0) ? 0xff0000u : 0u) | ((h3 && ref.w < 0) ? 0xff000000u : 0u));
-            ltri = (int)((lcnt & 0xffu) + ((lcnt >> 8) & 0xffu) + ((lcnt >> 16) & 0xffu) + (lcnt >> 24));
+            const int c0n = (h0 && ref.x < 0) ? (int)(r2.z & 0xffu) : 0;
+            const int c1n = (h1 && ref.y < 0) ? (int)((r2.z >> 8) & 0xffu) : 0;
+            const int c2n = (h2 && ref.z < 0) ? (int)((r2.z >> 16) & 0xffu) : 0;
+            const int c3n = (h3 && ref.w < 0) ? (int)(r2.z >> 24) : 0;
+            const int e1 = c0n + c1n, e2 = e1 + c2n;
+            lend = (uint32_t)c0n | ((uint32_t)e1 << 10) | ((uint32_t)e2 << 20);
+            lb = make_int4(~ref.x, ~ref.y - c0n, ~ref.z - e1, ~ref.w - e2);
+            ltri = e2 + c3n;
             lj = 0;
             // hit internal children: keys = entry distances (+inf: not
             // taken), sorted by a 5-exchange network; the nearest is visited
@@ -333,9 +432,7 @@ __device__ __forceinline__ void traverse_persistent(const BvhView& bvh, uint32_t
             cswap(k1, c1, k3, c3);
             cswap(k1, c1, k2, c2);
             if (k0 != INFINITY) {
-                if (k3 != INFINITY) stk.push(sp, c3);
-                if (k2 != INFINITY) stk.push(sp, c2);
-                if (k1 != INFINITY) stk.push(sp, c1);
+                stk.push3(sp, c3, k3 != INFINITY, c2, k2 != INFINITY, c1, k1 != INFINITY);
                 cur = c0;
             } else if (sp == 0) {
                 last = true;
@@ -345,7 +442,9 @@ __device__ __forceinline__ void traverse_persistent(const BvhView& bvh, uint32_t
             done = last && ltri == 0;
         }
         if (done) {
-            if (ANY)
+            if (ANY && IO::kResolve)
+                pend = !hit_any;
+            else if (ANY)
                 io.store_occ(ray, hit_any, cnt.nodes, cnt.tris);
             else
                 io.store_hit(ray, best, best_t, bu, bv, cnt.nodes, cnt.tris);  // a miss keeps t = tmax
@@ -355,6 +454,11 @@ __device__ __forceinline__ void traverse_persistent(const BvhView& bvh, uint32_t
             }
             active = false;
         }
+    }
+    if (ANY && IO::kResolve && pend) {
+        float4 ra, rb;
+        io.resolve_load(ray, ra, rb);
+        io.resolve_store(ray, ra, rb);
     }
 }
 

@@ -10,6 +10,7 @@
 namespace dl {
 
 // Rays of a batch: 8 planes of n floats; results in planes of n.
+template <bool COUNT>
 struct BatchIO {
     const float* __restrict__ rays;
     size_t N;
@@ -30,20 +31,23 @@ struct BatchIO {
         tmax = rays[7 * N + i];
     }
     __device__ __forceinline__ int root(uint32_t) const { return 0; }
+    static constexpr bool kResolve = false;
+    __device__ __forceinline__ void resolve_load(uint32_t, float4&, float4&) const {}
+    __device__ __forceinline__ void resolve_store(uint32_t, const float4&, const float4&) const {}
     __device__ __forceinline__ void store_hit(uint32_t i, uint32_t p, float t, float u, float v, uint32_t nn,
                                               uint32_t nt) const {
         prim[i] = p;
         th[i] = t;
         uh[i] = u;
         vh[i] = v;
-        if (cn) {
+        if (COUNT) {
             cn[i] = nn;
             ct[i] = nt;
         }
     }
     __device__ __forceinline__ void store_occ(uint32_t i, bool o, uint32_t nn, uint32_t nt) const {
         occ[i] = o ? 1 : 0;
-        if (cn) {
+        if (COUNT) {
             cn[i] = nn;
             ct[i] = nt;
         }
@@ -52,23 +56,23 @@ struct BatchIO {
 
 // Persistent grids (Ctx::trace_grid / trace_grid_count blocks) with per-lane refill.
 template <bool COUNT>
-__global__ __launch_bounds__(kTraceBlock) void k_trace_closest(BvhView bvh, BatchIO io, uint32_t n, uint32_t* work,
+__global__ __launch_bounds__(kTraceBlock, COUNT ? 4 : 8) void k_trace_closest(BvhView bvh, BatchIO<COUNT> io, uint32_t n, uint32_t* work,
                                                                int* __restrict__ ovf) {
     __shared__ int lds[kLdsStack * kTraceBlock];
     const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x, G = gridDim.x * kTraceBlock;
     LaneStack stk{lds, (int)threadIdx.x, kTraceBlock, ovf + g, G};
     TraceCounters tot;
-    traverse_persistent<false, COUNT>(bvh, n, work, stk, io, tot);
+    traverse_persistent<false, COUNT>(bvh, trace_work(work, n), stk, io, tot);
 }
 
 template <bool COUNT>
-__global__ __launch_bounds__(kTraceBlock) void k_trace_shadow(BvhView bvh, BatchIO io, uint32_t n, uint32_t* work,
+__global__ __launch_bounds__(kTraceBlock, COUNT ? 4 : 8) void k_trace_shadow(BvhView bvh, BatchIO<COUNT> io, uint32_t n, uint32_t* work,
                                                               int* __restrict__ ovf) {
     __shared__ int lds[kLdsStack * kTraceBlock];
     const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x, G = gridDim.x * kTraceBlock;
     LaneStack stk{lds, (int)threadIdx.x, kTraceBlock, ovf + g, G};
     TraceCounters tot;
-    traverse_persistent<true, COUNT>(bvh, n, work, stk, io, tot);
+    traverse_persistent<true, COUNT>(bvh, trace_work(work, n), stk, io, tot);
 }
 
 // Resident blocks per CU of the batch traversal kernels (the fewer of the
@@ -84,27 +88,41 @@ int batch_trace_blocks_per_cu(bool counting) {
     return std::max(1, std::min(kTraceBlocksPerCu, std::min(a, b)));
 }
 
-__global__ void k_zero_work(uint32_t* w) {
-    if (threadIdx.x < 4) w[threadIdx.x] = 0;
-}
+__global__ void k_zero_work(uint32_t* w) { w[threadIdx.x * kWorkStride] = 0; }
 
 // Lanes of a persistent grid step through ray indices by the grid size; a
 // 32-bit index must not wrap past n.
 constexpr uint32_t kMaxBatchRays = 1u << 31;
+
+// Blocks that trace n rays: a few rays per wave until every block of the
+// grid is in use (a wave takes as long as its slowest ray).
+constexpr uint32_t kBatchRaysPerWave = 4;
+uint32_t batch_blocks(uint32_t grid, uint32_t n) {
+    constexpr uint32_t per_block = kBatchRaysPerWave * (uint32_t)(kTraceBlock / 64);
+    return std::min(grid, (n + per_block - 1) / per_block);
+}
+
+// Whether trace_work leaves rays to claim, so that the counters have to be
+// cleared first: from 16 rays per wave on.
+bool claims_work(uint32_t blocks, uint32_t n) {
+    const uint32_t waves = blocks * (uint32_t)(kTraceBlock / 64);
+    return (n + waves - 1) / waves >= 16u;
+}
 
 dl_status launch_trace_closest(Ctx* c, const float* rays, uint32_t n, uint32_t* prim, float* t, float* u, float* v,
                                uint32_t* cn, uint32_t* ct) {
     if (n == 0) return DL_OK;
     if (n > kMaxBatchRays) return set_error(c, DL_ERR_INVALID, "more than 2^31 rays in one batch");
     BvhView bvh{c->ds.nodes, c->ds.tris};
-    const uint32_t blocks = cn ? c->trace_grid_count : c->trace_grid;
+    const uint32_t blocks = batch_blocks(cn ? c->trace_grid_count : c->trace_grid, n);
     DL_HIP_CHECK(c, hipEventRecord(c->ev0, c->stream));
-    BatchIO io{rays, (size_t)n, prim, t, u, v, cn, ct, nullptr};
-    k_zero_work<<<1, 64, 0, c->stream>>>(c->work);
+    if (claims_work(blocks, n)) k_zero_work<<<1, kWorkGroups, 0, c->stream>>>(c->work);
     if (cn)
-        k_trace_closest<true><<<blocks, kTraceBlock, 0, c->stream>>>(bvh, io, n, c->work, c->stack_ovf);
+        k_trace_closest<true><<<blocks, kTraceBlock, 0, c->stream>>>(
+            bvh, BatchIO<true>{rays, (size_t)n, prim, t, u, v, cn, ct, nullptr}, n, c->work, c->stack_ovf);
     else
-        k_trace_closest<false><<<blocks, kTraceBlock, 0, c->stream>>>(bvh, io, n, c->work, c->stack_ovf);
+        k_trace_closest<false><<<blocks, kTraceBlock, 0, c->stream>>>(
+            bvh, BatchIO<false>{rays, (size_t)n, prim, t, u, v, nullptr, nullptr, nullptr}, n, c->work, c->stack_ovf);
     DL_HIP_CHECK(c, hipGetLastError());
     DL_HIP_CHECK(c, hipEventRecord(c->ev1, c->stream));
     DL_HIP_CHECK(c, hipEventSynchronize(c->ev1));
@@ -118,14 +136,17 @@ dl_status launch_trace_shadow(Ctx* c, const float* rays, uint32_t n, uint8_t* oc
     if (n == 0) return DL_OK;
     if (n > kMaxBatchRays) return set_error(c, DL_ERR_INVALID, "more than 2^31 rays in one batch");
     BvhView bvh{c->ds.nodes, c->ds.tris};
-    const uint32_t blocks = cn ? c->trace_grid_count : c->trace_grid;
+    const uint32_t blocks = batch_blocks(cn ? c->trace_grid_count : c->trace_grid, n);
     DL_HIP_CHECK(c, hipEventRecord(c->ev0, c->stream));
-    BatchIO io{rays, (size_t)n, nullptr, nullptr, nullptr, nullptr, cn, ct, occ};
-    k_zero_work<<<1, 64, 0, c->stream>>>(c->work);
+    if (claims_work(blocks, n)) k_zero_work<<<1, kWorkGroups, 0, c->stream>>>(c->work);
     if (cn)
-        k_trace_shadow<true><<<blocks, kTraceBlock, 0, c->stream>>>(bvh, io, n, c->work, c->stack_ovf);
+        k_trace_shadow<true><<<blocks, kTraceBlock, 0, c->stream>>>(
+            bvh, BatchIO<true>{rays, (size_t)n, nullptr, nullptr, nullptr, nullptr, cn, ct, occ}, n, c->work,
+            c->stack_ovf);
     else
-        k_trace_shadow<false><<<blocks, kTraceBlock, 0, c->stream>>>(bvh, io, n, c->work, c->stack_ovf);
+        k_trace_shadow<false><<<blocks, kTraceBlock, 0, c->stream>>>(
+            bvh, BatchIO<false>{rays, (size_t)n, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, occ}, n, c->work,
+            c->stack_ovf);
     DL_HIP_CHECK(c, hipGetLastError());
     DL_HIP_CHECK(c, hipEventRecord(c->ev1, c->stream));
     DL_HIP_CHECK(c, hipEventSynchronize(c->ev1));
@@ -145,7 +166,7 @@ dl_status launch_trace_shadow(Ctx* c, const float* rays, uint32_t n, uint8_t* oc
 // (noalloc_scratch_init) and kept in g_scratch.
 constexpr uint32_t kNoAllocBlocks = 1024;
 constexpr size_t kNoAllocOvfInts = (size_t)kNoAllocBlocks * kTraceBlock * (kMaxStack - kLdsStack);
-constexpr size_t kNoAllocInts = kNoAllocOvfInts + 64;
+constexpr size_t kNoAllocInts = kNoAllocOvfInts + kWorkGroups * kWorkStride;
 static __device__ __align__(256) int scratch[kNoAllocInts];
 
 namespace {
@@ -177,11 +198,12 @@ dl_status launch_trace_closest_noalloc(Ctx* c, const float* rays, uint32_t n, ui
     }
     if (!s) return set_error(c, DL_ERR_STATE, "no scratch address for this device");
     BvhView bvh{c->ds.nodes, c->ds.tris};
-    BatchIO io{rays, (size_t)n, prim, t, u, v, nullptr, nullptr, nullptr};
+    const BatchIO<false> io{rays, (size_t)n, prim, t, u, v, nullptr, nullptr, nullptr};
+    const uint32_t blocks = batch_blocks(kNoAllocBlocks, n);
     uint32_t* work = (uint32_t*)(s + kNoAllocOvfInts);
     DL_HIP_CHECK(c, hipEventRecord(c->ev0, c->stream));
-    k_zero_work<<<1, 64, 0, c->stream>>>(work);
-    k_trace_closest<false><<<kNoAllocBlocks, kTraceBlock, 0, c->stream>>>(bvh, io, n, work, s);
+    if (claims_work(blocks, n)) k_zero_work<<<1, kWorkGroups, 0, c->stream>>>(work);
+    k_trace_closest<false><<<blocks, kTraceBlock, 0, c->stream>>>(bvh, io, n, work, s);
     DL_HIP_CHECK(c, hipGetLastError());
     DL_HIP_CHECK(c, hipEventRecord(c->ev1, c->stream));
     DL_HIP_CHECK(c, hipEventSynchronize(c->ev1));

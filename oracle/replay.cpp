@@ -39,13 +39,16 @@ inline float dot(F3 a, F3 b) {
 }
 inline F3 cross(F3 a, F3 b) { return F3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x}; }
 
+// Per axis the lo plane is the near one for a reciprocal direction >= 0, else
+// the hi plane.
 inline bool slab1(float lx, float hx, float ly, float hy, float lz, float hz, F3 o, F3 rcp, float tmin, float tmax,
                   float& n) {
-    const float a0 = (lx - o.x) * rcp.x, b0 = (hx - o.x) * rcp.x;
-    const float a1 = (ly - o.y) * rcp.y, b1 = (hy - o.y) * rcp.y;
-    const float a2 = (lz - o.z) * rcp.z, b2 = (hz - o.z) * rcp.z;
-    n = std::fmax(std::fmax(std::fmin(a0, b0), std::fmin(a1, b1)), std::fmax(std::fmin(a2, b2), tmin));
-    const float f = std::fmin(std::fmin(std::fmax(a0, b0), std::fmax(a1, b1)), std::fmin(std::fmax(a2, b2), tmax));
+    const bool px = rcp.x >= 0.0f, py = rcp.y >= 0.0f, pz = rcp.z >= 0.0f;
+    const float n0 = ((px ? lx : hx) - o.x) * rcp.x, f0 = ((px ? hx : lx) - o.x) * rcp.x;
+    const float n1 = ((py ? ly : hy) - o.y) * rcp.y, f1 = ((py ? hy : ly) - o.y) * rcp.y;
+    const float n2 = ((pz ? lz : hz) - o.z) * rcp.z, f2 = ((pz ? hz : lz) - o.z) * rcp.z;
+    n = std::fmax(std::fmax(n0, n1), std::fmax(n2, tmin));
+    const float f = std::fmin(std::fmin(f0, f1), std::fmin(f2, tmax));
     return n <= f * kFarSlack;
 }
 

@@ -43,15 +43,16 @@ constexpr int kTypes = 8;  // material queue segments (DL_BSDF_COUNT rounded up)
 enum : uint32_t { kFlagDiffuse = 1u, kFlagCamera = 2u };
 // Material-queue segment of paths that pass straight through a hidden
 // light's surface (after the BSDF types).
-constexpr int kPassQ = DL_BSDF_COUNT;
-static_assert(kPassQ < kTypes, "pass-through queue needs a segment");
+constexpr int kPassQ = DL_BSDF_COUNT + 1;
+// Segment of paths whose continuation hit an emitter (k_post -> k_post_emit).
+constexpr int kEmitQ = DL_BSDF_COUNT;
+static_assert(kPassQ < kTypes, "pass-through and emission queues need a segment each");
 
 struct Counters {
     uint32_t mat[2][kTypes];
     uint32_t ray;     // continuation rays queued (block_append index 0)
     uint32_t shadow;  // shadow rays queued (block_append index 1)
-    uint32_t emit;    // continuations that hit an emitter (k_post -> k_post_emit)
-    uint32_t pad[13];
+    uint32_t pad[14];
     unsigned long long nodes;
     unsigned long long tris;
     unsigned long long invalid;
@@ -73,7 +74,6 @@ struct RenderBufs {
     uint32_t* matq[2];
     uint32_t* rayq;
     uint32_t* shq;
-    uint32_t* emq;  // paths whose continuation hit an emitter (MIS-weighted emission pending)
     Counters* cnt;
     uint32_t* work;  // work counters of the closest-hit, then of the shadow traversal (trace.h)
     float4* film;
@@ -195,7 +195,6 @@ __global__ __launch_bounds__(kStageBlock) void k_reset(Counters* cnt, uint32_t* 
     if (t == 0) {
         cnt->ray = 0;
         cnt->shadow = 0;
-        cnt->emit = 0;
     }
     static_assert(2 * kWorkGroups <= kStageBlock, "a thread per work counter");
     if (t < 2 * (int)kWorkGroups) work[t * kWorkStride] = 0;
@@ -302,10 +301,9 @@ struct QueueIO {
     float4* __restrict__ rad;
     const uint8_t* __restrict__ sid;
     const int32_t* __restrict__ roots;
-    // a refill loads the queue entry and then the ray it names (8 measured
-    // best of 1, 8 and 16 on the 2M-triangle displaced-sphere render; for
-    // shadow rays 1 is 2% faster there but 15% slower on the MIS plates)
-    static constexpr uint32_t kRefillMin = 8, kRefillMinAny = 8;
+    // (the 1080p 64-spp render of the 2M-triangle scene takes 73.1, 72.0 and
+    // 71.1 ms with 4, 8 and 16)
+    static constexpr uint32_t kRefillMin = 16, kRefillMinAny = 16;
     __device__ __forceinline__ uint32_t entry(uint32_t i) const { return q[i]; }
     // first node of the ray's scene
     __device__ __forceinline__ int root(uint32_t p) const { return roots ? roots[sid[p]] : 0; }
@@ -708,26 +706,18 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
 // the throughput before Russian roulette, kept in the path's NEE slot (the
 // NEE contribution has been consumed) -- this keeps the rarely needed
 // emitter pdf out of k_post's registers.
-// The lanes of a wave that call it together take consecutive queue slots
-// with one atomic (the queue's order does not matter: each entry is one
-// path's own emission).
-__device__ __forceinline__ void defer_emission(const RenderBufs& rs, uint32_t p, vec3 thr) {
-    rs.nee[p] = f4(thr, 0.f);
-    const unsigned long long mask = __ballot(1);
-    const int lane = __lane_id();
-    const int leader = __ffsll((long long)mask) - 1;
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(&rs.cnt->emit, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader);
-    rs.emq[base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = p;
-}
+// The path is queued with the block's other appends: one atomic per wave on
+// the queue's counter made k_post three times as long on the MIS plates,
+// whose waves nearly all hold a light hit.
+__device__ __forceinline__ void defer_emission(const RenderBufs& rs, uint32_t p, vec3 thr) { rs.nee[p] = f4(thr, 0.f); }
 
 // Emission of the continuations k_post deferred: rad += thr * mis * Le, in
 // the order k_post would have added it (after the NEE contribution).
-__global__ __launch_bounds__(kStageBlock) void k_post_emit(SceneView s, RenderBufs rs) {
-    const uint32_t n = rs.cnt->emit;
+__global__ __launch_bounds__(kStageBlock) void k_post_emit(PassParams pp, SceneView s, RenderBufs rs, int next) {
+    const uint32_t n = rs.cnt->mat[next][kEmitQ];
+    const uint32_t* __restrict__ queue = rs.matq[next] + (size_t)kEmitQ * pp.cap;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const uint32_t p = rs.emq[i];
+        const uint32_t p = queue[i];
         const float4 h = rs.hit[p];
         const uint32_t prim = __float_as_uint(h.x);
         const float4 t4 = rs.nee[p];
@@ -799,7 +789,7 @@ __global__ __launch_bounds__(kStageBlock) void k_post(PassParams pp, SceneView s
         for (int u = 0; u < kStageItems; u++) {
             const uint32_t info = s_b[u][threadIdx.x];
             const uint32_t p = s_p[u][threadIdx.x];
-            bool alive = false;
+            bool alive = false, emits = false;
             int ntype = 0;
             if (info != kNone) {
                 if (grec) {
@@ -836,7 +826,8 @@ __global__ __launch_bounds__(kStageBlock) void k_post(PassParams pp, SceneView s
                     }
                 } else if (HIDE && (cam || info_light(info))) {
                     if (info_light(info)) {
-                        if (!cam) defer_emission(rs, p, f3(rs.thr[p]));
+                        emits = !cam;
+                        if (emits) defer_emission(rs, p, f3(rs.thr[p]));
                         rs.depth[p].y = 0;  // the record's radiance before its continuation is already kept
                         alive = true;
                         ntype = kPassQ;
@@ -846,7 +837,8 @@ __global__ __launch_bounds__(kStageBlock) void k_post(PassParams pp, SceneView s
                         ntype = info_type(info);
                     }
                 } else {
-                    if (info_light(info)) defer_emission(rs, p, f3(rs.thr[p]));
+                    emits = info_light(info);
+                    if (emits) defer_emission(rs, p, f3(rs.thr[p]));
                     const int at = HIDE ? rs.depth[p].x : depth;
                     // (at the cap no path survives, so no roulette is drawn)
                     alive = !(pp.max_depth >= 0 && at + 1 + 2 > pp.max_depth);
@@ -868,7 +860,7 @@ __global__ __launch_bounds__(kStageBlock) void k_post(PassParams pp, SceneView s
                     if (HIDE && alive) rs.depth[p].x = at + 1;
                 }
             }
-            s_b[u][threadIdx.x] = alive ? 1u << ntype : 0u;
+            s_b[u][threadIdx.x] = (alive ? 1u << ntype : 0u) | (emits ? 1u << kEmitQ : 0u);
         }
         uint32_t pv[kStageItems], bv[kStageItems];
 #pragma unroll
@@ -878,7 +870,7 @@ __global__ __launch_bounds__(kStageBlock) void k_post(PassParams pp, SceneView s
         }
         uint32_t* const mq = rs.matq[next];
         const uint32_t cap = pp.cap;
-        block_append<HIDE ? kPassQ + 1 : DL_BSDF_COUNT, kStageItems>(rs.cnt->mat[next], bv,
+        block_append<HIDE ? kPassQ + 1 : kEmitQ + 1, kStageItems>(rs.cnt->mat[next], bv,
                                                                      [&](int t, int u, uint32_t slot) {
             mq[(size_t)t * cap + slot] = pv[u];
         });
@@ -1206,7 +1198,6 @@ dl_status ensure_state(Ctx* c, uint32_t P, uint32_t pixels) {
     DL_TRY(alloc(c, rs, &rs->b.matq[1], (size_t)P * kTypes));
     DL_TRY(alloc(c, rs, &rs->b.rayq, P));
     DL_TRY(alloc(c, rs, &rs->b.shq, P));
-    DL_TRY(alloc(c, rs, &rs->b.emq, P));
     DL_TRY(alloc(c, rs, &rs->b.cnt, 1));
     DL_TRY(alloc(c, rs, &rs->b.work, 2 * kWorkGroups * kWorkStride));
     DL_TRY(alloc(c, rs, &rs->b.film, pixels));
@@ -1220,7 +1211,7 @@ static_assert(kGRecFloats == dl_sizes::kGuideRecordFloats && kGMix == dl_sizes::
               "guided buffer sizes the render service reserves");
 // the per-path bytes ensure_state allocates, as the render service reserves them
 static_assert(7 * sizeof(float4) + sizeof(uint2) + sizeof(int2) + sizeof(uint64_t) + sizeof(uint32_t) + sizeof(float2) + sizeof(uint8_t) +
-                      2 * kTypes * sizeof(uint32_t) + 3 * sizeof(uint32_t) ==
+                      2 * kTypes * sizeof(uint32_t) + 2 * sizeof(uint32_t) ==
                   dl_sizes::kStateBytesPerPath &&
               kTypes == dl_sizes::kMatQueueSegs && sizeof(float4) + 3 * sizeof(float) == dl_sizes::kFilmBytesPerPixel,
               "path state bytes the render service reserves");
@@ -1382,7 +1373,7 @@ dl_status run_bounces(Ctx* c, RenderState* rs, const PassParams& pp, const Scene
             k_post<true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur ^ 1, k, gv.rec);
         else
             k_post<false><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur ^ 1, k, gv.rec);
-        k_post_emit<<<stage_grid, kStageBlock, 0, c->stream>>>(sv, rs->b);
+        k_post_emit<<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur ^ 1);
         DL_TRY(tm.stop());
         DL_HIP_CHECK(c, hipGetLastError());
         return DL_OK;
@@ -1404,7 +1395,7 @@ dl_status run_bounces(Ctx* c, RenderState* rs, const PassParams& pp, const Scene
             shadow += s.shadow;
         }
         uint32_t live = 0;
-        for (int t = 0; t < kTypes; t++) live += s.mat[cur][t];
+        for (int t = 0; t < kTypes; t++) live += t != kEmitQ ? s.mat[cur][t] : 0u;
         if (live == 0) break;
         uint32_t len[kTypes];
         for (int t = 0; t < kTypes; t++) len[t] = s.mat[cur][t];

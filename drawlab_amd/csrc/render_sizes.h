@@ -12,10 +12,10 @@ namespace dl_sizes {
 // radiance and pending NEE term (one 16-byte vector each), the aux word (8),
 // the depth and record slot (8), the pcg32 state (8), the sample index (4),
 // the film position (8), the scene index (1), two double-buffered material queues of kMatQueueSegs
-// segments (4 bytes per path per segment each), and the ray, shadow and
-// emission queues (4 each).
+// segments (4 bytes per path per segment each), and the ray and shadow
+// queues (4 each).
 constexpr int kMatQueueSegs = 8;
-constexpr uint64_t kStateBytesPerPath = 7 * 16 + 8 + 8 + 8 + 4 + 8 + 1 + 2 * kMatQueueSegs * 4 + 3 * 4;  // 225
+constexpr uint64_t kStateBytesPerPath = 7 * 16 + 8 + 8 + 8 + 4 + 8 + 1 + 2 * kMatQueueSegs * 4 + 2 * 4;  // 221
 
 // Film: float4 accumulation (sum w L, sum w) + resolved RGB per pixel.
 constexpr uint64_t kFilmBytesPerPixel = 16 + 12;

@@ -857,7 +857,8 @@ __global__ __launch_bounds__(kStageBlock) void k_post(PassParams pp, SceneView s
                             rs.rng[p] = rng.state;
                         }
                     }
-                    if (HIDE && alive) rs.depth[p].x = at + 1;
+                    // (what the next vertex's training record is filed under)
+                    if ((HIDE || grec) && alive) rs.depth[p].x = at + 1;
                 }
             }
             s_b[u][threadIdx.x] = (alive ? 1u << ntype : 0u) | (emits ? 1u << kEmitQ : 0u);

@@ -8,6 +8,7 @@
 #include "../host/bvh_build.h"
 #include "../host/scene_prep.h"
 #include "backend.h"
+#include "dl_math.h"
 
 #include <algorithm>
 
@@ -141,7 +142,43 @@ __global__ __launch_bounds__(256) void k_copy(uint4* __restrict__ dst, const uin
     if (i0 < ntail) dtail[i0] = stail[i0];
 }
 
+// The shading record of every primitive (backend.h): one thread each.
+__global__ __launch_bounds__(256) void k_prim_recs(const float* __restrict__ pos, const uint32_t* __restrict__ idx,
+                                                   const uint32_t* __restrict__ prim_mesh,
+                                                   const MeshRec* __restrict__ meshes,
+                                                   const dl_material_desc* __restrict__ mats, size_t n,
+                                                   float4* __restrict__ recs) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+        vec3 p[3];
+        for (int k = 0; k < 3; k++) {
+            const float* q = pos + 3 * (size_t)idx[3 * i + k];
+            p[k] = v3(q[0], q[1], q[2]);
+        }
+        const uint32_t m = prim_mesh[i];
+        const MeshRec& r = meshes[m];
+        const dl_material_desc& md = mats[r.material];
+        uint32_t flags = (r.has_normals ? kRecNormals : 0u) | (r.has_tangents ? kRecTangents : 0u) |
+                         (r.has_texcoords ? kRecTexcoords : 0u);
+        for (int k = 0; k < DL_TEX_SLOTS; k++) flags |= md.tex[k] ? kRecTextured : 0u;
+        const vec3 nrm = normalized(cross(sub(p[1], p[0]), sub(p[2], p[0])));
+        recs[4 * i] = make_float4(p[0].x, p[0].y, p[0].z, __uint_as_float(m));
+        recs[4 * i + 1] = make_float4(p[1].x, p[1].y, p[1].z, __int_as_float(r.material));
+        recs[4 * i + 2] = make_float4(p[2].x, p[2].y, p[2].z, __uint_as_float(flags));
+        recs[4 * i + 3] = make_float4(nrm.x, nrm.y, nrm.z, __int_as_float(r.light));
+    }
+}
+
 }  // namespace
+
+dl_status launch_prim_recs(Ctx* c, const DevScene& ds, size_t prims, float4* recs) {
+    if (prims == 0) return DL_OK;
+    const size_t blocks = std::min<size_t>((prims + 255) / 256, 8192);
+    k_prim_recs<<<(uint32_t)blocks, 256, 0, c->stream>>>(ds.pos, ds.idx, ds.prim_mesh, (const MeshRec*)ds.meshes,
+                                                         (const dl_material_desc*)ds.materials, prims, recs);
+    DL_HIP_CHECK(c, hipGetLastError());
+    return DL_OK;
+}
+
 }  // namespace dl
 
 using namespace dl;
@@ -345,6 +382,14 @@ dl_status dl_hip_upload_scene(void* h, const dl_scene_desc* sd) {
         if (ld.type == DL_LIGHT_AREA) {
             if (ld.mesh < 0 || (uint32_t)ld.mesh >= sd->num_meshes || sd->meshes[ld.mesh].light != (int32_t)l)
                 return set_error(c, DL_ERR_INVALID, "area light must reference the mesh that references it");
+            const MeshRec& m = c->mesh_recs[ld.mesh];
+            r.prim_offset = m.prim_offset;
+            r.num_prims = m.num_prims;
+            r.cdf_offset = m.cdf_offset;
+            r.guide_offset = m.guide_offset;
+            r.guide_bits = m.guide_bits;
+            r.area_norm = m.area_norm;
+            r.has_normals = m.has_normals;
         } else if (ld.type == DL_LIGHT_ENV) {
             if (c->env_light >= 0) return set_error(c, DL_ERR_INVALID, "There is more than one envmap in the scene!");
             if (!ld.env_rgb || ld.env_width <= 0 || ld.env_height <= 0)
@@ -390,6 +435,8 @@ dl_status dl_hip_upload_scene(void* h, const dl_scene_desc* sd) {
     LightRec* dl_ = nullptr;
     DL_TRY(upload(c, &dl_, c->light_recs.data(), c->light_recs.size()));
     ds.lights = dl_;
+    DL_TRY(upload(c, &ds.recs, (const float4*)nullptr, 4 * (size_t)nf));
+    DL_TRY(launch_prim_recs(c, ds, (size_t)nf, ds.recs));
     DL_TRY(upload(c, &ds.light_cdf, cdf_all.data(), cdf_all.size()));
     DL_TRY(upload(c, &ds.light_guide, guide_all.data(), guide_all.size()));
     DL_TRY(upload(c, &ds.env_rgb, env_rgb.data(), env_rgb.size()));

@@ -31,6 +31,7 @@ struct DevScene {
     uint32_t* idx = nullptr;     // 3 * nprims (global vertex indices)
     uint32_t* prim_mesh = nullptr;  // nprims -> mesh index
     uint8_t* prim_info = nullptr;   // nprims -> material type | kPrimLight (one byte: 2 MB per 2M triangles)
+    float4* recs = nullptr;         // 4 * nprims: what shading reads of a primitive (below)
     float* uv = nullptr;         // 2 * nv   (texture coordinates; zeros for meshes without)
     // bitmap textures: texels (rgb, 0) of all textures, per texture
     // (first texel, width, height, 0)
@@ -73,6 +74,15 @@ struct MeshRec {
     int32_t pad;
 };
 
+// What the shading kernels read of one primitive, 64 bytes in one cache line
+// (k_prim_recs gathers it at upload): the three vertices, and in the fourth
+// components the mesh, the material, the flags below and the area light (-1:
+// none); the last record also holds the face normal.
+//   r0 = p0, mesh   r1 = p1, material   r2 = p2, flags   r3 = normal, light
+// One gather of four 16-byte loads instead of about sixteen dependent ones
+// (mesh, mesh record, vertex indices, vertices).
+enum : uint32_t { kRecNormals = 1u, kRecTangents = 2u, kRecTexcoords = 4u, kRecTextured = 8u };
+
 // Bucket index of an area CDF c[0..n] (c[n] = 1): entry g, for g = 0 ..
 // 2^bits, is lower_bound(c, g / 2^bits), so the lower_bound of any x in
 // [g, g + 1) / 2^bits lies in [guide[g], guide[g + 1]] -- a search of that
@@ -92,7 +102,14 @@ struct LightRec {
     float env_scale;
     int32_t env_visual;
     uint32_t env_base;  // first texel of the environment in the env_* arrays
-    int32_t pad[3];
+    // area lights: what emitter sampling reads of the emitting mesh (MeshRec)
+    uint32_t prim_offset;
+    uint32_t num_prims;
+    uint32_t cdf_offset;
+    uint32_t guide_offset;
+    uint32_t guide_bits;
+    float area_norm;
+    int32_t has_normals;
 };
 
 // Lights, background and BVH root of one scene of a layout that holds
@@ -263,6 +280,9 @@ dl_status launch_trace_closest(Ctx* c, const float* rays, uint32_t n, uint32_t* 
 dl_status launch_trace_shadow(Ctx* c, const float* rays, uint32_t n, uint8_t* occ, uint32_t* cn = nullptr,
                               uint32_t* ct = nullptr);
 dl_status noalloc_scratch_init(Ctx* c);
+// Fills recs (4 float4 per primitive) from a layout's geometry, meshes and
+// materials, on the context's stream.
+dl_status launch_prim_recs(Ctx* c, const DevScene& ds, size_t prims, float4* recs);
 int render_trace_blocks_per_cu(bool counting);
 int batch_trace_blocks_per_cu(bool counting);
 dl_status launch_trace_closest_noalloc(Ctx* c, const float* rays, uint32_t n, uint32_t* prim, float* t, float* u,

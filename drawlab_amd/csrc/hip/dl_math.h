@@ -66,7 +66,9 @@ struct Frame {
 };
 __device__ __forceinline__ Frame frame_from_normal(vec3 n) {
     vec3 t;
-    if (fabs((double)n.z - 1.0) > (double)kEpsilon && fabs((double)n.z + 1.0) > (double)kEpsilon)
+    // (the reference compares in binary64; near +-1 the binary32 difference is
+    // exact, elsewhere it is far from the bound)
+    if (fabsf(n.z - 1.0f) > kEpsilon && fabsf(n.z + 1.0f) > kEpsilon)
         t = v3(0.0f, 0.0f, 1.0f);
     else
         t = v3(1.0f, 0.0f, 0.0f);

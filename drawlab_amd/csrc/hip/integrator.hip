@@ -381,7 +381,9 @@ __device__ __forceinline__ uint32_t prim_info(const SceneView& s, uint32_t prim)
 __device__ __forceinline__ int info_type(uint32_t info) { return (int)(info & (kPrimLight - 1u)); }
 __device__ __forceinline__ bool info_light(uint32_t info) { return (info & kPrimLight) != 0; }
 // the area light of a primitive whose info has kPrimLight
-__device__ __forceinline__ int light_of(const SceneView& s, uint32_t prim) { return s.meshes[s.prim_mesh[prim]].light; }
+__device__ __forceinline__ int light_of(const SceneView& s, uint32_t prim) {
+    return __float_as_int(s.recs[4 * (size_t)prim + 3].w);
+}
 
 // First intersection (path.cpp:21-29) and a camera-ray miss (miss.cu:23-29).
 // HIDE: light surfaces are hidden (hitgroup_pgs.cu:55-64): a camera ray that
@@ -545,9 +547,8 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
                 rng.state = rs.rng[p];
                 rng.inc = ((uint64_t)rs.seq[p] << 1u) | 1u;
                 Its its;
-                int mat;
                 float prm[8];
-                shading_point(s, prim, h.z, h.w, type, its, mat, prm);
+                shading_point(s, prim, h.z, h.w, type, its, prm);
                 const float* gm = GUIDED ? gv.mix + (size_t)i * kGMix : nullptr;
                 uint32_t flags = 0;
                 // ---- emitter sampling (Scene::sampleEmitterDirection, scene.cpp:139-170)
@@ -559,9 +560,9 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
                 vec3 spectrum = v3(0, 0, 0);
                 const SceneRec sc = path_scene(s, p);
                 const int L = sc.num_lights;
-                if (L == 1) {
-                    spectrum = emitter_sample(s, s.lights[sc.light0], lx, ly, its, ds, rng);
-                } else if (L > 1) {
+                // (one emitter: the pick is exact -- index 0, lx, scale and pdf
+                // unchanged -- so it needs no path of its own)
+                if (L > 0) {
                     const float epdf = 1.f / (float)L;
                     uint32_t idx = (uint32_t)(lx * (float)L);
                     idx = idx < (uint32_t)(L - 1) ? idx : (uint32_t)(L - 1);
@@ -899,9 +900,8 @@ __global__ __launch_bounds__(kGWaves * 64) void k_guide_infer(PassParams pp, Sce
             const uint32_t p = queue[i];
             const float4 h = rs.hit[p];
             Its its;
-            int mat;
             float prm[8];
-            shading_point(s, __float_as_uint(h.x), h.z, h.w, TYPE, its, mat, prm);
+            shading_point(s, __float_as_uint(h.x), h.z, h.w, TYPE, its, prm);
             pn = v3((its.p.x - gv.lo[0]) * gv.inv[0], (its.p.y - gv.lo[1]) * gv.inv[1], (its.p.z - gv.lo[2]) * gv.inv[2]);
             wo = neg(normalized(f3(rs.ray_d[p])));
             nn = its.sh.n;
@@ -1240,6 +1240,7 @@ SceneView layout_view(const DevScene& d, int num_lights, int env_light, const fl
     s.idx = d.idx;
     s.prim_mesh = d.prim_mesh;
     s.prim_info = d.prim_info;
+    s.recs = d.recs;
     s.meshes = (const MeshRec*)d.meshes;
     s.mats = (const dl_material_desc*)d.materials;
     s.lights = (const LightRec*)d.lights;

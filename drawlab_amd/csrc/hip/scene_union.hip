@@ -241,6 +241,7 @@ dl_status build_union(Ctx* c, SceneUnion* u, const std::vector<uint64_t>& member
     DL_TRY(union_alloc(c, u, &d.idx, 3 * tot.prims));
     DL_TRY(union_alloc(c, u, &d.prim_mesh, tot.prims));
     DL_TRY(union_alloc(c, u, &d.prim_info, tot.prims));
+    DL_TRY(union_alloc(c, u, &d.recs, 4 * tot.prims));
     DL_TRY(union_alloc(c, u, &d_meshes, tot.meshes));
     DL_TRY(union_alloc(c, u, &d_mats, tot.mats));
     DL_TRY(union_alloc(c, u, &d_lights, tot.lights));
@@ -285,6 +286,9 @@ dl_status build_union(Ctx* c, SceneUnion* u, const std::vector<uint64_t>& member
         for (LightRec l : *s.lights) {
             if (l.mesh >= 0) l.mesh += (int32_t)o.meshes;
             l.env_base += (uint32_t)o.env;
+            l.prim_offset += (uint32_t)o.prims;
+            l.cdf_offset += (uint32_t)o.cdf;
+            l.guide_offset += (uint32_t)o.guide;
             lights.push_back(l);
         }
         if (e.textures > 0) {
@@ -352,6 +356,7 @@ dl_status build_union(Ctx* c, SceneUnion* u, const std::vector<uint64_t>& member
     DL_TRY(up(d_lights, lights));
     DL_TRY(up(d.tex_info, tex_info));
     DL_TRY(up(u->roots, u->root));
+    DL_TRY(launch_prim_recs(c, d, tot.prims, d.recs));
     DL_HIP_CHECK(c, hipStreamSynchronize(c->stream));  // the host vectors leave scope
     return DL_OK;
 }

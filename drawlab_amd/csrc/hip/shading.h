@@ -14,6 +14,7 @@ struct SceneView {
     const uint32_t* __restrict__ idx;
     const uint32_t* __restrict__ prim_mesh;
     const uint8_t* __restrict__ prim_info;  // material type | kPrimLight
+    const float4* __restrict__ recs;        // 4 per primitive (backend.h)
     const MeshRec* __restrict__ meshes;
     const dl_material_desc* __restrict__ mats;
     const LightRec* __restrict__ lights;
@@ -55,28 +56,40 @@ __device__ __forceinline__ vec3 ld3(const float* p, uint32_t i) { return v3(p[3 
 struct Its {
     vec3 p;
     Frame sh;
-    int mesh;
+    int mat;
+    uint32_t flags;  // kRec*
 };
+
+__device__ __forceinline__ vec3 xyz(const float4& a) { return v3(a.x, a.y, a.z); }
+
+// Position and shading normal of a hit (OCTree::rayIntersect,
+// src/tracer/accel/octree.cpp:166-209).
+__device__ __forceinline__ void hit_point(const SceneView& s, uint32_t prim, float u, float v, vec3& p, vec3& n,
+                                          int& mat, uint32_t& flags) {
+    const float4* __restrict__ r = s.recs + 4 * (size_t)prim;
+    const float4 r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3];
+    const float b0 = (1.0f - u) - v, b1 = u, b2 = v;
+    p = add(add(scale(xyz(r0), b0), scale(xyz(r1), b1)), scale(xyz(r2), b2));
+    mat = __float_as_int(r1.w);
+    flags = __float_as_uint(r2.w);
+    n = xyz(r3);
+    if (flags & kRecNormals) {
+        const uint32_t i0 = s.idx[3 * prim], i1 = s.idx[3 * prim + 1], i2 = s.idx[3 * prim + 2];
+        n = add(add(scale(ld3(s.nrm, i0), b0), scale(ld3(s.nrm, i1), b1)), scale(normalized(ld3(s.nrm, i2)), b2));
+    }
+}
 
 // OCTree::rayIntersect record construction (src/tracer/accel/octree.cpp:166-209);
 // the anisotropic GGX frame follows src/optix/cuda/shader_common.h:121-133 and
 // include/optix/math/onb.h:11-33.
 __device__ __forceinline__ void make_its(const SceneView& s, uint32_t prim, float u, float v, bool want_tangent,
                                          Its& its) {
-    const uint32_t m = s.prim_mesh[prim];
-    const MeshRec& mr = s.meshes[m];
-    const uint32_t i0 = s.idx[3 * prim], i1 = s.idx[3 * prim + 1], i2 = s.idx[3 * prim + 2];
-    const float b0 = (1.0f - u) - v, b1 = u, b2 = v;
-    const vec3 p0 = ld3(s.pos, i0), p1 = ld3(s.pos, i1), p2 = ld3(s.pos, i2);
-    its.mesh = (int)m;
-    its.p = add(add(scale(p0, b0), scale(p1, b1)), scale(p2, b2));
-    if (mr.has_normals) {
-        const vec3 n = add(add(scale(ld3(s.nrm, i0), b0), scale(ld3(s.nrm, i1), b1)), scale(normalized(ld3(s.nrm, i2)), b2));
-        its.sh = frame_from_normal(n);
-    } else {
-        its.sh = frame_from_normal(normalized(cross(sub(p1, p0), sub(p2, p0))));
-    }
-    if (want_tangent && mr.has_tangents) {
+    vec3 n;
+    hit_point(s, prim, u, v, its.p, n, its.mat, its.flags);
+    its.sh = frame_from_normal(n);
+    if (want_tangent && (its.flags & kRecTangents)) {
+        const uint32_t i0 = s.idx[3 * prim], i1 = s.idx[3 * prim + 1], i2 = s.idx[3 * prim + 2];
+        const float b0 = (1.0f - u) - v, b1 = u, b2 = v;
         const vec3 t0 = ld3(s.tan, i0);
         if (!(isnan(t0.x) || isnan(t0.y) || isnan(t0.z))) {
             const vec3 st = normalized(add(add(scale(t0, b0), scale(ld3(s.tan, i1), b1)), scale(ld3(s.tan, i2), b2)));
@@ -89,9 +102,8 @@ __device__ __forceinline__ void make_its(const SceneView& s, uint32_t prim, floa
 // ---- bitmap textures (reference GPU path) ---------------------------------
 // Texture coordinates of a hit as the reference's GPU path interpolates them
 // (src/optix/cuda/shader_common.h:36-45): zero for a mesh without them.
-__device__ __forceinline__ float2 hit_texcoord(const SceneView& s, uint32_t prim, float u, float v) {
-    const MeshRec& mr = s.meshes[s.prim_mesh[prim]];
-    if (!mr.has_texcoords) return make_float2(0.0f, 0.0f);
+__device__ __forceinline__ float2 hit_texcoord(const SceneView& s, uint32_t prim, uint32_t flags, float u, float v) {
+    if (!(flags & kRecTexcoords)) return make_float2(0.0f, 0.0f);
     const uint32_t i0 = s.idx[3 * prim], i1 = s.idx[3 * prim + 1], i2 = s.idx[3 * prim + 2];
     const float b0 = (1.0f - u) - v;
     return make_float2((b0 * s.uv[2 * i0] + u * s.uv[2 * i1]) + v * s.uv[2 * i2],
@@ -127,22 +139,20 @@ __device__ __forceinline__ vec3 tex_sample(const SceneView& s, int t, float u, f
               (t00.z * bx + t10.z * ax) * by + (t01.z * bx + t11.z * ax) * ay);
 }
 
-__device__ __forceinline__ bool has_textures(const dl_material_desc& m) {
-    return (m.tex[0] | m.tex[1] | m.tex[2] | m.tex[3] | m.tex[4]) != 0;
-}
-
 // The first 8 material parameters at a surface point: textured slots
 // replaced by their texture values (diffuse.cu:16-19 albedo;
 // aniso_ggx.cu:17-36 pd, ps, axay).
-__device__ __forceinline__ void resolve_params(const SceneView& s, const dl_material_desc& m, float2 tc, float* p) {
+__device__ __forceinline__ void resolve_params(const SceneView& s, const dl_material_desc& m, int type, bool textured,
+                                               float2 tc, float* p) {
     for (int k = 0; k < 8; k++) p[k] = m.params[k];
-    if (m.type == DL_BSDF_DIFFUSE && m.tex[DL_TEX_ALBEDO]) {
+    if (!textured) return;
+    if (type == DL_BSDF_DIFFUSE && m.tex[DL_TEX_ALBEDO]) {
         const vec3 a = tex_sample(s, m.tex[DL_TEX_ALBEDO] - 1, tc.x, tc.y);
         p[0] = a.x;
         p[1] = a.y;
         p[2] = a.z;
     }
-    if (m.type == DL_BSDF_ANISO_GGX) {
+    if (type == DL_BSDF_ANISO_GGX) {
         if (m.tex[DL_TEX_PD]) {
             const vec3 a = tex_sample(s, m.tex[DL_TEX_PD] - 1, tc.x, tc.y);
             p[0] = a.x;
@@ -236,41 +246,76 @@ __device__ __forceinline__ Frame map_frame(const SceneView& s, uint32_t prim, fl
 // reference CPU record (make_its); for a textured material the texture
 // values, and for aniso_ggx with normal / tangent maps the mapped frame.
 __device__ __forceinline__ void shading_point(const SceneView& s, uint32_t prim, float u, float v, int type, Its& its,
-                                              int& mat, float (&p)[8]) {
+                                              float (&p)[8]) {
     make_its(s, prim, u, v, type == DL_BSDF_ANISO_GGX, its);
-    mat = s.meshes[its.mesh].material;
-    const dl_material_desc& md = s.mats[mat];
+    const dl_material_desc& md = s.mats[its.mat];
+    const bool textured = (its.flags & kRecTextured) != 0;
     float2 tc = make_float2(0.0f, 0.0f);
-    if (has_textures(md)) {
-        tc = hit_texcoord(s, prim, u, v);
+    if (textured) {
+        tc = hit_texcoord(s, prim, its.flags, u, v);
         if (type == DL_BSDF_ANISO_GGX && (md.tex[DL_TEX_NORMAL] | md.tex[DL_TEX_TANGENT]) != 0)
             its.sh = map_frame(s, prim, u, v, md, tc);
     }
-    resolve_params(s, md, tc, p);
+    resolve_params(s, md, type, textured, tc, p);
 }
 
-// Shading normal only (emitter hits need its.p and shFrame.n).
+// Position and shading normal only (emitter hits).
 __device__ __forceinline__ void hit_point_normal(const SceneView& s, uint32_t prim, float u, float v, vec3& p, vec3& n) {
-    const uint32_t m = s.prim_mesh[prim];
-    const MeshRec& mr = s.meshes[m];
-    const uint32_t i0 = s.idx[3 * prim], i1 = s.idx[3 * prim + 1], i2 = s.idx[3 * prim + 2];
-    const float b0 = (1.0f - u) - v, b1 = u, b2 = v;
-    const vec3 p0 = ld3(s.pos, i0), p1 = ld3(s.pos, i1), p2 = ld3(s.pos, i2);
-    p = add(add(scale(p0, b0), scale(p1, b1)), scale(p2, b2));
-    if (mr.has_normals)
-        n = add(add(scale(ld3(s.nrm, i0), b0), scale(ld3(s.nrm, i1), b1)), scale(normalized(ld3(s.nrm, i2)), b2));
-    else
-        n = normalized(cross(sub(p1, p0), sub(p2, p0)));
+    int mat;
+    uint32_t flags;
+    hit_point(s, prim, u, v, p, n, mat, flags);
 }
 
 // ---- warps (src/core/math/wrap.cpp), binary64 transcendentals ------------
-__device__ __forceinline__ float dsqrtf(float x) { return (float)sqrt((double)x); }
+// The reference's (float)sqrt((double)x): a binary64 square root (or quotient)
+// of binary32 operands rounds to binary32 as the binary32 operation does, as
+// binary64 carries more than 2 * 24 + 2 digits.
+__device__ __forceinline__ float dsqrtf(float x) { return sqrtf(x); }
+
+// sin and cos in binary64 of an angle of at most a few turns: reduced by the
+// nearest multiple of pi / 2 (two parts), then the Taylor series to r^17 and
+// r^18, whose next terms are below 2^-60 on [-pi/4, pi/4].  Rounded to
+// binary32 it gives libm's sin and cos for every angle tried (8e7 floats up
+// to 2 pi).  The library functions also reduce huge arguments, which took the
+// shading kernels registers and code for a case that cannot occur.
+__device__ __forceinline__ void sincos_small(double x, double& s, double& c) {
+    const double n = __builtin_rint(x * 0.63661977236758134308);
+    double r = __builtin_fma(-n, 1.57079632679489655800, x);
+    r = __builtin_fma(-n, 6.12323399573676603587e-17, r);
+    const double z = r * r;
+    double p = 1.0 / 355687428096000.0;
+    p = __builtin_fma(p, z, -1.0 / 1307674368000.0);
+    p = __builtin_fma(p, z, 1.0 / 6227020800.0);
+    p = __builtin_fma(p, z, -1.0 / 39916800.0);
+    p = __builtin_fma(p, z, 1.0 / 362880.0);
+    p = __builtin_fma(p, z, -1.0 / 5040.0);
+    p = __builtin_fma(p, z, 1.0 / 120.0);
+    p = __builtin_fma(p, z, -1.0 / 6.0);
+    const double sr = __builtin_fma(p * z, r, r);
+    double q = -1.0 / 6402373705728000.0;
+    q = __builtin_fma(q, z, 1.0 / 20922789888000.0);
+    q = __builtin_fma(q, z, -1.0 / 87178291200.0);
+    q = __builtin_fma(q, z, 1.0 / 479001600.0);
+    q = __builtin_fma(q, z, -1.0 / 3628800.0);
+    q = __builtin_fma(q, z, 1.0 / 40320.0);
+    q = __builtin_fma(q, z, -1.0 / 720.0);
+    q = __builtin_fma(q, z, 1.0 / 24.0);
+    // 1 - z / 2 + z^2 q, with what 1 - z / 2 rounds away added back
+    const double h = 0.5 * z, w = 1.0 - h;
+    const double cr = w + __builtin_fma(z * z, q, (1.0 - w) - h);
+    const int k = (int)n;
+    const double a = (k & 1) ? cr : sr, b = (k & 1) ? sr : cr;
+    s = (k & 2) ? -a : a;
+    c = ((k + 1) & 2) ? -b : b;
+}
 
 __device__ __forceinline__ vec3 sq_cos_hemi(float sx, float sy) {
     const float r = dsqrtf(sx);
     const float th = 2 * kPi * sy;
-    const float px = (float)((double)r * cos((double)th));
-    const float py = (float)((double)r * sin((double)th));
+    double st, ct;
+    sincos_small((double)th, st, ct);
+    const float px = (float)((double)r * ct);
+    const float py = (float)((double)r * st);
     float sum = 0.0f;
     sum = sum + px * px;
     sum = sum + py * py;
@@ -280,8 +325,10 @@ __device__ __forceinline__ float sq_cos_hemi_pdf(vec3 v) { return v.z <= 0 ? 0.0
 __device__ __forceinline__ vec3 sq_beckmann(float sx, float sy, float alpha) {
     const float theta = (float)atan(sqrt((double)(-alpha * alpha) * log((double)(1 - sx))));
     const float phi = 2 * kPi * sy;
-    const double st = sin((double)theta);
-    return v3((float)(st * cos((double)phi)), (float)(st * sin((double)phi)), (float)cos((double)theta));
+    double st, ct, sp, cp;
+    sincos_small((double)theta, st, ct);
+    sincos_small((double)phi, sp, cp);
+    return v3((float)(st * cp), (float)(st * sp), (float)ct);
 }
 __device__ __forceinline__ float sq_beckmann_pdf(vec3 m, float alpha) {
     if (m.z <= 0) return 0;
@@ -340,7 +387,7 @@ __device__ __forceinline__ float mf_g1(vec3 wv, vec3 wh, float alpha) {  // micr
     if (c <= 0) return 0.0f;
     const float tmp = 1 - wv.z * wv.z;
     const float tanT = tmp <= 0.0f ? 0.0f : dsqrtf(tmp) / wv.z;
-    const float b = (float)(1.0 / (double)(alpha * tanT));
+    const float b = 1.0f / (alpha * tanT);
     const double bd = b;
     return bd < 1.6 ? (float)((3.535 * bd + 2.181 * bd * bd) / (1 + 2.276 * bd + 2.577 * bd * bd)) : 1.0f;
 }
@@ -354,14 +401,16 @@ __device__ __forceinline__ float ggx_d(vec3 m, float ax, float ay) {  // include
 __device__ __forceinline__ vec3 ggx_sample(float sx, float sy, float ax, float ay) {  // wrap.h:70-77
     const double sz = sqrt((double)sx), sw = sqrt((double)(1 - sx));
     const float ang = 2 * kPi * sy;
-    const float x = (float)((double)ax * sz / sw * cos((double)ang));
-    const float y = (float)((double)ay * sz / sw * sin((double)ang));
+    double sa, ca;
+    sincos_small((double)ang, sa, ca);
+    const float x = (float)((double)ax * sz / sw * ca);
+    const float y = (float)((double)ay * sz / sw * sa);
     return normalized(v3(-x, -y, 1));
 }
 __device__ __forceinline__ float ggx_g1(vec3 v, float ax, float ay) {  // aniso_ggx.cu:9-15
     if (v.z <= 0.0f) return 0.0f;
     const vec3 vv = v3(v.x * ax, v.y * ay, v.z);
-    return (float)(2.0 * (double)v.z / (double)(v.z + length(vv)));
+    return (2.0f * v.z) / (v.z + length(vv));
 }
 __device__ __forceinline__ float schlick(float ldoth) {  // aniso_ggx.cu:53-58
     const float F0 = 0.04f;
@@ -641,23 +690,23 @@ __device__ __forceinline__ uint32_t cdf_sample_reuse(const float* __restrict__ c
 __device__ inline vec3 emitter_sample(const SceneView& s, const LightRec& e, float sx, float sy, const Its& its,
                                       DirSample& ds, Pcg32& rng) {
     if (e.type == DL_LIGHT_AREA) {
-        const MeshRec& m = s.meshes[e.mesh];
         float x = sx;
-        const uint32_t f = cdf_sample_reuse(s.light_cdf + m.cdf_offset, m.num_prims, s.light_guide + m.guide_offset,
-                                            m.guide_bits, x) +
-                           m.prim_offset;
-        const uint32_t i0 = s.idx[3 * f], i1 = s.idx[3 * f + 1], i2 = s.idx[3 * f + 2];
-        const vec3 p0 = ld3(s.pos, i0), p1 = ld3(s.pos, i1), p2 = ld3(s.pos, i2);
+        const uint32_t f = cdf_sample_reuse(s.light_cdf + e.cdf_offset, e.num_prims, s.light_guide + e.guide_offset,
+                                            e.guide_bits, x) +
+                           e.prim_offset;
+        const float4* __restrict__ r = s.recs + 4 * (size_t)f;
+        const vec3 p0 = xyz(r[0]), p1 = xyz(r[1]), p2 = xyz(r[2]);
         const vec3 b = sq_triangle(x, sy);
         const vec3 position = add(add(scale(p0, b.x), scale(p1, b.y)), scale(p2, b.z));
         vec3 normal;
-        if (m.has_normals)
+        if (e.has_normals) {
+            const uint32_t i0 = s.idx[3 * f], i1 = s.idx[3 * f + 1], i2 = s.idx[3 * f + 2];
             normal = add(add(scale(ld3(s.nrm, i0), b.x), scale(ld3(s.nrm, i1), b.y)), scale(ld3(s.nrm, i2), b.z));
-        else
+        } else
             normal = cross(sub(p1, p0), sub(p2, p1));
         normal = normalized(normal);
         ds = dir_sample(its.p, position, normal);
-        const float pA = m.area_norm;
+        const float pA = e.area_norm;
         const float dp = fmax0(dot(normal, neg(ds.d)), 0.0f);
         const float pw = dp != 0 ? pA * ds.dist * ds.dist / dp : 0;
         ds.pdf = pw;
@@ -690,11 +739,17 @@ __device__ inline vec3 emitter_sample(const SceneView& s, const LightRec& e, flo
     const float phi = (float)((double)u * 2.0 * (double)kPi - (double)kPi);
     const float step = kPi / (float)e.env_h;
     const float th0 = (float)py * step;
-    const float c0 = (float)cos((double)th0), c1 = (float)cos((double)(th0 + step));
+    double sn, cs;
+    sincos_small((double)th0, sn, cs);
+    const float c0 = (float)cs;
+    sincos_small((double)(th0 + step), sn, cs);
+    const float c1 = (float)cs;
     const float ct = c0 * (1.0f - xz) + c1 * xz;
     const float theta = (float)acos((double)ct);
-    const float st = (float)sin((double)theta);
-    const vec3 dir = v3((float)cos((double)phi) * st, ct, (float)sin((double)phi) * st);
+    sincos_small((double)theta, sn, cs);
+    const float st = (float)sn;
+    sincos_small((double)phi, sn, cs);
+    const vec3 dir = v3((float)cs * st, ct, (float)sn * st);
     ds.d = dir;
     ds.dist = 1e16f;
     ds.delta = false;
@@ -717,7 +772,7 @@ __device__ __forceinline__ float pdf_emitter_direction(const SceneView& s, int l
     const LightRec& e = s.lights[l];
     float p;
     if (e.type == DL_LIGHT_AREA) {
-        const float pA = s.meshes[e.mesh].area_norm;
+        const float pA = e.area_norm;
         const float dp = fmax0(dot(ds.n, neg(ds.d)), 0.0f);
         p = dp != 0 ? pA * ds.dist * ds.dist / dp : 0;
     } else if (e.type == DL_LIGHT_POINT) {

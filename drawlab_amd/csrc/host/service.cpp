@@ -58,7 +58,8 @@ constexpr uint64_t kPathsPerPass = 64u << 20;  // paths per pass of a job or a s
 constexpr uint64_t kStateBytesPerPath = dl_sizes::kStateBytesPerPath;  // path state + queues
 constexpr uint64_t kFilmBytesPerPixel = dl_sizes::kFilmBytesPerPixel;  // accumulation film + resolved RGB
 constexpr uint64_t kBytesPerVertex = 44;        // positions, normals, tangents, texture coordinates
-constexpr uint64_t kBytesPerPrim = 16 + 112 + 256;  // indices + mesh map, BVH nodes + triangles, build scratch
+// indices + mesh map, shading record, BVH nodes + triangles, build scratch
+constexpr uint64_t kBytesPerPrim = 16 + 64 + 112 + 256;
 constexpr uint64_t kBytesPerTexel = 32;         // environment texels + alias tables
 constexpr uint64_t kSlackBytes = 4u << 20;
 

@@ -58,6 +58,8 @@ struct Counters {
     unsigned long long invalid;
     unsigned long long nodes_sh;  // shadow rays: node visits, triangle tests (counting renders)
     unsigned long long tris_sh;
+    unsigned long long fin_closest;  // queries traced by k_finish
+    unsigned long long fin_shadow;
 };
 
 // Device buffers of a render (plain pointers: passed by value to kernels).
@@ -340,7 +342,7 @@ __global__ __launch_bounds__(kTraceBlock, COUNT ? 4 : 8) void k_trace_queue(BvhV
     LaneStack stk{lds, (int)threadIdx.x, kTraceBlock, ovf + g, G};
     QueueIO io{rs.rayq, rs.ray_o, rs.ray_d, rs.hit, nullptr, nullptr, rs.sid, rs.roots};
     TraceCounters cnt;
-    traverse_persistent<false, COUNT>(bvh, trace_work(rs.work, n), stk, io, cnt);
+    traverse_persistent<false, COUNT>(bvh, trace_work(rs.work, n, grid_wave(), grid_waves()), stk, io, cnt);
     if (COUNT) {
         wave_add(&rs.cnt->nodes, cnt.nodes);
         wave_add(&rs.cnt->tris, cnt.tris);
@@ -355,10 +357,36 @@ __global__ __launch_bounds__(kTraceBlock, COUNT ? 4 : 8) void k_shadow_queue(Bvh
     LaneStack stk{lds, (int)threadIdx.x, kTraceBlock, ovf + g, G};
     QueueIO io{rs.shq, rs.ray_o, rs.sh_d, nullptr, rs.nee, rs.rad, rs.sid, rs.roots};
     TraceCounters cnt;
-    traverse_persistent<true, COUNT>(bvh, trace_work(rs.work + kWorkGroups * kWorkStride, n), stk, io, cnt);
+    traverse_persistent<true, COUNT>(bvh, trace_work(rs.work + kWorkGroups * kWorkStride, n, grid_wave(), grid_waves()), stk, io, cnt);
     if (COUNT) {
         wave_add(&rs.cnt->nodes_sh, cnt.nodes);
         wave_add(&rs.cnt->tris_sh, cnt.tris);
+    }
+}
+
+// Both queries of a bounce of few rays in one launch: the grid's waves are
+// shared out in proportion to the rays, and each goes on with the other query
+// when its own has no more rays, so that the two wait for one slowest ray.
+__global__ __launch_bounds__(kTraceBlock, 8) void k_trace_both(BvhView bvh, RenderBufs rs, int* __restrict__ ovf) {
+    __shared__ int lds[kLdsStack * kTraceBlock];
+    const uint32_t nc = rs.cnt->ray, ns = rs.cnt->shadow;
+    const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x, G = gridDim.x * kTraceBlock;
+    LaneStack stk{lds, (int)threadIdx.x, kTraceBlock, ovf + g, G};
+    const uint32_t wave = grid_wave(), waves = grid_waves();
+    // (at most 2^24 rays of each and 2^13 waves)
+    uint32_t wc = nc + ns != 0 ? (uint32_t)((float)waves * (float)nc / (float)(nc + ns)) : waves;
+    wc = min(waves - 1u, max(1u, wc));
+    TraceCounters cnt;
+    for (int k = 0; k < 2; k++) {
+        if ((wave < wc) == (k == 0)) {
+            QueueIO io{rs.rayq, rs.ray_o, rs.ray_d, rs.hit, nullptr, nullptr, rs.sid, rs.roots};
+            traverse_persistent<false, false>(bvh, trace_work(rs.work, nc, wave, wc), stk, io, cnt);
+        } else {
+            QueueIO io{rs.shq, rs.ray_o, rs.sh_d, nullptr, rs.nee, rs.rad, rs.sid, rs.roots};
+            traverse_persistent<true, false>(
+                bvh, trace_work(rs.work + kWorkGroups * kWorkStride, ns, wave >= wc ? wave - wc : 0xffffffffu, waves - wc),
+                stk, io, cnt);
+        }
     }
 }
 
@@ -510,7 +538,171 @@ __global__ __launch_bounds__(kStageBlock) void k_normals(SceneView s, RenderBufs
 }
 
 // One bounce at the current vertex: emitter sampling + BSDF sampling
-// (path.cpp:32-69).
+// (path.cpp:32-69).  `d`: the direction the vertex was reached in; thr, eta
+// and rng are the path's, advanced; dep: its depth and, on return, 1 + the
+// slot of its training record (GUIDED, 0: none).  What the vertex leads to is
+// handed to `out` as it arises: shadow(contrib, dir, dist) for an emitter
+// sample that a shadow ray decides, add(contrib) for one that needs none,
+// origin(o) of the rays that leave, spawn(dir) for the continuation, and
+// vertex(pdf, flags) for the MIS of what it hits.
+template <bool GUIDED, class Out>
+__device__ __forceinline__ void shade_vertex(const PassParams& pp, const SceneView& s, int type, uint32_t p,
+                                             const float4& h, const vec3& d, vec3& thr, float& eta, Pcg32& rng,
+                                             const GuideView& gv, const float* gm, int2& dep, Out& out) {
+    const uint32_t prim = __float_as_uint(h.x);
+    Its its;
+    float prm[8];
+    shading_point(s, prim, h.z, h.w, type, its, prm);
+    bool want_shadow = false;
+    // ---- emitter sampling (Scene::sampleEmitterDirection, scene.cpp:139-170)
+    float lx = rng.next_float();
+    const float ly = rng.next_float();
+    DirSample ds;
+    ds.pdf = 0.0f;
+    ds.delta = false;
+    vec3 spectrum = v3(0, 0, 0);
+    const SceneRec sc = path_scene(s, p);
+    const int L = sc.num_lights;
+    // (one emitter: the pick is exact -- index 0, lx, scale and pdf
+    // unchanged -- so it needs no path of its own)
+    if (L > 0) {
+        const float epdf = 1.f / (float)L;
+        uint32_t idx = (uint32_t)(lx * (float)L);
+        idx = idx < (uint32_t)(L - 1) ? idx : (uint32_t)(L - 1);
+        lx = lx * (float)L - (float)idx;
+        spectrum = emitter_sample(s, s.lights[sc.light0 + (int)idx], lx, ly, its, ds, rng);
+        spectrum = scale(spectrum, (float)L);
+        ds.pdf *= epdf;
+    }
+    const vec3 wi = to_local(its.sh, neg(normalized(d)));
+    if (ds.pdf > 0) {
+        BRec q;
+        q.wi = wi;
+        q.wo = to_local(its.sh, ds.d);
+        q.eta = 1.f;
+        q.measure = kMeasureSolidAngle;
+        const vec3 bv = bsdf_eval(type, prm, q);
+        float bp = bsdf_pdf(type, prm, q);
+        // with the proposal, directions come from the 50/50 mixture
+        // of BSDF and proposal sampling: its pdf enters the MIS
+        if (GUIDED && gv.frac > 0.0f && guide_material(type, prm))
+            bp = (1.0f - gv.frac) * bp + gv.frac * guide_pdf(gm, ds.d);
+        const float mis = ds.delta ? 1.0f : mis_weight(ds.pdf, bp);
+        const vec3 contrib = mul(mul(scale(thr, mis), bv), spectrum);
+        if (csum(spectrum) > 0) {
+            out.shadow(contrib, ds.d, ds.dist - pp.eps);  // from the continuation's origin
+            want_shadow = true;
+        } else {
+            out.add(contrib);
+        }
+    }
+    // ---- BSDF sampling
+    BRec br;
+    br.wi = wi;
+    br.wo = v3(0, 0, 0);
+    br.eta = 1.f;
+    br.measure = kMeasureUnknown;
+    vec3 fr;
+    float prev_pdf;
+    vec3 wd = v3(0.0f, 0.0f, 0.0f);
+    if (GUIDED) {
+        // one-sample MIS: proposal with probability frac, else
+        // the BSDF; the weight divides by the mixture density
+        const float fg = guide_material(type, prm) ? gv.frac : 0.0f;
+        const float us = rng.next_float();
+        const float bx = rng.next_float();
+        const float by = rng.next_float();
+        if (us < fg) {
+            wd = guide_sample(gm, bx, by);
+            br.wo = to_local(its.sh, wd);
+            br.measure = kMeasureSolidAngle;
+            br.eta = 1.0f;
+            const float pb = bsdf_pdf(type, prm, br);
+            const float pm = (1.0f - fg) * pb + fg * guide_pdf(gm, wd);
+            fr = (br.wo.z > 0.0f && pm > 0.0f) ? scale(bsdf_eval(type, prm, br), br.wo.z / pm)
+                                               : v3(0.0f, 0.0f, 0.0f);
+            prev_pdf = pm;
+        } else {
+            const vec3 f0 = bsdf_sample(type, prm, br, bx, by);
+            wd = to_world(its.sh, br.wo);
+            const float pb = bsdf_pdf(type, prm, br);
+            const float pm = fg > 0.0f ? (1.0f - fg) * pb + fg * guide_pdf(gm, wd) : pb;
+            fr = pm > 0.0f ? scale(f0, pb / pm) : v3(0.0f, 0.0f, 0.0f);
+            prev_pdf = pm;
+        }
+    } else {
+        const float bx = rng.next_float();
+        const float by = rng.next_float();
+        fr = bsdf_sample(type, prm, br, bx, by);
+        prev_pdf = bsdf_pdf(type, prm, br);
+    }
+    thr = mul(thr, fr);
+    eta *= br.eta;
+    const bool cont = !is_zero(thr);
+    // the origin of the continuation and of the shadow ray
+    if (want_shadow || cont) out.origin(its.p);
+    if (cont) out.spawn(to_world(its.sh, br.wo));
+    out.vertex(prev_pdf, bsdf_is_diffuse(type) ? (uint32_t)kFlagDiffuse : 0u);
+    const int depth0 = dep.x;
+    dep.y = 0;
+    if (GUIDED && gv.rec && cont && guide_material(type, prm)) {
+        // training record of this vertex (its radiance before the
+        // continuation is completed by k_post)
+        const uint32_t depth = (uint32_t)depth0;
+        const uint32_t slot = (p / gv.rec_stride) * kGRecDepth + depth;
+        if (depth < (uint32_t)kGRecDepth && p % gv.rec_stride == 0 && slot < gv.rec_cap) {
+            float* r = gv.rec + (size_t)slot * kGRecFloats;
+            const vec3 wo = neg(normalized(d));
+            r[kRecPos] = (its.p.x - gv.lo[0]) * gv.inv[0];
+            r[kRecPos + 1] = (its.p.y - gv.lo[1]) * gv.inv[1];
+            r[kRecPos + 2] = (its.p.z - gv.lo[2]) * gv.inv[2];
+            r[kRecWo] = wo.x;
+            r[kRecWo + 1] = wo.y;
+            r[kRecWo + 2] = wo.z;
+            r[kRecN] = its.sh.n.x;
+            r[kRecN + 1] = its.sh.n.y;
+            r[kRecN + 2] = its.sh.n.z;
+            r[kRecRough] = guide_roughness(type, prm);
+            r[kRecDir] = wd.x;
+            r[kRecDir + 1] = wd.y;
+            r[kRecDir + 2] = wd.z;
+            r[kRecPdf] = prev_pdf;
+            r[kRecThr] = thr.x;
+            r[kRecThr + 1] = thr.y;
+            r[kRecThr + 2] = thr.z;
+            r[kRecPath] = __uint_as_float(p);
+            r[kRecValid] = 1.0f;
+            dep.y = (int)slot + 1;
+        }
+    }
+}
+
+// A vertex's results in the path's memory.
+struct PathMemory {
+    const RenderBufs& rs;
+    uint32_t p;
+    float eps;
+    bool want_shadow, want_cont;
+    __device__ __forceinline__ void shadow(const vec3& contrib, const vec3& dir, float dist) {
+        rs.nee[p] = f4(contrib, 0.f);
+        rs.sh_d[p] = f4(dir, dist);
+        want_shadow = true;
+    }
+    // (the path's radiance is read and written only here: the traversal and
+    // post read it next)
+    __device__ __forceinline__ void add(const vec3& contrib) {
+        rs.rad[p] = f4(dl::add(f3(rs.rad[p]), contrib), 0.f);
+    }
+    __device__ __forceinline__ void origin(const vec3& o) { rs.ray_o[p] = f4(o, eps); }
+    __device__ __forceinline__ void spawn(const vec3& dir) {
+        rs.ray_d[p] = f4(dir, INFINITY);
+        want_cont = true;
+    }
+    __device__ __forceinline__ void vertex(float pdf, uint32_t flags) {
+        rs.aux[p] = make_uint2(__float_as_uint(pdf), flags);
+    }
+};
+
 // One kernel instantiation per BSDF type (the material-sorted queue of that
 // type), so each carries only its own BSDF's code and registers.
 template <int TYPE, bool GUIDED>
@@ -518,7 +710,6 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
                                                        GuideView gv, bool first, bool track) {
     const uint32_t n = rs.cnt->mat[cur][TYPE];
     const uint32_t* __restrict__ queue = rs.matq[cur] + (size_t)TYPE * pp.cap;
-    constexpr int type = TYPE;
     __shared__ uint32_t s_p[kStageItems][kStageBlock];
     __shared__ uint32_t s_b[kStageItems][kStageBlock];
     const uint32_t items = stage_items(n);
@@ -528,12 +719,11 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
 #pragma unroll 1
         for (int u = 0; u < kStageItems; u++) {
             const uint32_t i = (uint32_t)u < items ? i0 + (uint32_t)u * kStageBlock + threadIdx.x : n;
-            bool want_shadow = false, want_cont = false;
             uint32_t p = 0;
+            bool want_shadow = false, want_cont = false;
             if (i < n) {
                 p = queue[i];
                 const float4 h = rs.hit[p];
-                const uint32_t prim = __float_as_uint(h.x);
                 const vec3 d = f3(rs.ray_d[p]);
                 // the first shading vertex of a camera path: throughput 1,
                 // eta 1, depth 0 (not stored by k_raygen)
@@ -546,140 +736,14 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
                 Pcg32 rng;
                 rng.state = rs.rng[p];
                 rng.inc = ((uint64_t)rs.seq[p] << 1u) | 1u;
-                Its its;
-                float prm[8];
-                shading_point(s, prim, h.z, h.w, type, its, prm);
                 const float* gm = GUIDED ? gv.mix + (size_t)i * kGMix : nullptr;
-                uint32_t flags = 0;
-                // ---- emitter sampling (Scene::sampleEmitterDirection, scene.cpp:139-170)
-                float lx = rng.next_float();
-                const float ly = rng.next_float();
-                DirSample ds;
-                ds.pdf = 0.0f;
-                ds.delta = false;
-                vec3 spectrum = v3(0, 0, 0);
-                const SceneRec sc = path_scene(s, p);
-                const int L = sc.num_lights;
-                // (one emitter: the pick is exact -- index 0, lx, scale and pdf
-                // unchanged -- so it needs no path of its own)
-                if (L > 0) {
-                    const float epdf = 1.f / (float)L;
-                    uint32_t idx = (uint32_t)(lx * (float)L);
-                    idx = idx < (uint32_t)(L - 1) ? idx : (uint32_t)(L - 1);
-                    lx = lx * (float)L - (float)idx;
-                    spectrum = emitter_sample(s, s.lights[sc.light0 + (int)idx], lx, ly, its, ds, rng);
-                    spectrum = scale(spectrum, (float)L);
-                    ds.pdf *= epdf;
-                }
-                const vec3 wi = to_local(its.sh, neg(normalized(d)));
-                if (ds.pdf > 0) {
-                    BRec q;
-                    q.wi = wi;
-                    q.wo = to_local(its.sh, ds.d);
-                    q.eta = 1.f;
-                    q.measure = kMeasureSolidAngle;
-                    const vec3 bv = bsdf_eval(type, prm, q);
-                    float bp = bsdf_pdf(type, prm, q);
-                    // with the proposal, directions come from the 50/50 mixture
-                    // of BSDF and proposal sampling: its pdf enters the MIS
-                    if (GUIDED && gv.frac > 0.0f && guide_material(type, prm))
-                        bp = (1.0f - gv.frac) * bp + gv.frac * guide_pdf(gm, ds.d);
-                    const float mis = ds.delta ? 1.0f : mis_weight(ds.pdf, bp);
-                    const vec3 contrib = mul(mul(scale(thr, mis), bv), spectrum);
-                    if (csum(spectrum) > 0) {
-                        rs.nee[p] = f4(contrib, 0.f);
-                        rs.sh_d[p] = f4(ds.d, ds.dist - pp.eps);  // from ray_o, written below
-                        want_shadow = true;
-                    } else {
-                        // (the path's radiance is read and written only here:
-                        // post reads it next)
-                        rs.rad[p] = f4(add(f3(rs.rad[p]), contrib), 0.f);
-                    }
-                }
-                // ---- BSDF sampling
-                BRec br;
-                br.wi = wi;
-                br.wo = v3(0, 0, 0);
-                br.eta = 1.f;
-                br.measure = kMeasureUnknown;
-                vec3 fr;
-                float prev_pdf;
-                vec3 wd = v3(0.0f, 0.0f, 0.0f);
-                if (GUIDED) {
-                    // one-sample MIS: proposal with probability frac, else
-                    // the BSDF; the weight divides by the mixture density
-                    const float fg = guide_material(type, prm) ? gv.frac : 0.0f;
-                    const float us = rng.next_float();
-                    const float bx = rng.next_float();
-                    const float by = rng.next_float();
-                    if (us < fg) {
-                        wd = guide_sample(gm, bx, by);
-                        br.wo = to_local(its.sh, wd);
-                        br.measure = kMeasureSolidAngle;
-                        br.eta = 1.0f;
-                        const float pb = bsdf_pdf(type, prm, br);
-                        const float pm = (1.0f - fg) * pb + fg * guide_pdf(gm, wd);
-                        fr = (br.wo.z > 0.0f && pm > 0.0f) ? scale(bsdf_eval(type, prm, br), br.wo.z / pm)
-                                                           : v3(0.0f, 0.0f, 0.0f);
-                        prev_pdf = pm;
-                    } else {
-                        const vec3 f0 = bsdf_sample(type, prm, br, bx, by);
-                        wd = to_world(its.sh, br.wo);
-                        const float pb = bsdf_pdf(type, prm, br);
-                        const float pm = fg > 0.0f ? (1.0f - fg) * pb + fg * guide_pdf(gm, wd) : pb;
-                        fr = pm > 0.0f ? scale(f0, pb / pm) : v3(0.0f, 0.0f, 0.0f);
-                        prev_pdf = pm;
-                    }
-                } else {
-                    const float bx = rng.next_float();
-                    const float by = rng.next_float();
-                    fr = bsdf_sample(type, prm, br, bx, by);
-                    prev_pdf = bsdf_pdf(type, prm, br);
-                }
-                thr = mul(thr, fr);
-                eta *= br.eta;
-                if (bsdf_is_diffuse(type)) flags |= kFlagDiffuse;
-                // the origin of the continuation and of the shadow ray
-                if (want_shadow || !is_zero(thr)) rs.ray_o[p] = f4(its.p, pp.eps);
-                if (!is_zero(thr)) {
-                    rs.ray_d[p] = f4(to_world(its.sh, br.wo), INFINITY);
-                    want_cont = true;
-                }
-                dep.y = 0;
-                if (GUIDED && gv.rec && want_cont && guide_material(type, prm)) {
-                    // training record of this vertex (its radiance before the
-                    // continuation is completed by k_post)
-                    const uint32_t depth = (uint32_t)dep.x;
-                    const uint32_t slot = (p / gv.rec_stride) * kGRecDepth + depth;
-                    if (depth < (uint32_t)kGRecDepth && p % gv.rec_stride == 0 && slot < gv.rec_cap) {
-                        float* r = gv.rec + (size_t)slot * kGRecFloats;
-                        const vec3 wo = neg(normalized(d));
-                        r[kRecPos] = (its.p.x - gv.lo[0]) * gv.inv[0];
-                        r[kRecPos + 1] = (its.p.y - gv.lo[1]) * gv.inv[1];
-                        r[kRecPos + 2] = (its.p.z - gv.lo[2]) * gv.inv[2];
-                        r[kRecWo] = wo.x;
-                        r[kRecWo + 1] = wo.y;
-                        r[kRecWo + 2] = wo.z;
-                        r[kRecN] = its.sh.n.x;
-                        r[kRecN + 1] = its.sh.n.y;
-                        r[kRecN + 2] = its.sh.n.z;
-                        r[kRecRough] = guide_roughness(type, prm);
-                        r[kRecDir] = wd.x;
-                        r[kRecDir + 1] = wd.y;
-                        r[kRecDir + 2] = wd.z;
-                        r[kRecPdf] = prev_pdf;
-                        r[kRecThr] = thr.x;
-                        r[kRecThr + 1] = thr.y;
-                        r[kRecThr + 2] = thr.z;
-                        r[kRecPath] = __uint_as_float(p);
-                        r[kRecValid] = 1.0f;
-                        dep.y = (int)slot + 1;
-                    }
-                }
+                PathMemory out{rs, p, pp.eps, false, false};
+                shade_vertex<GUIDED>(pp, s, TYPE, p, h, d, thr, eta, rng, gv, gm, dep, out);
                 rs.thr[p] = f4(thr, eta);
                 rs.rng[p] = rng.state;
-                rs.aux[p] = make_uint2(__float_as_uint(prev_pdf), flags);
                 if (track) rs.depth[p] = dep;
+                want_shadow = out.want_shadow;
+                want_cont = out.want_cont;
             }
             s_p[u][threadIdx.x] = p;
             s_b[u][threadIdx.x] = (want_cont ? 1u : 0u) | (want_shadow ? 2u : 0u);
@@ -877,6 +941,244 @@ __global__ __launch_bounds__(kStageBlock) void k_post(PassParams pp, SceneView s
             mq[(size_t)t * cap + slot] = pv[u];
         });
     }
+}
+
+// ---------------------------------------------------------------------------
+// Paths carried to their end in one launch
+// ---------------------------------------------------------------------------
+// A bounce of few paths costs its chain of launches (about 8) and the slowest
+// ray of each traversal, however few rays there are: a 64x64 thumbnail of the
+// Cornell box took 0.88 ms for 16,384 paths, and the last bounces of a 1080p
+// frame of the 2M-triangle scene about 0.4 ms each.  Once few paths are left
+// (or from the camera on, for small passes) k_finish takes them over: a wave
+// holds up to kFinishLanes paths in its lower lanes, shades them, traces their
+// continuations there and their shadow rays in the upper lanes at the same
+// time, and goes on until each has ended, without leaving its registers.
+// Every path does what the stage kernels do, operation for operation.
+constexpr uint32_t kFinishLanes = 32;
+// Paths are handed over when at most kFinishPaths are left; a pass of at most
+// kFinishCamera is carried from its camera rays on.  Measured (ms, handing
+// over at 2^16, 2^17, 2^18, 2^19 paths): the 1080p 1-spp frame of the
+// 2M-triangle scene 5.46, 5.22, 5.06, 5.31, the material zoo at 512x512x4
+// 1.87, 1.79, 1.66, 1.84; passes of 131,072 paths bounce by bounce against
+// from the camera: Cornell box 0.65, 0.34, MIS plates 0.60, 0.38, zoo 0.79,
+// 0.75; of 262,144: 0.75, 0.50, 0.70, 0.59, 0.96, 1.07, sphere 1.72, 2.02.
+constexpr uint32_t kFinishPaths = 1u << 18, kFinishCamera = 1u << 17;
+// A path ends after this many bounces in k_finish: Russian roulette leaves
+// 0.99^4096 = 1e-18 of the paths that long, and a throughput of NaN, which
+// roulette never ends, must not keep the kernel running.
+constexpr int kFinishBounces = 4096;
+// Bounces of at most this many paths trace both queries in one launch (the
+// 1080p frame takes 5.43, 5.22 and 5.04 ms with 2^20, 2^22 and 2^24, the
+// 64-spp sphere 67.3, 66.6 and 65.8); larger ones keep a launch and a time of
+// their own for each.
+constexpr uint32_t kBothPaths = 1u << 24;
+
+// A vertex's results in registers.
+struct PathRegisters {
+    vec3 nee, sh_d, o, d;
+    vec3& rad;
+    float sh_t, pdf;
+    uint32_t flags;
+    bool want_shadow, want_cont;
+    __device__ __forceinline__ void shadow(const vec3& contrib, const vec3& dir, float dist) {
+        nee = contrib;
+        sh_d = dir;
+        sh_t = dist;
+        want_shadow = true;
+    }
+    __device__ __forceinline__ void add(const vec3& contrib) { rad = dl::add(rad, contrib); }
+    __device__ __forceinline__ void origin(const vec3& org) { o = org; }
+    __device__ __forceinline__ void spawn(const vec3& dir) {
+        d = dir;
+        want_cont = true;
+    }
+    __device__ __forceinline__ void vertex(float p, uint32_t f) {
+        pdf = p;
+        flags = f;
+    }
+};
+
+// CAMERA: the pass's camera rays (path i = 0 .. pp.P - 1, from k_raygen), else
+// the paths of the material queues `cur` at bounce `depth`.
+template <bool CAMERA>
+__global__ __launch_bounds__(kStageBlock) void k_finish(PassParams pp, SceneView s, RenderBufs rs, BvhView bvh,
+                                                        int* __restrict__ ovf, int cur, int depth) {
+    __shared__ int lds[kLdsStack * kStageBlock];
+    const uint32_t lane = __lane_id();
+    uint32_t counts[DL_BSDF_COUNT], n = 0;
+    if (CAMERA) {
+        n = pp.P;
+    } else {
+#pragma unroll
+        for (int t = 0; t < DL_BSDF_COUNT; t++) {
+            counts[t] = rs.cnt->mat[cur][t];
+            n += counts[t];
+        }
+    }
+    const uint32_t waves = grid_waves();
+    const uint32_t share = (n + waves - 1) / waves;
+    uint32_t next = min(n, grid_wave() * share);
+    const uint32_t end = min(n, next + share);
+    const uint32_t g = blockIdx.x * kStageBlock + threadIdx.x;
+    LaneStack stk{lds, (int)threadIdx.x, kStageBlock, ovf + g, gridDim.x * kStageBlock};
+    bool alive = false, cam = false;
+    uint32_t p = 0;
+    int type = 0, at = 0;
+    vec3 d = v3(0, 0, 0), thr = v3(1, 1, 1), rad = v3(0, 0, 0);
+    float eta = 1.f;
+    float4 h = make_float4(0, 0, 0, 0);
+    Pcg32 rng;
+    rng.state = rng.inc = 0;
+    unsigned long long closest = 0, shadow = 0;
+    for (;;) {
+        // lanes whose path ended take the wave's next ones
+        const unsigned long long idle = __ballot(lane < kFinishLanes && !alive);
+        if (next < end && idle != 0) {
+            const uint32_t i = next + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+            if (lane < kFinishLanes && !alive && i < end) {
+                if (CAMERA) {
+                    p = i;
+                    cam = true;
+                } else {
+                    uint32_t j = i;
+                    bool found = false;
+#pragma unroll
+                    for (int t = 0; t < DL_BSDF_COUNT; t++) {
+                        if (!found && j < counts[t]) {
+                            type = t;
+                            p = rs.matq[cur][(size_t)t * pp.cap + j];
+                            found = true;
+                        }
+                        j -= counts[t];
+                    }
+                    h = rs.hit[p];
+                    d = f3(rs.ray_d[p]);
+                    rad = f3(rs.rad[p]);
+                }
+                thr = v3(1, 1, 1);
+                eta = 1.f;
+                at = depth;
+                if (!CAMERA && depth > 0) {
+                    const float4 th4 = rs.thr[p];
+                    thr = f3(th4);
+                    eta = th4.w;
+                }
+                rng.state = rs.rng[p];
+                rng.inc = ((uint64_t)rs.seq[p] << 1u) | 1u;
+                alive = true;
+            }
+            next = min(end, next + (uint32_t)__popcll(idle));
+        }
+        if (!__ballot(alive)) break;
+        // the vertex (k_shade)
+        PathRegisters v{v3(0, 0, 0), v3(0, 0, 0), v3(0, 0, 0), d, rad, 0.f, 0.f, 0u, false, false};
+        float tmin = pp.eps, tmax = INFINITY;
+        if (alive) {
+            if (CAMERA && cam) {
+                const float4 ro = rs.ray_o[p], rd = rs.ray_d[p];
+                v.o = f3(ro);
+                v.d = f3(rd);
+                tmin = ro.w;
+                tmax = rd.w;
+                v.want_cont = true;
+            } else {
+                int2 dep = make_int2(0, 0);
+                shade_vertex<false>(pp, s, type, p, h, d, thr, eta, rng, GuideView{}, nullptr, dep, v);
+            }
+        }
+        d = v.d;
+        // the continuations in the lower lanes, the shadow rays in the upper
+        closest += (unsigned long long)__popcll(__ballot(v.want_cont && !(CAMERA && cam)));
+        shadow += (unsigned long long)__popcll(__ballot(v.want_shadow));
+        const int from = (int)(lane & (kFinishLanes - 1));
+        const bool upper = lane >= kFinishLanes;
+        const int root = rs.roots ? rs.roots[rs.sid[p]] : 0;
+        RayState r;
+        r.clear();
+        r.o = v3(__shfl(v.o.x, from), __shfl(v.o.y, from), __shfl(v.o.z, from));
+        const vec3 sd = v3(__shfl(v.sh_d.x, from), __shfl(v.sh_d.y, from), __shfl(v.sh_d.z, from));
+        const float st = __shfl(v.sh_t, from);
+        const int sroot = __shfl(root, from);
+        const bool sw = __shfl((int)v.want_shadow, from) != 0;
+        r.d = upper ? sd : v.d;
+        r.tmin = upper ? pp.eps : tmin;
+        bool active = (upper ? sw : v.want_cont) && r.start(upper ? st : tmax, upper ? sroot : root);
+        bool occluded = false;
+        while (__ballot(active)) {
+            const bool tri_step = r.lj < r.ltri;
+            const bool tri_mode = wave_tests_triangles(active, tri_step);
+            if (!active || tri_step != tri_mode) continue;
+            if (tri_mode)
+                occluded = r.test_triangles(bvh, upper);
+            else
+                r.visit_node(bvh, stk);
+            active = !(occluded || (r.last && r.lj == r.ltri));
+        }
+        const bool occ = __shfl((int)occluded, (int)((lane + kFinishLanes) & 63u)) != 0;
+        if (alive) {
+            // what they lead to (the shadow traversal, k_post_camera, k_post and
+            // k_post_emit)
+            if (v.want_shadow && !occ) rad = add(rad, v.nee);
+            alive = false;
+            if (v.want_cont) {
+                h = make_float4(__uint_as_float(r.best), r.best_t, r.bu, r.bv);
+                const SceneRec sc = path_scene(s, p);
+                if (r.best == 0xffffffffu) {
+                    if (CAMERA && cam) rad = v3(0, 0, 0);
+                    if (sc.env_light >= 0) {
+                        const LightRec& e = s.lights[sc.env_light];
+                        if (CAMERA && cam) {
+                            rad = e.env_visual ? env_eval(s, e, d) : v3(sc.bg[0], sc.bg[1], sc.bg[2]);
+                        } else {
+                            float epdf;
+                            const vec3 ev = env_eval_pdf(s, e, sc.num_lights, d, epdf);
+                            const float mis = (v.flags & kFlagDiffuse) != 0 ? mis_weight(v.pdf, epdf) : 1.f;
+                            rad = add(rad, mul(scale(thr, mis), ev));
+                        }
+                    }
+                } else {
+                    const uint32_t info = prim_info(s, r.best);
+                    type = info_type(info);
+                    if (CAMERA && cam) {
+                        rad = v3(0, 0, 0);
+                        if (info_light(info)) {
+                            vec3 hp, hn;
+                            hit_point_normal(s, r.best, r.bu, r.bv, hp, hn);
+                            const vec3 le =
+                                dot(hn, neg(d)) > 0.f ? pcol(s.lights[light_of(s, r.best)].radiance) : v3(0, 0, 0);
+                            rad = add(rad, mul(v3(1.f, 1.f, 1.f), le));
+                        }
+                        alive = !(pp.max_depth >= 0 && 0 + 2 > pp.max_depth);
+                    } else {
+                        if (info_light(info)) {
+                            const int light = light_of(s, r.best);
+                            vec3 hp, hn;
+                            hit_point_normal(s, r.best, r.bu, r.bv, hp, hn);
+                            const vec3 ev = dot(hn, neg(d)) > 0.f ? pcol(s.lights[light].radiance) : v3(0, 0, 0);
+                            const DirSample hs = dir_sample(v.o, hp, hn);
+                            const float epdf = pdf_emitter_direction(s, light, sc.num_lights, hs);
+                            const float mis = (v.flags & kFlagDiffuse) != 0 ? mis_weight(v.pdf, epdf) : 1.f;
+                            rad = add(rad, mul(scale(thr, mis), ev));
+                        }
+                        alive = !(pp.max_depth >= 0 && at + 1 + 2 > pp.max_depth) && at - depth < kFinishBounces;
+                        if (alive && at >= pp.rr_depth) {
+                            const float pr = fmin0(cmax(scale(scale(thr, eta), eta)), 0.99f);
+                            if (rng.next_float() > pr)
+                                alive = false;
+                            else
+                                thr = divs(thr, pr);
+                        }
+                        at++;
+                    }
+                }
+            }
+            cam = false;
+            if (!alive) rs.rad[p] = f4(rad, 0.f);
+        }
+    }
+    if (lane == 0 && closest != 0) atomicAdd(&rs.cnt->fin_closest, closest);
+    if (lane == 0 && shadow != 0) atomicAdd(&rs.cnt->fin_shadow, shadow);
 }
 
 // Proposal mixtures for the queue of material TYPE: features of each queued
@@ -1269,6 +1571,7 @@ struct Timer {
     Ctx* c;
     RenderState* rs;
     std::vector<int>* tags;
+    std::vector<double> share;  // kTagBoth: the closest-hit queries' share of the launch's rays
     dl_status start(int tag) {
         const size_t k = tags->size();
         while (rs->evs.size() < 2 * (k + 1)) {
@@ -1277,6 +1580,7 @@ struct Timer {
             rs->evs.push_back(e);
         }
         tags->push_back(tag);
+        share.push_back(1.0);
         DL_HIP_CHECK(c, hipEventRecord(rs->evs[2 * k], c->stream));
         return DL_OK;
     }
@@ -1287,7 +1591,8 @@ struct Timer {
     }
 };
 
-enum { kTagClosest = 0, kTagShadow = 1, kTagShade = 2, kTagFilm = 3, kTagOther = 4, kTagGuide = 5, kTagTrain = 6 };
+enum { kTagClosest = 0, kTagShadow = 1, kTagShade = 2, kTagFilm = 3, kTagOther = 4, kTagGuide = 5, kTagTrain = 6,
+       kTagBoth = 7 };  // closest-hit and shadow queries in one launch: its time is shared out by rays
 
 }  // namespace
 
@@ -1296,14 +1601,30 @@ enum { kTagClosest = 0, kTagShadow = 1, kTagShade = 2, kTagFilm = 3, kTagOther =
 // path of the pass has ended.
 dl_status run_bounces(Ctx* c, RenderState* rs, const PassParams& pp, const SceneView& sv, const BvhView& bvh,
                       bool count, bool normals, bool hide, bool guided, const bool* guide_types, const GuideView& gv,
-                      const Net& net, int guide_grid, int stage_grid, int trace_grid, Timer& tm, double& closest,
+                      const Net& net, int guide_grid, int stage_grid_full, int trace_grid, Timer& tm, double& closest,
                       double& shadow) {
+    // k_finish follows the plain paths only, and only where their number of
+    // bounces is bounded
+    const bool finish = !count && !normals && !hide && !guided &&
+                        (pp.rr_depth <= 1024 || (pp.max_depth >= 0 && pp.max_depth <= 1024));
+    // (its time counts as closest-hit time, which it mostly is)
+    auto finish_grid = [&](uint32_t paths) {
+        return (int)std::min<uint32_t>((uint32_t)std::max(1, c->num_cus) * 2u, (paths + 15u) / 16u);
+    };
+    if (finish && pp.P <= kFinishCamera) {
+        DL_TRY(tm.start(kTagClosest));
+        k_finish<true><<<finish_grid(pp.P), kStageBlock, 0, c->stream>>>(pp, sv, rs->b, bvh, c->stack_ovf, 0, 0);
+        DL_TRY(tm.stop());
+        DL_HIP_CHECK(c, hipGetLastError());
+        return DL_OK;
+    }
     DL_TRY(tm.start(kTagClosest));
     if (count)
         k_trace_queue<true><<<trace_grid, kTraceBlock, 0, c->stream>>>(bvh, rs->b, c->stack_ovf);
     else
         k_trace_queue<false><<<trace_grid, kTraceBlock, 0, c->stream>>>(bvh, rs->b, c->stack_ovf);
     DL_TRY(tm.stop());
+    const int stage_grid = std::min(stage_grid_full, (int)((pp.P + kStageBlock - 1) / kStageBlock));
     DL_TRY(tm.start(kTagShade));
     if (normals)
         k_normals<<<stage_grid, kStageBlock, 0, c->stream>>>(sv, rs->b);
@@ -1321,9 +1642,12 @@ dl_status run_bounces(Ctx* c, RenderState* rs, const PassParams& pp, const Scene
     // queue length from the device counters; the host skips the shading
     // kernels of empty queues.
     const bool track = hide || gv.rec != nullptr;
-    auto bounce = [&](int k, const uint32_t* len) -> dl_status {
+    int both = -1;  // the timed launch of the last bounce that traced both queries
+    auto bounce = [&](int k, const uint32_t* len, uint32_t live) -> dl_status {
         const int cur = k & 1;
         const bool first = k == 0;
+        // no more blocks than the live paths fill
+        const int stage_grid = std::min(stage_grid_full, (int)((live + kStageBlock - 1) / kStageBlock));
         k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, rs->b.work, cur ^ 1);
         DL_TRY(tm.start(kTagShade));
         if (hide && len[kPassQ] > 0) k_pass<<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur);
@@ -1358,18 +1682,28 @@ dl_status run_bounces(Ctx* c, RenderState* rs, const PassParams& pp, const Scene
             }
         }
         DL_TRY(tm.stop());
-        DL_TRY(tm.start(kTagClosest));
-        if (count)
-            k_trace_queue<true><<<trace_grid, kTraceBlock, 0, c->stream>>>(bvh, rs->b, c->stack_ovf);
-        else
-            k_trace_queue<false><<<trace_grid, kTraceBlock, 0, c->stream>>>(bvh, rs->b, c->stack_ovf);
-        DL_TRY(tm.stop());
-        DL_TRY(tm.start(kTagShadow));
-        if (count)
-            k_shadow_queue<true><<<trace_grid, kTraceBlock, 0, c->stream>>>(bvh, rs->b, c->stack_ovf);
-        else
-            k_shadow_queue<false><<<trace_grid, kTraceBlock, 0, c->stream>>>(bvh, rs->b, c->stack_ovf);
-        DL_TRY(tm.stop());
+        both = -1;
+        if (!count && live <= kBothPaths) {
+            // a few rays per wave until the grid is full (at most 2 * live rays)
+            const int blocks = std::min(trace_grid, std::max((int)kWorkGroups, (int)((live + 3) / 4)));
+            both = (int)tm.tags->size();
+            DL_TRY(tm.start(kTagBoth));
+            k_trace_both<<<blocks, kTraceBlock, 0, c->stream>>>(bvh, rs->b, c->stack_ovf);
+            DL_TRY(tm.stop());
+        } else {
+            DL_TRY(tm.start(kTagClosest));
+            if (count)
+                k_trace_queue<true><<<trace_grid, kTraceBlock, 0, c->stream>>>(bvh, rs->b, c->stack_ovf);
+            else
+                k_trace_queue<false><<<trace_grid, kTraceBlock, 0, c->stream>>>(bvh, rs->b, c->stack_ovf);
+            DL_TRY(tm.stop());
+            DL_TRY(tm.start(kTagShadow));
+            if (count)
+                k_shadow_queue<true><<<trace_grid, kTraceBlock, 0, c->stream>>>(bvh, rs->b, c->stack_ovf);
+            else
+                k_shadow_queue<false><<<trace_grid, kTraceBlock, 0, c->stream>>>(bvh, rs->b, c->stack_ovf);
+            DL_TRY(tm.stop());
+        }
         DL_TRY(tm.start(kTagShade));
         if (hide)
             k_post<true><<<stage_grid, kStageBlock, 0, c->stream>>>(pp, sv, rs->b, cur ^ 1, k, gv.rec);
@@ -1395,13 +1729,21 @@ dl_status run_bounces(Ctx* c, RenderState* rs, const PassParams& pp, const Scene
         if (k > 0) {
             closest += s.ray;
             shadow += s.shadow;
+            if (both >= 0 && s.ray + s.shadow > 0) tm.share[both] = (double)s.ray / ((double)s.ray + s.shadow);
         }
         uint32_t live = 0;
         for (int t = 0; t < kTypes; t++) live += t != kEmitQ ? s.mat[cur][t] : 0u;
         if (live == 0) break;
+        if (finish && live <= kFinishPaths) {
+            DL_TRY(tm.start(kTagClosest));
+            k_finish<false><<<finish_grid(live), kStageBlock, 0, c->stream>>>(pp, sv, rs->b, bvh, c->stack_ovf, cur, k);
+            DL_TRY(tm.stop());
+            DL_HIP_CHECK(c, hipGetLastError());
+            break;
+        }
         uint32_t len[kTypes];
         for (int t = 0; t < kTypes; t++) len[t] = s.mat[cur][t];
-        DL_TRY(bounce(k, len));
+        DL_TRY(bounce(k, len, live));
     }
     return DL_OK;
 }
@@ -1466,7 +1808,7 @@ dl_status render(Ctx* c, const dl_render_params* prm, float* rgb_host, dl_render
     const int stage_grid = std::max(1, c->num_cus) * 8;
     const int trace_grid = (int)(count ? c->trace_grid_count : c->trace_grid);
     std::vector<int> tags;
-    Timer tm{c, rs, &tags};
+    Timer tm{c, rs, &tags, {}};
     double closest = 0, shadow = 0, paths = 0;
 
     DL_HIP_CHECK(c, hipEventRecord(c->ev0, c->stream));
@@ -1556,6 +1898,12 @@ dl_status render(Ctx* c, const dl_render_params* prm, float* rgb_host, dl_render
             switch (tags[i]) {
                 case kTagClosest: stats->ms_closest += e; stats->launches_closest += 1; break;
                 case kTagShadow: stats->ms_shadow += e; stats->launches_shadow += 1; break;
+                case kTagBoth:
+                    stats->ms_closest += e * tm.share[i];
+                    stats->ms_shadow += e * (1.0 - tm.share[i]);
+                    stats->launches_closest += 1;
+                    stats->launches_shadow += 1;
+                    break;
                 case kTagShade: stats->ms_shade += e; break;
                 case kTagFilm: stats->ms_film += e; break;
                 case kTagGuide: stats->ms_guide += e; break;
@@ -1565,8 +1913,8 @@ dl_status render(Ctx* c, const dl_render_params* prm, float* rgb_host, dl_render
         }
         DL_HIP_CHECK(c, hipMemcpy(rs->cnt_host, rs->b.cnt, sizeof(Counters), hipMemcpyDeviceToHost));
         stats->paths = paths;
-        stats->closest_rays = closest;
-        stats->shadow_rays = shadow;
+        stats->closest_rays = closest + (double)rs->cnt_host->fin_closest;
+        stats->shadow_rays = shadow + (double)rs->cnt_host->fin_shadow;
         stats->invalid_samples = (double)rs->cnt_host->invalid;
         stats->nodes_closest = (double)rs->cnt_host->nodes;
         stats->tris_closest = (double)rs->cnt_host->tris;
@@ -1676,7 +2024,7 @@ dl_status render_batch(Ctx* c, const dl_render_params* prm, const dl_batch_item*
     const int stage_grid = std::max(1, c->num_cus) * 8;
     const int trace_grid = (int)(count ? c->trace_grid_count : c->trace_grid);
     std::vector<int> tags;
-    Timer tm{c, rs, &tags};
+    Timer tm{c, rs, &tags, {}};
     double closest = 0, shadow = 0;
     PassParams pp{};
     pp.P = P;
@@ -1749,6 +2097,12 @@ dl_status render_batch(Ctx* c, const dl_render_params* prm, const dl_batch_item*
             switch (tags[i]) {
                 case kTagClosest: stats->ms_closest += e; stats->launches_closest += 1; break;
                 case kTagShadow: stats->ms_shadow += e; stats->launches_shadow += 1; break;
+                case kTagBoth:
+                    stats->ms_closest += e * tm.share[i];
+                    stats->ms_shadow += e * (1.0 - tm.share[i]);
+                    stats->launches_closest += 1;
+                    stats->launches_shadow += 1;
+                    break;
                 case kTagShade: stats->ms_shade += e; break;
                 case kTagFilm: stats->ms_film += e; break;
                 default: stats->ms_other += e; break;
@@ -1756,8 +2110,8 @@ dl_status render_batch(Ctx* c, const dl_render_params* prm, const dl_batch_item*
         }
         DL_HIP_CHECK(c, hipMemcpy(rs->cnt_host, rs->b.cnt, sizeof(Counters), hipMemcpyDeviceToHost));
         stats->paths = P;
-        stats->closest_rays = closest;
-        stats->shadow_rays = shadow;
+        stats->closest_rays = closest + (double)rs->cnt_host->fin_closest;
+        stats->shadow_rays = shadow + (double)rs->cnt_host->fin_shadow;
         stats->invalid_samples = (double)rs->cnt_host->invalid;
         stats->nodes_closest = (double)rs->cnt_host->nodes;
         stats->tris_closest = (double)rs->cnt_host->tris;

@@ -169,9 +169,9 @@ struct TraceWork {
     uint32_t unit;
     uint32_t group;
 };
-__device__ __forceinline__ TraceWork trace_work(uint32_t* counters, uint32_t n) {
-    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
-    const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+// wave / waves: this wave's index among those that start with slots of their
+// own, and their number; a wave beyond them only claims.
+__device__ __forceinline__ TraceWork trace_work(uint32_t* counters, uint32_t n, uint32_t wave, uint32_t waves) {
     // (n is at most 2^31 and a grid has at most 2^13 waves)
     const uint32_t share = (n + waves - 1) / waves;
     // Few slots: a few lanes of every wave rather than all lanes of some, as
@@ -185,10 +185,170 @@ __device__ __forceinline__ TraceWork trace_work(uint32_t* counters, uint32_t n) 
     w.counter = counters + w.group * kWorkStride;
     w.n = n;
     w.base = min(n, per * waves);
-    w.first = min(wave * per, w.base);
-    w.count = min(per, w.base - w.first);
+    w.first = min(min(wave, waves) * per, w.base);
+    w.count = wave < waves ? min(per, w.base - w.first) : 0u;
     w.unit = share >= 256u ? 64u : share >= 128u ? 32u : share >= 64u ? 16u : 8u;
     return w;
+}
+
+// This wave's index in the grid and the grid's number of waves.
+__device__ __forceinline__ uint32_t grid_wave() {
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+}
+__device__ __forceinline__ uint32_t grid_waves() { return gridDim.x * (blockDim.x >> 6); }
+
+// One ray in flight: a lane's traversal state and its two kinds of step.
+struct RayState {
+    vec3 o, d, rcp;
+    float tmin, best_t, bu, bv;
+    uint32_t best;
+    int sp, cur;
+    // triangles of the last visited node's hit leaves: triangle j lies at
+    // j + lb[c], c the first slot whose running total of triangles exceeds j
+    // (totals of slots 0, 0-1 and 0-2 packed in lend, 10 bits each: a leaf
+    // holds at most kMaxLeafCount = 255), their number and the next one to
+    // test; `last`: no node left to visit once they are tested
+    int4 lb;
+    uint32_t lend;
+    int ltri, lj;
+    bool last;
+
+    __device__ __forceinline__ void clear() {
+        o = d = rcp = v3(0, 0, 0);
+        tmin = best_t = bu = bv = 0.f;
+        best = 0xffffffffu;
+        sp = cur = 0;
+        lb = make_int4(0, 0, 0, 0);
+        lend = 0;
+        ltri = lj = 0;
+        last = false;
+    }
+
+    // Starts the ray in o, d, tmin at node `root`.  False for a ray that holds
+    // a NaN: it makes every Moller-Trumbore comparison false (no hit), but
+    // would pass every slab test, so it is finished at once as a miss.
+    __device__ __forceinline__ bool start(float tmax, int root) {
+        rcp = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+        best_t = tmax;
+        best = 0xffffffffu;
+        bu = bv = 0.0f;
+        sp = 0;
+        cur = root;
+        ltri = lj = 0;
+        last = false;
+        return !(isnan(o.x) || isnan(o.y) || isnan(o.z) || isnan(d.x) || isnan(d.y) || isnan(d.z) || isnan(tmin) ||
+                 isnan(tmax));
+    }
+
+    // The next one or two triangles of the last visit's hit leaves, in slot
+    // order: both fetched before the first is tested, so a pair costs one
+    // dependent wait; the second is accepted against the best t the first
+    // left, as a sequential loop would.  any: stops at the first accepted
+    // triangle, and returns true for it.
+    __device__ __forceinline__ bool test_triangles(const BvhView& bvh, bool any) {
+        const int e0 = (int)(lend & 0x3ffu), e1 = (int)((lend >> 10) & 0x3ffu), e2 = (int)(lend >> 20);
+        const int j = lj;
+        const bool two = j + 1 < ltri;
+        const int j1 = two ? j + 1 : j;
+        int k0 = lb.w, k1 = lb.w;
+        k0 = j < e2 ? lb.z : k0;
+        k1 = j1 < e2 ? lb.z : k1;
+        k0 = j < e1 ? lb.y : k0;
+        k1 = j1 < e1 ? lb.y : k1;
+        k0 = (j < e0 ? lb.x : k0) + j;
+        k1 = (j1 < e0 ? lb.x : k1) + j1;
+        const float4* tp0 = bvh.tris + 3 * k0;
+        const float4* tp1 = bvh.tris + 3 * k1;
+        const float4 ta = tp0[0], tb = tp0[1], tc = tp0[2];
+        const float4 sa = tp1[0], sb = tp1[1], sc = tp1[2];
+        float u, v, t;
+        const bool h0 = mt_test(ta, tb, tc, o, d, u, v, t) && t >= tmin && t <= best_t;
+        lj++;
+        if (any && h0) return true;
+        if (!any && h0) accept(t, u, v, __float_as_uint(tc.y));
+        if (two) {
+            lj++;
+            if (mt_test(sa, sb, sc, o, d, u, v, t) && t >= tmin && t <= best_t) {
+                if (any) return true;
+                accept(t, u, v, __float_as_uint(sc.y));
+            }
+        }
+        return false;
+    }
+    __device__ __forceinline__ void accept(float t, float u, float v, uint32_t id) {
+        if (t < best_t || id < best) {
+            best_t = t;
+            best = id;
+            bu = u;
+            bv = v;
+        }
+    }
+
+    // Visits node cur: its hit leaves' triangles become the ones to test, the
+    // nearest hit internal child (or a stack pop) the next node.
+    __device__ __forceinline__ void visit_node(const BvhView& bvh, LaneStack& stk) {
+        const float4* np = bvh.nodes + 4 * (size_t)cur;
+        const float4 r0 = np[0];
+        const uint4 r1 = reinterpret_cast<const uint4*>(np)[1];
+        const uint4 r2 = reinterpret_cast<const uint4*>(np)[2];
+        const int4 ref = reinterpret_cast<const int4*>(np)[3];
+        // child boxes: origin + q * step (q * step exact, one rounding)
+        const uint32_t eb = __float_as_uint(r0.w);
+        const vec3 step = v3(__uint_as_float((eb & 0xffu) << 23), __uint_as_float(((eb >> 8) & 0xffu) << 23),
+                             __uint_as_float(((eb >> 16) & 0xffu) << 23));
+        const vec3 org = v3(r0.x, r0.y, r0.z);
+        const bool px = rcp.x >= 0.0f, py = rcp.y >= 0.0f, pz = rcp.z >= 0.0f;
+        const uint32_t nw[3] = {px ? r1.x : r1.y, py ? r1.z : r1.w, pz ? r2.x : r2.y};
+        const uint32_t fw[3] = {px ? r1.y : r1.x, py ? r1.w : r1.z, pz ? r2.y : r2.x};
+        float n0, n1, n2, n3;
+        const bool h0 = slab_q(nw, fw, 0, step, org, o, rcp, tmin, best_t, n0);
+        const bool h1 = slab_q(nw, fw, 8, step, org, o, rcp, tmin, best_t, n1);
+        const bool h2 = slab_q(nw, fw, 16, step, org, o, rcp, tmin, best_t, n2);
+        const bool h3 = slab_q(nw, fw, 24, step, org, o, rcp, tmin, best_t, n3);
+        // triangles of the hit leaf children, tested in the next steps (the
+        // closest hit is the minimum over (t, id), so their order does not
+        // change it)
+        const int c0n = (h0 && ref.x < 0) ? (int)(r2.z & 0xffu) : 0;
+        const int c1n = (h1 && ref.y < 0) ? (int)((r2.z >> 8) & 0xffu) : 0;
+        const int c2n = (h2 && ref.z < 0) ? (int)((r2.z >> 16) & 0xffu) : 0;
+        const int c3n = (h3 && ref.w < 0) ? (int)(r2.z >> 24) : 0;
+        const int e1 = c0n + c1n, e2 = e1 + c2n;
+        lend = (uint32_t)c0n | ((uint32_t)e1 << 10) | ((uint32_t)e2 << 20);
+        lb = make_int4(~ref.x, ~ref.y - c0n, ~ref.z - e1, ~ref.w - e2);
+        ltri = e2 + c3n;
+        lj = 0;
+        // hit internal children: keys = entry distances (+inf: not taken),
+        // sorted by a 5-exchange network; the nearest is visited next and the
+        // others are stacked farthest first
+        float k0 = (h0 && ref.x >= 0) ? n0 : INFINITY, k1 = (h1 && ref.y >= 0) ? n1 : INFINITY;
+        float k2 = (h2 && ref.z >= 0) ? n2 : INFINITY, k3 = (h3 && ref.w >= 0) ? n3 : INFINITY;
+        int c0 = ref.x, c1 = ref.y, c2 = ref.z, c3 = ref.w;
+        cswap(k0, c0, k1, c1);
+        cswap(k2, c2, k3, c3);
+        cswap(k0, c0, k2, c2);
+        cswap(k1, c1, k3, c3);
+        cswap(k1, c1, k2, c2);
+        if (k0 != INFINITY) {
+            stk.push3(sp, c3, k3 != INFINITY, c2, k2 != INFINITY, c1, k1 != INFINITY);
+            cur = c0;
+        } else if (sp == 0) {
+            last = true;
+        } else {
+            cur = stk.pop(sp);
+        }
+    }
+};
+
+// Which kind of step a wave takes next: the lanes whose next step is a
+// triangle test and those whose next step is a node visit would otherwise run
+// both branches every iteration under partial masks.  Triangle steps run when
+// enough lanes wait for one (a triangle step costs about kTriCost / kNodeCost
+// of a node visit); the other lanes hold their step, so every ray still makes
+// its own sequence of visits and tests.
+__device__ __forceinline__ bool wave_tests_triangles(bool active, bool tri_step) {
+    const uint32_t ntri = (uint32_t)__popcll(__ballot(active && tri_step));
+    const uint32_t nnode = (uint32_t)__popcll(__ballot(active && !tri_step));
+    return ntri != 0 && ntri * kNodeCost >= nnode * kTriCost;
 }
 
 // Persistent traversal with per-lane ray refill.  Every lane of a wave stays
@@ -242,19 +402,8 @@ __device__ __forceinline__ void traverse_persistent(const BvhView& bvh, const Tr
     if (more) claim_next();
     uint32_t ray = 0;
     bool active = false;
-    vec3 o = v3(0, 0, 0), d = v3(0, 0, 0), rcp = v3(0, 0, 0);
-    float tmin = 0.f, best_t = 0.f, bu = 0.f, bv = 0.f;
-    uint32_t best = 0xffffffffu;
-    int sp = 0, cur = 0;
-    // triangles of the last visited node's hit leaves: triangle j lies at
-    // j + lb[c], c the first slot whose running total of triangles exceeds j
-    // (totals of slots 0, 0-1 and 0-2 packed in lend, 10 bits each: a leaf
-    // holds at most kMaxLeafCount = 255), their number and the next one to
-    // test; `last`: no node left to visit once they are tested
-    int4 lb = make_int4(0, 0, 0, 0);
-    uint32_t lend = 0;
-    int ltri = 0, lj = 0;
-    bool last = false;
+    RayState r;
+    r.clear();
     bool pend = false;  // (kResolve) the lane's finished ray is unoccluded and not yet resolved
     TraceCounters cnt;
     for (;;) {
@@ -288,29 +437,16 @@ __device__ __forceinline__ void traverse_persistent(const BvhView& bvh, const Tr
                 if (at < len) {
                     ray = e;
                     float tmax;
-                    io.load(ray, o, d, tmin, tmax);
-                    rcp = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-                    best_t = tmax;
-                    best = 0xffffffffu;
-                    bu = bv = 0.0f;
-                    sp = 0;
-                    cur = io.root(ray);
-                    ltri = lj = 0;
-                    last = false;
+                    io.load(ray, r.o, r.d, r.tmin, tmax);
                     cnt = TraceCounters();
-                    // A NaN anywhere in the ray makes every Moller-Trumbore
-                    // comparison false (no hit), but would pass every slab
-                    // test: finish it at once as a miss.
-                    if (isnan(o.x) || isnan(o.y) || isnan(o.z) || isnan(d.x) || isnan(d.y) || isnan(d.z) || isnan(tmin) ||
-                        isnan(tmax)) {
+                    active = r.start(tmax, io.root(ray));
+                    if (!active) {
                         if (ANY && IO::kResolve)
                             pend = true;
                         else if (ANY)
                             io.store_occ(ray, false, 0, 0);
                         else
-                            io.store_hit(ray, best, best_t, 0.0f, 0.0f, 0, 0);
-                    } else {
-                        active = true;
+                            io.store_hit(ray, r.best, r.best_t, 0.0f, 0.0f, 0, 0);
                     }
                 }
                 if (resolve) io.resolve_store(fin, ra, rb);
@@ -319,136 +455,27 @@ __device__ __forceinline__ void traverse_persistent(const BvhView& bvh, const Tr
         } else if (idle == 64u && pos == len && !more) {
             break;
         }
-        // One kind of step per wave and iteration: the lanes whose next
-        // step is a triangle test and those whose next step is a node visit
-        // would otherwise run both branches every iteration under partial
-        // masks.  Triangle steps run when enough lanes wait for one (a
-        // triangle step costs about kTriCost / kNodeCost of a node visit);
-        // the other lanes hold their step, so every ray still makes its own
-        // sequence of visits and tests.
-        const bool tri_step = lj < ltri;
-        const uint32_t ntri = (uint32_t)__popcll(__ballot(active && tri_step));
-        const uint32_t nnode = (uint32_t)__popcll(__ballot(active && !tri_step));
-        const bool tri_mode = ntri != 0 && ntri * kNodeCost >= nnode * kTriCost;
+        const bool tri_step = r.lj < r.ltri;
+        const bool tri_mode = wave_tests_triangles(active, tri_step);
         if (!active || tri_step != tri_mode) continue;
 
-        bool done = false, hit_any = false;
+        bool hit_any = false;
         if (tri_mode) {
-            // the next one or two triangles of the last visit's hit leaves, in
-            // slot order: both fetched before the first is tested, so a pair
-            // costs one dependent wait; the second is accepted against the
-            // best t the first left, as a sequential loop would
-            const int e0 = (int)(lend & 0x3ffu), e1 = (int)((lend >> 10) & 0x3ffu), e2 = (int)(lend >> 20);
-            const int j = lj;
-            const bool two = j + 1 < ltri;
-            const int j1 = two ? j + 1 : j;
-            int k0 = lb.w, k1 = lb.w;
-            k0 = j < e2 ? lb.z : k0;
-            k1 = j1 < e2 ? lb.z : k1;
-            k0 = j < e1 ? lb.y : k0;
-            k1 = j1 < e1 ? lb.y : k1;
-            k0 = (j < e0 ? lb.x : k0) + j;
-            k1 = (j1 < e0 ? lb.x : k1) + j1;
-            const float4* tp0 = bvh.tris + 3 * k0;
-            const float4* tp1 = bvh.tris + 3 * k1;
-            const float4 ta = tp0[0], tb = tp0[1], tc = tp0[2];
-            const float4 sa = tp1[0], sb = tp1[1], sc = tp1[2];
-            float u, v, t;
-            const bool h0 = mt_test(ta, tb, tc, o, d, u, v, t) && t >= tmin && t <= best_t;
-            if (ANY) {
-                hit_any = h0;
-                if (two && !h0) {
-                    hit_any = mt_test(sa, sb, sc, o, d, u, v, t) && t >= tmin && t <= best_t;
-                    lj++;
-                    if (COUNT) cnt.tris++;
-                }
-            } else {
-                if (h0) {
-                    const uint32_t id = __float_as_uint(tc.y);
-                    if (t < best_t || id < best) {
-                        best_t = t;
-                        best = id;
-                        bu = u;
-                        bv = v;
-                    }
-                }
-                if (two) {
-                    lj++;
-                    if (COUNT) cnt.tris++;
-                    if (mt_test(sa, sb, sc, o, d, u, v, t) && t >= tmin && t <= best_t) {
-                        const uint32_t id = __float_as_uint(sc.y);
-                        if (t < best_t || id < best) {
-                            best_t = t;
-                            best = id;
-                            bu = u;
-                            bv = v;
-                        }
-                    }
-                }
-            }
-            lj++;
-            if (COUNT) cnt.tris++;
-            done = hit_any || (last && lj == ltri);
+            const int j = r.lj;
+            hit_any = r.test_triangles(bvh, ANY);
+            if (COUNT) cnt.tris += (uint32_t)(r.lj - j);
         } else {
-            const float4* np = bvh.nodes + 4 * (size_t)cur;
-            const float4 r0 = np[0];
-            const uint4 r1 = reinterpret_cast<const uint4*>(np)[1];
-            const uint4 r2 = reinterpret_cast<const uint4*>(np)[2];
-            const int4 ref = reinterpret_cast<const int4*>(np)[3];
             if (COUNT) cnt.nodes++;
-            // child boxes: origin + q * step (q * step exact, one rounding)
-            const uint32_t eb = __float_as_uint(r0.w);
-            const vec3 step = v3(__uint_as_float((eb & 0xffu) << 23), __uint_as_float(((eb >> 8) & 0xffu) << 23),
-                                 __uint_as_float(((eb >> 16) & 0xffu) << 23));
-            const vec3 org = v3(r0.x, r0.y, r0.z);
-            const bool px = rcp.x >= 0.0f, py = rcp.y >= 0.0f, pz = rcp.z >= 0.0f;
-            const uint32_t nw[3] = {px ? r1.x : r1.y, py ? r1.z : r1.w, pz ? r2.x : r2.y};
-            const uint32_t fw[3] = {px ? r1.y : r1.x, py ? r1.w : r1.z, pz ? r2.y : r2.x};
-            float n0, n1, n2, n3;
-            const bool h0 = slab_q(nw, fw, 0, step, org, o, rcp, tmin, best_t, n0);
-            const bool h1 = slab_q(nw, fw, 8, step, org, o, rcp, tmin, best_t, n1);
-            const bool h2 = slab_q(nw, fw, 16, step, org, o, rcp, tmin, best_t, n2);
-            const bool h3 = slab_q(nw, fw, 24, step, org, o, rcp, tmin, best_t, n3);
-            // triangles of the hit leaf children, tested in the next
-            // iterations (the closest hit is the minimum over (t, id), so
-            // their order does not change it)
-            const int c0n = (h0 && ref.x < 0) ? (int)(r2.z & 0xffu) : 0;
-            const int c1n = (h1 && ref.y < 0) ? (int)((r2.z >> 8) & 0xffu) : 0;
-            const int c2n = (h2 && ref.z < 0) ? (int)((r2.z >> 16) & 0xffu) : 0;
-            const int c3n = (h3 && ref.w < 0) ? (int)(r2.z >> 24) : 0;
-            const int e1 = c0n + c1n, e2 = e1 + c2n;
-            lend = (uint32_t)c0n | ((uint32_t)e1 << 10) | ((uint32_t)e2 << 20);
-            lb = make_int4(~ref.x, ~ref.y - c0n, ~ref.z - e1, ~ref.w - e2);
-            ltri = e2 + c3n;
-            lj = 0;
-            // hit internal children: keys = entry distances (+inf: not
-            // taken), sorted by a 5-exchange network; the nearest is visited
-            // next and the others are stacked farthest first
-            float k0 = (h0 && ref.x >= 0) ? n0 : INFINITY, k1 = (h1 && ref.y >= 0) ? n1 : INFINITY;
-            float k2 = (h2 && ref.z >= 0) ? n2 : INFINITY, k3 = (h3 && ref.w >= 0) ? n3 : INFINITY;
-            int c0 = ref.x, c1 = ref.y, c2 = ref.z, c3 = ref.w;
-            cswap(k0, c0, k1, c1);
-            cswap(k2, c2, k3, c3);
-            cswap(k0, c0, k2, c2);
-            cswap(k1, c1, k3, c3);
-            cswap(k1, c1, k2, c2);
-            if (k0 != INFINITY) {
-                stk.push3(sp, c3, k3 != INFINITY, c2, k2 != INFINITY, c1, k1 != INFINITY);
-                cur = c0;
-            } else if (sp == 0) {
-                last = true;
-            } else {
-                cur = stk.pop(sp);
-            }
-            done = last && ltri == 0;
+            r.visit_node(bvh, stk);
         }
+        const bool done = hit_any || (r.last && r.lj == r.ltri);
         if (done) {
             if (ANY && IO::kResolve)
                 pend = !hit_any;
             else if (ANY)
                 io.store_occ(ray, hit_any, cnt.nodes, cnt.tris);
             else
-                io.store_hit(ray, best, best_t, bu, bv, cnt.nodes, cnt.tris);  // a miss keeps t = tmax
+                io.store_hit(ray, r.best, r.best_t, r.bu, r.bv, cnt.nodes, cnt.tris);  // a miss keeps t = tmax
             if (COUNT) {
                 total.nodes += cnt.nodes;
                 total.tris += cnt.tris;

@@ -61,7 +61,7 @@ __global__ __launch_bounds__(kTraceBlock, COUNT ? 4 : 8) void k_trace_closest(Bv
     const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x, G = gridDim.x * kTraceBlock;
     LaneStack stk{lds, (int)threadIdx.x, kTraceBlock, ovf + g, G};
     TraceCounters tot;
-    traverse_persistent<false, COUNT>(bvh, trace_work(work, n), stk, io, tot);
+    traverse_persistent<false, COUNT>(bvh, trace_work(work, n, grid_wave(), grid_waves()), stk, io, tot);
 }
 
 template <bool COUNT>
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(kTraceBlock, COUNT ? 4 : 8) void k_trace_shadow(Bvh
     const uint32_t g = blockIdx.x * kTraceBlock + threadIdx.x, G = gridDim.x * kTraceBlock;
     LaneStack stk{lds, (int)threadIdx.x, kTraceBlock, ovf + g, G};
     TraceCounters tot;
-    traverse_persistent<true, COUNT>(bvh, trace_work(work, n), stk, io, tot);
+    traverse_persistent<true, COUNT>(bvh, trace_work(work, n, grid_wave(), grid_waves()), stk, io, tot);
 }
 
 // Resident blocks per CU of the batch traversal kernels (the fewer of the

@@ -215,7 +215,9 @@ typedef struct dl_render_stats {
     double shadow_rays;        /* shadow queries issued */
     double invalid_samples;    /* NaN / Inf / negative samples dropped (block.cpp:82-88) */
     double ms_total;           /* wall time of the render loop (hipEvents) */
-    double ms_closest;         /* summed kernel time per stage */
+    double ms_closest;         /* summed kernel time per stage (a launch that traces both queries of a
+                                  bounce of few rays: shared out by rays; the launch that carries a
+                                  pass's last paths to their end: closest) */
     double ms_shadow;
     double ms_shade;
     double ms_film;

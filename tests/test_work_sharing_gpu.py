@@ -1,0 +1,70 @@
+"""How work is shared out over waves and launches must not show in results:
+ray batches around the sizes at which a traversal's waves start to claim
+chunks, and renders around the sizes at which paths are carried to their end
+in one launch or bounces trace both queries in one launch."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import drawlab_amd
+from drawlab_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _rays(n, seed):
+    r = np.random.default_rng(seed)
+    rays = np.empty((8, n), np.float32)
+    rays[0:3] = r.uniform(-2.5, 2.5, (3, n))
+    d = r.standard_normal((3, n))
+    rays[3:6] = d / np.linalg.norm(d, axis=0)
+    rays[6], rays[7] = 1e-4, np.where(r.random(n) < 0.5, np.inf, 3.0)
+    rays[3, ::97] = np.nan  # finished at once, also when a whole wave holds nothing else
+    rays[3, 640:768] = np.nan
+    return rays
+
+
+@pytest.mark.parametrize("n", [1, 63, 8191, 131071, 131073, 1048577, 2200003])
+def test_ray_batches_of_any_size_give_the_hits_of_small_ones(backend, n):
+    """Results of a batch equal those of its rays traced 4,000 at a time (a
+    few rays per wave, nothing claimed)."""
+    backend.upload_scene(scenes.displaced_sphere(width=32, height=18, grid=64, glass_level=2, env_size=(32, 16)))
+    backend.build_accel(drawlab_amd.BUILD_GPU)
+    rays = _rays(n, n)
+    hits, occ = backend.trace_closest(rays), backend.trace_shadow(rays)
+    pick = np.unique(np.concatenate([np.arange(min(n, 4000)), np.arange(max(0, n - 4000), n),
+                                     np.random.default_rng(1).integers(0, n, 4000)]))
+    for s in range(0, len(pick), 4000):
+        sub = np.ascontiguousarray(rays[:, pick[s:s + 4000]])
+        for a, b in zip(hits, backend.trace_closest(sub)):
+            assert np.array_equal(a[pick[s:s + 4000]].view(np.uint32), b.view(np.uint32))
+        assert np.array_equal(occ[pick[s:s + 4000]], backend.trace_shadow(sub))
+
+
+SCENES = {
+    "zoo": lambda: scenes.material_zoo(64, 48),
+    "textured": lambda: scenes.textured_box(64, 64),
+    "sphere": lambda: scenes.displaced_sphere(width=64, height=36, grid=64, glass_level=2, env_size=(64, 32)),
+    "plates": lambda: scenes.mis_plates(64, 36),
+}
+
+
+@pytest.mark.parametrize("name", sorted(SCENES))
+@pytest.mark.parametrize("size", [(1, 1, 3), (31, 1, 2), (43, 33, 5), (362, 362, 2), (363, 361, 2)],
+                         ids=lambda s: "%dx%dx%d" % s)
+def test_paths_finished_in_one_launch_equal_the_bounce_by_bounce_ones(backend, name, size):
+    """A counting render goes bounce by bounce to the end; a plain one hands
+    the paths over when few are left, or from the camera on when its passes
+    are small (131,072 paths): same images and same ray counts."""
+    W, H, spp = size
+    d = SCENES[name]()
+    d = dataclasses.replace(d, camera=dataclasses.replace(d.camera, width=W, height=H))
+    backend.upload_scene(d)
+    backend.build_accel(drawlab_amd.BUILD_GPU)
+    for depth, rr in ((d.max_depth, d.rr_depth), (1, 4), (2, 0), (-1, 1)):
+        ref, rs = backend.render(spp=spp, seed=3, max_depth=depth, rr_depth=rr, count_traversal=True)
+        for per_pass in (0, 1):
+            img, st = backend.render(spp=spp, seed=3, max_depth=depth, rr_depth=rr, spp_per_pass=per_pass)
+            assert np.array_equal(img.view(np.uint32), ref.view(np.uint32)), (depth, rr, per_pass)
+            assert st["closest_rays"] == rs["closest_rays"] and st["shadow_rays"] == rs["shadow_rays"]

@@ -303,7 +303,7 @@ struct Net;
 void free_guide(Ctx* c);
 dl_status guide_init(Ctx* c, uint64_t seed, float lr, const float* params);
 // bf16 weights / biases of the current network (guide must be initialised)
-void guide_net_ptrs(Ctx* c, const uint16_t** w, const uint16_t** wt, const float** bias);
+Net guide_net(Ctx* c);
 // one training step on R records; rad: final path radiance (float4 per path)
 dl_status guide_train_records(Ctx* c, const float* records, uint32_t R, const float4* rad, int steps);
 int guide_step_count(Ctx* c);  // Adam steps taken since guide_init

@@ -204,10 +204,26 @@ __device__ __forceinline__ bf16x8 pack8(const float* v) {
     return r;
 }
 
+// The bfloat16 copies of a layer's weights lie in the order in which the
+// matrix instructions take them: 32x16 tiles (row tiles outer, K / 16 of them
+// per row tile), in each the 8 values of lane 0, of lane 1, ... -- lane l holds
+// row l % 32, columns (l / 32) * 8 + 0..7 -- so that a wave reads a tile as
+// 1024 consecutive bytes.  (Read from [row][column] order, consecutive lanes
+// lie a row apart and the texture path takes 56 cycles per load, which bound
+// the network kernels.)
+__host__ __device__ constexpr int operand_index(int row, int col, int K) {
+    return (((row / 32) * (K / 16) + col / 16) * 64 + row % 32 + 32 * ((col % 16) / 8)) * 8 + col % 8;
+}
+// The same in 16x32 tiles, for the 16x16x32 products of training: lane l holds
+// row l % 16, columns (l / 16) * 8 + 0..7.
+__host__ __device__ constexpr int operand16_index(int row, int col, int K) {
+    return (((row / 16) * (K / 32) + col / 32) * 64 + row % 16 + 16 * ((col % 32) / 8)) * 8 + col % 8;
+}
 struct Net {
-    const uint16_t* w;   // W[l]: [64][in(l)] bf16 (layer 4 rows 48..63 zero), slot kGWSlot
-    const uint16_t* wt;  // W^T[l]: [in(l)][64] bf16
-    const float* bias;   // [5][64] (layer 4 entries 48..63 zero)
+    const uint16_t* w;     // W[l] (64 x in(l), rows 48..63 of layer 4 zero), slot kGWSlot, in 32x16 tiles
+    const uint16_t* w16;   // the same in 16x32 tiles
+    const uint16_t* wt16;  // W^T[l] (in(l) x 64) in 16x32 tiles
+    const float* bias;     // [5][64] (layer 4 entries 48..63 zero)
 };
 
 // One layer for the wave's 64 LDS rows (stride kGRowStride): out = act W^T
@@ -223,12 +239,12 @@ __device__ __forceinline__ void layer(const Net& net, int l, uint16_t* s, Emit e
     for (int rb = 0; rb < 2; rb++) {
         f32x16 acc0 = {0}, acc1 = {0};
         const uint16_t* arow = s + (rb * 32 + (lane & 31)) * kGRowStride + (lane >> 5) * 8;
-        const uint16_t* b0 = W + (lane & 31) * K + (lane >> 5) * 8;
-        const uint16_t* b1 = W + (32 + (lane & 31)) * K + (lane >> 5) * 8;
+        const uint16_t* b0 = W + lane * 8;
+        const uint16_t* b1 = b0 + (K / 16) * 512;
         for (int kt = 0; kt < K / 16; kt++) {
             const bf16x8 a = *reinterpret_cast<const bf16x8*>(arow + kt * 16);
-            acc0 = mfma(a, *reinterpret_cast<const bf16x8*>(b0 + kt * 16), acc0);
-            acc1 = mfma(a, *reinterpret_cast<const bf16x8*>(b1 + kt * 16), acc1);
+            acc0 = mfma(a, *reinterpret_cast<const bf16x8*>(b0 + kt * 512), acc0);
+            acc1 = mfma(a, *reinterpret_cast<const bf16x8*>(b1 + kt * 512), acc1);
         }
         const int c0 = lane & 31, c1 = 32 + (lane & 31);
         const float bb0 = bias[c0], bb1 = bias[c1];
@@ -251,26 +267,12 @@ __device__ __forceinline__ void layer(const Net& net, int l, uint16_t* s, Emit e
     __builtin_amdgcn_wave_barrier();
 }
 
-// Forward pass of rows [row0, row0 + 64) whose bfloat16 inputs are already
-// in the wave's LDS rows.  keep: copy each layer's input rows to act[l].
+// Forward pass of the wave's 64 rows, whose bfloat16 inputs are already in
+// its LDS rows.
 template <typename Emit>
-__device__ __forceinline__ void forward_rows(const Net& net, uint16_t* s, uint32_t row0, uint32_t n, bool keep,
-                                             uint16_t* const* act, Emit emit) {
-    const int lane = threadIdx.x & 63;
+__device__ __forceinline__ void forward_rows(const Net& net, uint16_t* s, Emit emit) {
     __builtin_amdgcn_wave_barrier();  // input rows were written by their own lanes
-    for (int l = 0; l < 5; l++) {
-        if (keep) {
-            const int K = glayer_in(l);
-            const uint32_t row = row0 + lane;
-            if (row < n) {
-                const uint4* src = reinterpret_cast<const uint4*>(s + lane * kGRowStride);
-                uint4* dst = reinterpret_cast<uint4*>(act[l] + (size_t)row * K);
-                for (int q = 0; q < K / 8; q++) dst[q] = src[q];
-            }
-        }
-        layer(net, l, s, emit);
-    }
+    for (int l = 0; l < 5; l++) layer(net, l, s, emit);
 }
-
 
 }  // namespace dl

@@ -10,12 +10,13 @@
 //   forward     a wave takes 64 rows (two 32-row blocks); activations live
 //               in the wave's LDS rows (bfloat16, in place layer by layer);
 //               weights are read from global memory (43 KB, L2-resident) as
-//               B operands from W[out][in]
-//   backward    dW = g^T act (tiles of dW per wave, batch chunks reduced by
-//               float32 atomics), dAct = g W (B operands from W^T), ReLU
-//               masks from the stored bfloat16 activations
-//   Adam        float32 master weights; the bfloat16 copies (W and W^T) are
-//               refreshed in the same kernel
+//               B operands, 1 KB in a row per tile
+//   training    one kernel per step for forward, loss and backward (16x16x32
+//               and 32x32x16 tiles): a block keeps its rows' activations in LDS
+//               and its share of dW in registers; per-block partial gradients are then summed in a
+//               fixed order, with Adam in the same kernel (float32 master
+//               weights; the bfloat16 copies of W and W^T, laid out in the
+//               order in which the operands are read, are refreshed there)
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -29,15 +30,12 @@ namespace dl {
 
 namespace {
 
-// Network evaluation / training forward on float32 inputs x (n x 96).
+// Network evaluation on float32 inputs x (n x 96).
 __global__ __launch_bounds__(kGWaves * 64) void k_mlp_forward(Net net, const float* __restrict__ x, uint32_t n,
-                                                             float* __restrict__ out, int keep, uint16_t* act0,
-                                                             uint16_t* act1, uint16_t* act2, uint16_t* act3,
-                                                             uint16_t* act4) {
+                                                             float* __restrict__ out) {
     __shared__ uint16_t s_act[kGWaves][kGRowsPerWave * kGRowStride];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     uint16_t* s = s_act[wave];
-    uint16_t* const act[5] = {act0, act1, act2, act3, act4};
     for (uint32_t tile = blockIdx.x * kGWaves + wave; (size_t)tile * kGRowsPerWave < n; tile += gridDim.x * kGWaves) {
         const uint32_t row0 = tile * kGRowsPerWave;
         const uint32_t row = row0 + lane;
@@ -46,7 +44,7 @@ __global__ __launch_bounds__(kGWaves * 64) void k_mlp_forward(Net net, const flo
             for (int j = 0; j < 8; j++) f[j] = row < n ? x[(size_t)row * kGIn + q * 8 + j] : 0.0f;
             *reinterpret_cast<bf16x8*>(s + lane * kGRowStride + q * 8) = pack8(f);
         }
-        forward_rows(net, s, row0, n, keep != 0, act, [&](int r, int c, float v) {
+        forward_rows(net, s, [&](int r, int c, float v) {
             if (row0 + r < n) out[(size_t)(row0 + r) * kGOut + c] = v;
         });
     }
@@ -62,200 +60,459 @@ __global__ void k_mlp_decode(const float* __restrict__ out, uint32_t n, float* _
     }
 }
 
-// Sum of a 256-thread block's values added to *dst with one atomic.
-__device__ __forceinline__ void block_sum_add(float v, float* dst) {
+// Sum of a 256-thread block's values, in every thread of the first wave.
+__device__ __forceinline__ float block_sum(float v) {
     __shared__ float s_part[4];
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
     if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = v;
     __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(dst, s_part[0] + s_part[1] + s_part[2] + s_part[3]);
+    return (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
 }
 
-__global__ __launch_bounds__(256) void k_sum(const float* __restrict__ c, uint32_t n, float* __restrict__ total) {
+// Partial sums of the training weights, one per block (kSumBlocks blocks),
+// which every training block adds in the same order.
+__global__ __launch_bounds__(256) void k_sum(const float* __restrict__ c, uint32_t n, float* __restrict__ part) {
     float acc = 0.0f;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) acc += c[i];
-    block_sum_add(acc, total);
+    acc = block_sum(acc);
+    if (threadIdx.x == 0) part[blockIdx.x] = acc;
 }
 
-// dLoss/dout for loss = sum(-c log q(d)) / sum(c); loss accumulated in *loss.
-__global__ __launch_bounds__(256) void k_loss_grad(const float* __restrict__ out, const float* __restrict__ dirs,
-                            const float* __restrict__ c, uint32_t n, const float* __restrict__ total,
-                            float* __restrict__ g, float* __restrict__ loss) {
-    const float invC = 1.0f / fmaxf(*total, 1e-30f);
-    float lacc = 0.0f;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        float o[kGOut];
-        for (int j = 0; j < kGOut; j++) o[j] = out[(size_t)i * kGOut + j];
-        float mix[kGMix];
-        guide_decode(o, mix);
-        const vec3 d = v3(dirs[3 * i], dirs[3 * i + 1], dirs[3 * i + 2]);
-        float f[kGLobes], dt[kGLobes], q = 0.0f;
-        for (int j = 0; j < kGLobes; j++) {
-            const vec3 mu = v3(mix[5 * j + 2], mix[5 * j + 3], mix[5 * j + 4]);
-            dt[j] = dot(mu, d);
-            f[j] = vmf_pdf(mix[5 * j + 1], mu, d);
-            q += mix[5 * j] * f[j];
-        }
-        const float ci = c[i];
-        const float qs = fmaxf(q, 1e-30f);
-        lacc += -ci * logf(qs) * invC;
-        const float gq = -ci / qs * invC;
-        float* gi = g + (size_t)i * kGOut;
-        for (int j = 0; j < kGLobes; j++) {
-            const float w = mix[5 * j], k = mix[5 * j + 1];
-            const float wf = w * f[j];
-            gi[5 * j] = gq * (wf - w * q);
-            const float sg = 1.0f / (1.0f + expf(-o[5 * j + 1]));
-            const float em = -expm1f(-2.0f * k);
-            const float dlogf = 1.0f / k - 2.0f * expf(-2.0f * k) / em + (dt[j] - 1.0f);
-            gi[5 * j + 1] = gq * wf * dlogf * k * (kGKappaHi - kGKappaLo) * sg * (1.0f - sg);
-            const float mx = o[5 * j + 2], my = o[5 * j + 3], mz = o[5 * j + 4];
-            const float nm = fmaxf(sqrtf(mx * mx + my * my + mz * mz), 1e-6f);
-            const float s = gq * wf * k / nm;
-            gi[5 * j + 2] = s * (d.x - dt[j] * mix[5 * j + 2]);
-            gi[5 * j + 3] = s * (d.y - dt[j] * mix[5 * j + 3]);
-            gi[5 * j + 4] = s * (d.z - dt[j] * mix[5 * j + 4]);
-        }
-        for (int j = kGMix; j < kGOut; j++) gi[j] = 0.0f;
-    }
-    block_sum_add(lacc, loss);
-}
+// ---- one training step's forward, loss and backward -----------------------
+// loss = sum(-c log q(d)) / sum(c) and its gradient.  Each of a block's four
+// waves takes 16 rows of a 64-row tile through the network and back:
+//
+//   forward   D[out][row] = W act^T + b per layer (16x16x32): a lane's
+//             accumulators are one row's outputs in runs of four, so the next
+//             layer's operand rows are written 8 bytes at a time; every
+//             layer's inputs are also kept transposed ([column][row]) for dW
+//   loss      four lanes per row, two lobes each; dLoss/dout in registers
+//   backward  per layer, from the output: dW[out][in] += g^T act over the
+//             tile's 64 rows (22 tiles of 32x32 shared out over the waves,
+//             accumulated in registers over the block's whole run), and
+//             D[in][row] = W^T g^T with the ReLU mask the forward left in
+//             registers, in the same layout again
+//
+// The bias gradients are summed from the unrounded float32 gradients; what the
+// matrix products read is bfloat16, as in the forward.  Two blocks per CU (73
+// KB of LDS and up to 256 registers each).  What bounds it is latency: each
+// wave's chain of LDS and matrix steps, and the weights, read per tile from L1/L2: 144 us for 2^18 rows,
+// 0.23 PFLOP/s (249 us with the weights' pointers laundered into flat loads,
+// which also wait for the LDS, and a wait at each change of LDS type).  A step
+// of 2^18 rows took 814 us as fifteen launches (forward, loss, and dW, its
+// reduction and dAct per layer, 700 bytes of activations and gradients per row
+// through memory) and takes 208 us as three.
+constexpr int kTrainWaves = 4, kTrainRows = 16 * kTrainWaves;
+constexpr int kTrainStride = kTrainRows + 8;         // bf16 per transposed column
+constexpr int kTrainCols = kGIn + 4 * kGHid;         // the inputs of the five layers
+constexpr int kTrainOutStride = kGOut + 1;           // float32 outputs of a row
+constexpr int kSumBlocks = (int)dl_sizes::kGuideSumBlocks;
+static_assert(kSumBlocks == 64, "one partial sum per lane");
+static_assert(kTrainOutStride * 4 <= kGRowStride * 2, "outputs overlay the operand rows");
+constexpr int train_col(int l) { return l == 0 ? 0 : kGIn + (l - 1) * kGHid; }
 
-// Weight and bias gradients of one layer without atomics: block (tile o,
-// tile i, chunk of kChunk rows) of kDwWaves waves, each wave accumulating
-// g^T act over its share of the chunk on the matrix cores; the waves' tiles
-// are summed in LDS and the block writes its chunk's partial dW tile (and,
-// for i-tile 0, the partial bias sums of its outputs) to part[chunk]; then
-// k_dw_reduce adds the chunks to the gradient in a fixed order, so a
-// training step is deterministic.
-constexpr int kChunk = 1024, kDwWaves = 4;
-__global__ __launch_bounds__(kDwWaves * 64) void k_dw(const float* __restrict__ g, int gw,
-                                                      const uint16_t* __restrict__ act, int K, uint32_t n,
-                                                      float* __restrict__ part) {
-    __shared__ float s_acc[kDwWaves][16][64];
-    __shared__ float s_b[kDwWaves][64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int ot = blockIdx.x, it = blockIdx.y;
-    const uint32_t chunk = blockIdx.z;
-    const uint32_t r0 = chunk * kChunk + wave * (kChunk / kDwWaves);
-    const uint32_t r1 = min(r0 + kChunk / kDwWaves, n);
-    const int o = ot * 32 + (lane & 31), i = it * 32 + (lane & 31);
-    f32x16 acc = {0};
-    float bsum = 0.0f;
-    for (uint32_t kb = r0; kb < r1; kb += 16) {
-        float av[8];
-        bf16x8 b;
-        for (int j = 0; j < 8; j++) {
-            const uint32_t srow = kb + (lane >> 5) * 8 + j;
-            const bool ok = srow < r1;
-            av[j] = ok && o < gw ? g[(size_t)srow * gw + o] : 0.0f;
-            b[j] = ok ? (short)act[(size_t)srow * K + i] : (short)0;
-            bsum += av[j];
-        }
-        acc = mfma(pack8(av), b, acc);
-    }
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // a caller's rows
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
+    // lane l holds A[l%16][(l/16)*8 + 0..7] and B[(l/16)*8 + 0..7][l%16];
+    // register r of the result is D[4*(l/16) + r][l%16]
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
+                                                   0, 0, 0);
+}
+// Two float32 to bfloat16, rounded to nearest even, a in the low half.
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+    const f32x2_t v = {a, b};
+    const bf16x2_t r = __builtin_convertvector(v, bf16x2_t);
+    return __builtin_bit_cast(uint32_t, r);
+}
+// Orders a wave's own LDS accesses, which are of several types.
+__device__ __forceinline__ void lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// Sums over the 16 rows of a wave (lanes of equal quad) of each of a lane's 16
+// values: lane rl returns the sum of value rl (v[rl / 4][rl % 4]).  Four
+// exchange steps, each halving the values: lanes l and l ^ 8, l ^ 7, l ^ 2,
+// l ^ 1.  (Kept per lane until the end, the sums of the hidden layers' biases
+// took 64 registers, and the accumulators spilled.)
+template <int CTRL, int CNT>
+__device__ __forceinline__ void row_sum_step(float (&a)[16], bool up) {
 #pragma unroll
-    for (int r = 0; r < 16; r++) s_acc[wave][r][lane] = acc[r];
-    s_b[wave][lane] = bsum;
-    __syncthreads();
-    if (wave != 0) return;
-    const size_t stride = (size_t)gw * K + gw;
-    float* dst = part + (size_t)chunk * stride;
+    for (int i = 0; i < CNT; i++) {
+        const float keep = up ? a[i + CNT] : a[i], send = up ? a[i] : a[i + CNT];
+        a[i] = keep + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(send), CTRL, 0xf, 0xf, true));
+    }
+}
+__device__ __forceinline__ float row_sums(const float (&v)[4][4], int rl) {
+    float a[16];
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        float v = 0.0f;
-        for (int w = 0; w < kDwWaves; w++) v += s_acc[w][r][lane];
-        const int orow = ot * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (orow < gw) dst[(size_t)orow * K + i] = v;
-    }
-    if (it == 0 && lane < 32 && o < gw) {
-        float v = 0.0f;
-        for (int w = 0; w < kDwWaves; w++) v += s_b[w][lane] + s_b[w][lane + 32];
-        dst[(size_t)gw * K + o] = v;
-    }
-}
-
-// grad[e] += sum over chunks of part[chunk][e], e over the layer's weights
-// then biases (their order in the parameter vector).  Block: 64 elements x 4
-// groups of chunks (group q sums chunks q, q + 4, ...); the groups are added
-// in a fixed order.
-__global__ __launch_bounds__(256) void k_dw_reduce(const float* __restrict__ part, uint32_t chunks, uint32_t cnt,
-                                                   float* __restrict__ grad) {
-    __shared__ float s_sum[4][64];
-    const uint32_t e = blockIdx.x * 64 + (threadIdx.x & 63);
-    const uint32_t q = threadIdx.x >> 6;
-    float v = 0.0f;
-    if (e < cnt)
-        for (uint32_t c = q; c < chunks; c += 4) v += part[(size_t)c * cnt + e];
-    s_sum[q][threadIdx.x & 63] = v;
-    __syncthreads();
-    if (q == 0 && e < cnt) grad[e] += (s_sum[0][threadIdx.x] + s_sum[1][threadIdx.x]) + (s_sum[2][threadIdx.x] + s_sum[3][threadIdx.x]);
-}
-
-// g_prev = (g W) * (act > 0): rows of 64 per wave; K = gw (64 or 48), out
-// width 64 (layer input).
-__global__ __launch_bounds__(kGWaves * 64) void k_dact(Net net, int l, const float* __restrict__ g, int gw,
-                                                      const uint16_t* __restrict__ act, uint32_t n,
-                                                      float* __restrict__ gprev) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const uint16_t* WT = net.wt + l * kGWSlot;  // [in = 64][64]
-    for (uint32_t tile = blockIdx.x * kGWaves + wave; (size_t)tile * kGRowsPerWave < n; tile += gridDim.x * kGWaves) {
-        const uint32_t row0 = tile * kGRowsPerWave;
-        for (int rb = 0; rb < 2; rb++) {
-            f32x16 acc0 = {0}, acc1 = {0};
-            const uint32_t arow = row0 + rb * 32 + (lane & 31);
-            for (int kt = 0; kt < gw / 16; kt++) {
-                float av[8];
-                for (int j = 0; j < 8; j++)
-                    av[j] = arow < n ? g[(size_t)arow * gw + kt * 16 + (lane >> 5) * 8 + j] : 0.0f;
-                const bf16x8 a = pack8(av);
-                const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(WT + (lane & 31) * 64 + kt * 16 + (lane >> 5) * 8);
-                const bf16x8 b1 =
-                    *reinterpret_cast<const bf16x8*>(WT + (32 + (lane & 31)) * 64 + kt * 16 + (lane >> 5) * 8);
-                acc0 = mfma(a, b0, acc0);
-                acc1 = mfma(a, b1, acc1);
-            }
+    for (int t = 0; t < 4; t++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const uint32_t row = row0 + rb * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (row >= n) continue;
-                const int c0 = lane & 31, c1 = 32 + (lane & 31);
-                const bool m0 = act[(size_t)row * 64 + c0] != 0 && !(act[(size_t)row * 64 + c0] & 0x8000);
-                const bool m1 = act[(size_t)row * 64 + c1] != 0 && !(act[(size_t)row * 64 + c1] & 0x8000);
-                gprev[(size_t)row * 64 + c0] = m0 ? acc0[r] : 0.0f;
-                gprev[(size_t)row * 64 + c1] = m1 ? acc1[r] : 0.0f;
-            }
-        }
+        for (int r = 0; r < 4; r++) a[4 * t + r] = v[t][r];
+    row_sum_step<0x128, 8>(a, (rl & 8) != 0);  // row_ror:8
+    row_sum_step<0x141, 4>(a, (rl & 4) != 0);  // row_half_mirror
+    row_sum_step<0x4e, 2>(a, (rl & 2) != 0);   // quad_perm [2, 3, 0, 1]
+    row_sum_step<0xb1, 1>(a, (rl & 1) != 0);   // quad_perm [1, 0, 3, 2]
+    return a[0];
+}
+
+// A lane's 16 values of a row (four tiles of four, accumulator layout) as
+// bfloat16: into the row's operand row and the transposed columns.
+__device__ __forceinline__ void put_row(const float (&v)[4][4], int quad, uint16_t* __restrict__ row,
+                                        uint16_t* __restrict__ col) {
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int c = 16 * t + 4 * quad;
+        const uint32_t a = pack2(v[t][0], v[t][1]), b = pack2(v[t][2], v[t][3]);
+        *reinterpret_cast<uint2*>(row + c) = make_uint2(a, b);
+        uint16_t* k = col + c * kTrainStride;
+        k[0] = (uint16_t)a;
+        k[kTrainStride] = (uint16_t)(a >> 16);
+        k[2 * kTrainStride] = (uint16_t)b;
+        k[3 * kTrainStride] = (uint16_t)(b >> 16);
     }
 }
 
-// Adam on the float32 masters; refreshes the bfloat16 W, W^T and biases.
-__global__ void k_adam(float* __restrict__ theta, float* __restrict__ m, float* __restrict__ v,
-                       float* __restrict__ grad, float lr, float c1, float c2, int apply, uint16_t* __restrict__ w,
-                       uint16_t* __restrict__ wt, float* __restrict__ bias) {
-    for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < kGParams; idx += gridDim.x * blockDim.x) {
-        float th = theta[idx];
-        if (apply) {
-            const float gr = grad[idx];
-            const float mm = 0.9f * m[idx] + 0.1f * gr;
-            const float vv = 0.999f * v[idx] + 0.001f * gr * gr;
-            m[idx] = mm;
-            v[idx] = vv;
-            th = th - lr * (mm / c1) / (sqrtf(vv / c2) + 1e-8f);
-            theta[idx] = th;
-            grad[idx] = 0.0f;
-        }
-        int l = 4;
-        while (l > 0 && idx < glayer_w(l)) l--;
-        const int K = glayer_in(l), off = idx - glayer_w(l);
-        if (off < glayer_out(l) * K) {
-            const int o = off / K, i = off % K;
-            w[l * kGWSlot + o * K + i] = f2bf(th);
-            wt[l * kGWSlot + i * 64 + o] = f2bf(th);
+__global__ __launch_bounds__(kTrainWaves * 64, 2) void k_train(Net net, const float* __restrict__ x,
+                                                             const float* __restrict__ dirs,
+                                                             const float* __restrict__ cw, uint32_t n,
+                                                             const float* __restrict__ sums, float* __restrict__ part,
+                                                             float* __restrict__ loss) {
+    __shared__ __align__(16) uint16_t s_col[kTrainCols * kTrainStride];      // layer inputs, transposed
+    __shared__ __align__(16) uint16_t s_g[kGHid * kTrainStride];             // a layer's gradients, transposed
+    __shared__ __align__(16) uint16_t s_row[kTrainWaves][16 * kGRowStride];  // each wave's operand rows
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int rl = lane & 15, quad = lane >> 4;   // row and column group of the 16-row products
+    const int rl32 = lane & 31, half = lane >> 5;  // of the 32x32 tiles of dW
+    uint16_t* const myrow = s_row[wave] + rl * kGRowStride;
+    float* const outs = reinterpret_cast<float*>(s_row[wave]) + rl * kTrainOutStride;
+    const int trow = wave * 16 + rl;  // the lane's row of the tile
+    float invc;
+    {
+        float t = sums[lane];
+        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off);
+        invc = 1.0f / fmaxf(t, 1e-30f);
+    }
+    f32x16 dw[6];  // 0, 1: layer 0 (the second in waves 0 and 1 only); 1 + l: layer l
+#pragma unroll
+    for (int k = 0; k < 6; k++) dw[k] = f32x16{0};
+    // bias sums: of the hidden layers over the wave's rows (row_sums), of the
+    // output layer over the lane's
+    float db[4] = {0.f, 0.f, 0.f, 0.f}, db4[10], lacc = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 10; j++) db4[j] = 0.0f;
+
+    const uint32_t tiles = (n + kTrainRows - 1) / kTrainRows;
+    const uint32_t share = (tiles + gridDim.x - 1) / gridDim.x;  // consecutive tiles of a block
+    const uint32_t end = blockIdx.x < tiles / share ? (blockIdx.x + 1) * share : tiles;
+    for (uint32_t tile = blockIdx.x * share; tile < end; tile++) {
+        const uint32_t row = tile * kTrainRows + trow;
+        const bool valid = row < n;
+        // (the weights are read again for each tile: kept in registers over the
+        // loop, they would push the accumulators to scratch memory)
+        uint32_t again = 0;
+        asm volatile("" : "+s"(again));
+        const uint16_t *w_all = net.w16 + again, *wt_all = net.wt16 + again;
+        const float* b_all = net.bias + again;
+        // ---- inputs
+        f32x4 xin[6];
+        vec3 d = v3(0.f, 0.f, 1.f);
+        float ci = 0.0f;
+        if (valid) {
+            const f32x4_any* src = reinterpret_cast<const f32x4_any*>(x + (size_t)row * kGIn) + quad;
+#pragma unroll
+            for (int q = 0; q < 6; q++) xin[q] = src[4 * q];
+            d = v3(dirs[3 * (size_t)row], dirs[3 * (size_t)row + 1], dirs[3 * (size_t)row + 2]);
+            ci = cw[row];
         } else {
-            bias[l * 64 + (off - glayer_out(l) * K)] = th;
+#pragma unroll
+            for (int q = 0; q < 6; q++) xin[q] = f32x4{0};
+        }
+        __syncthreads();  // the previous tile's columns have been read
+#pragma unroll
+        for (int q = 0; q < 6; q++) {
+            const int c = 16 * q + 4 * quad;
+            const uint32_t a = pack2(xin[q].x, xin[q].y), b = pack2(xin[q].z, xin[q].w);
+            *reinterpret_cast<uint2*>(myrow + c) = make_uint2(a, b);
+            uint16_t* k = s_col + c * kTrainStride + trow;
+            k[0] = (uint16_t)a;
+            k[kTrainStride] = (uint16_t)(a >> 16);
+            k[2 * kTrainStride] = (uint16_t)b;
+            k[3 * kTrainStride] = (uint16_t)(b >> 16);
+        }
+        lds_order();
+        // ---- forward
+        uint32_t mask[4];  // ReLU of layers 0..3: bit 4 t + r
+        float v[4][4];
+#pragma unroll
+        for (int l = 0; l < 5; l++) {
+            constexpr int kK[5] = {kGIn, kGHid, kGHid, kGHid, kGHid};
+            const int T = l < 4 ? 4 : kGOut / 16;
+            const uint16_t* W = w_all + l * kGWSlot + lane * 8;
+            const float4* bias = reinterpret_cast<const float4*>(b_all + l * 64) + quad;
+            f32x4 acc[4];
+#pragma unroll
+            for (int t = 0; t < 4; t++) acc[t] = f32x4{0};
+#pragma unroll
+            for (int kt = 0; kt < kK[l] / 32; kt++) {
+                const bf16x8 b = *reinterpret_cast<const bf16x8*>(myrow + kt * 32 + quad * 8);
+#pragma unroll
+                for (int t = 0; t < T; t++)
+                    acc[t] = mfma16(*reinterpret_cast<const bf16x8*>(W + (t * (kK[l] / 32) + kt) * 512), b, acc[t]);
+            }
+            lds_order();
+            uint32_t m = 0;
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                const float4 b4 = bias[4 * t];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float a = acc[t][r] + (r == 0 ? b4.x : r == 1 ? b4.y : r == 2 ? b4.z : b4.w);
+                    v[t][r] = l < 4 ? fmaxf(a, 0.0f) : a;
+                    if (l < 4) m |= a > 0.0f ? 1u << (4 * t + r) : 0u;
+                }
+            }
+            if (l < 4) {
+                mask[l] = m;
+                put_row(v, quad, myrow, s_col + train_col(l + 1) * kTrainStride + trow);
+                lds_order();
+            }
+        }
+        // ---- loss
+#pragma unroll
+        for (int t = 0; t < kGOut / 16; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) outs[16 * t + 4 * quad + r] = v[t][r];
+        lds_order();
+        float o[10], gl[10];
+#pragma unroll
+        for (int j = 0; j < 10; j++) o[j] = outs[10 * quad + j];
+        lds_order();
+        {
+            auto over_quads = [](float a) {
+                a += __shfl_xor(a, 16);
+                return a + __shfl_xor(a, 32);
+            };
+            float mx = fmaxf(o[0], o[5]);
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            float e[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) e[j] = expf(o[5 * j] - mx);
+            const float sum = over_quads(e[0] + e[1]);
+            float w[2], kap[2], sg[2], nm[2], dt[2], f[2];
+            vec3 mu[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                w[j] = e[j] / sum;
+                sg[j] = 1.0f / (1.0f + expf(-o[5 * j + 1]));
+                kap[j] = expf(kGKappaLo + (kGKappaHi - kGKappaLo) * sg[j]);
+                const float a = o[5 * j + 2], b = o[5 * j + 3], c = o[5 * j + 4];
+                nm[j] = fmaxf(sqrtf(a * a + b * b + c * c), 1e-6f);
+                mu[j] = v3(a / nm[j], b / nm[j], c / nm[j]);
+                dt[j] = dot(mu[j], d);
+                f[j] = vmf_pdf(kap[j], mu[j], d);
+            }
+            const float q = over_quads(w[0] * f[0] + w[1] * f[1]);
+            const float qs = fmaxf(q, 1e-30f);
+            if (quad == 0) lacc += -ci * logf(qs) * invc;
+            const float gq = -ci / qs * invc;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const float wf = w[j] * f[j], k = kap[j];
+                gl[5 * j] = gq * (wf - w[j] * q);
+                const float em = -expm1f(-2.0f * k);
+                const float dlogf = 1.0f / k - 2.0f * expf(-2.0f * k) / em + (dt[j] - 1.0f);
+                gl[5 * j + 1] = gq * wf * dlogf * k * (kGKappaHi - kGKappaLo) * sg[j] * (1.0f - sg[j]);
+                const float s = gq * wf * k / nm[j];
+                gl[5 * j + 2] = s * (d.x - dt[j] * mu[j].x);
+                gl[5 * j + 3] = s * (d.y - dt[j] * mu[j].y);
+                gl[5 * j + 4] = s * (d.z - dt[j] * mu[j].z);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 10; j += 2) {
+            db4[j] += gl[j];
+            db4[j + 1] += gl[j + 1];
+            const uint32_t a = pack2(gl[j], gl[j + 1]);
+            const int c = 10 * quad + j;
+            *reinterpret_cast<uint32_t*>(myrow + c) = a;
+            s_g[c * kTrainStride + trow] = (uint16_t)a;
+            s_g[(c + 1) * kTrainStride + trow] = (uint16_t)(a >> 16);
+        }
+        // columns 40..47 carry no output (gradient zero), 48..63 pad the product
+        // (their dW is discarded)
+#pragma unroll
+        for (int j = 0; j < 6; j += 2) *reinterpret_cast<uint32_t*>(myrow + kGMix + 6 * quad + j) = 0u;
+#pragma unroll
+        for (int j = 0; j < 2; j++) s_g[(kGMix + 2 * quad + j) * kTrainStride + trow] = 0;
+        // ---- backward
+#pragma unroll
+        for (int l = 4; l >= 0; l--) {
+            __syncthreads();  // every wave's rows of s_g are there
+            auto dw_tile = [&](int ot, int it, f32x16& acc) {
+                const uint16_t* A = s_g + (ot * 32 + rl32) * kTrainStride + half * 8;
+                const uint16_t* B = s_col + (train_col(l) + it * 32 + rl32) * kTrainStride + half * 8;
+#pragma unroll
+                for (int kt = 0; kt < kTrainRows / 16; kt++)
+                    acc = mfma(*reinterpret_cast<const bf16x8*>(A + kt * 16),
+                               *reinterpret_cast<const bf16x8*>(B + kt * 16), acc);
+            };
+            if (l > 0) {
+                dw_tile(wave >> 1, wave & 1, dw[1 + l]);
+                const uint16_t* WT = wt_all + l * kGWSlot + lane * 8;
+                f32x4 acc[4];
+#pragma unroll
+                for (int t = 0; t < 4; t++) acc[t] = f32x4{0};
+#pragma unroll
+                for (int kt = 0; kt < 2; kt++) {
+                    const bf16x8 b = *reinterpret_cast<const bf16x8*>(myrow + kt * 32 + quad * 8);
+#pragma unroll
+                    for (int t = 0; t < 4; t++)
+                        acc[t] = mfma16(*reinterpret_cast<const bf16x8*>(WT + (2 * t + kt) * 512), b, acc[t]);
+                }
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) v[t][r] = (mask[l - 1] >> (4 * t + r)) & 1u ? acc[t][r] : 0.0f;
+                db[l - 1] += row_sums(v, rl);
+                __syncthreads();  // dW has read s_g
+                put_row(v, quad, myrow, s_g + trow);
+            } else {
+                dw_tile(wave / 3, wave % 3, dw[0]);
+                if (wave < 2) dw_tile(1, wave + 1, dw[1]);
+            }
         }
     }
+    // ---- the block's partial gradient
+    float* const dst = part + (size_t)blockIdx.x * kGParams;
+    auto put_dw = [&](int l, int ot, int it, const f32x16& acc) {
+        const int K = glayer_in(l);
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int o = ot * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+            if (o < glayer_out(l)) dst[glayer_w(l) + o * K + it * 32 + rl32] = acc[r];
+        }
+    };
+    put_dw(0, wave / 3, wave % 3, dw[0]);
+    if (wave < 2) put_dw(0, 1, wave + 1, dw[1]);
+#pragma unroll
+    for (int l = 1; l < 5; l++) put_dw(l, wave >> 1, wave & 1, dw[1 + l]);
+    // bias sums: over the wave's rows, then over the waves
+    __syncthreads();
+    float* const s_b = reinterpret_cast<float*>(s_col);  // [wave][5][64], then the losses
+    auto over_rows = [](float a) {
+        for (int off = 8; off > 0; off >>= 1) a += __shfl_xor(a, off);
+        return a;
+    };
+#pragma unroll
+    for (int l = 0; l < 4; l++) s_b[(wave * 5 + l) * 64 + 16 * (rl >> 2) + 4 * quad + (rl & 3)] = db[l];
+#pragma unroll
+    for (int j = 0; j < 10; j++) {
+        const float a = over_rows(db4[j]);
+        if (rl == 0) s_b[(wave * 5 + 4) * 64 + 10 * quad + j] = a;
+    }
+    if (quad == 0 && rl < kGOut - kGMix) s_b[(wave * 5 + 4) * 64 + kGMix + rl] = 0.0f;
+    lacc = over_rows(lacc);
+    if (lane == 0) s_b[kTrainWaves * 5 * 64 + wave] = lacc;
+    __syncthreads();
+    for (int k = threadIdx.x; k < 5 * 64; k += kTrainWaves * 64) {
+        const int l = k >> 6, o = k & 63;
+        if (o < glayer_out(l))
+            dst[glayer_b(l) + o] = (s_b[k] + s_b[5 * 64 + k]) + (s_b[10 * 64 + k] + s_b[15 * 64 + k]);
+    }
+    if (threadIdx.x == 0) {
+        const float* w = s_b + kTrainWaves * 5 * 64;
+        loss[blockIdx.x] = (w[0] + w[1]) + (w[2] + w[3]);
+    }
+}
+
+// A parameter's float32 value to the network's bfloat16 copies and biases.
+__device__ __forceinline__ void refresh_param(int idx, float th, uint16_t* __restrict__ w, uint16_t* __restrict__ w16,
+                                              uint16_t* __restrict__ wt16, float* __restrict__ bias) {
+    int l = 4;
+    while (l > 0 && idx < glayer_w(l)) l--;
+    const int K = glayer_in(l), off = idx - glayer_w(l);
+    if (off < glayer_out(l) * K) {
+        const int o = off / K, i = off % K;
+        w[l * kGWSlot + operand_index(o, i, K)] = f2bf(th);
+        w16[l * kGWSlot + operand16_index(o, i, K)] = f2bf(th);
+        wt16[l * kGWSlot + operand16_index(i, o, 64)] = f2bf(th);
+    } else {
+        bias[l * 64 + (off - glayer_out(l) * K)] = th;
+    }
+}
+
+__global__ void k_refresh(const float* __restrict__ theta, uint16_t* __restrict__ w, uint16_t* __restrict__ w16,
+                          uint16_t* __restrict__ wt16, float* __restrict__ bias) {
+    for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < kGParams; idx += gridDim.x * blockDim.x)
+        refresh_param(idx, theta[idx], w, w16, wt16, bias);
+}
+
+// grad[e] += sum over blocks of part[block][e], and with `apply` the Adam
+// update of parameter e from it; the step's loss from the blocks' losses.
+// Block: 64 parameters, read 16 bytes a lane, x 16 groups of partials (group q
+// sums blocks q, q + 16, ...); everything is added in a fixed order.  Bound by
+// the reads of the partials: 512 of 21,808 parameters (45 MB): 12.6 us.
+// With four groups of 4-byte reads a thread had 128 dependent additions and few
+// reads in flight: 39 us.
+constexpr int kReduceGroups = 16;
+struct AdamArgs {
+    float *theta, *m, *v, *grad;
+    float lr, c1, c2;
+    int apply;
+    uint16_t *w, *w16, *wt16;
+    float* bias;
+};
+__global__ __launch_bounds__(256) void k_train_reduce(const float* __restrict__ part, uint32_t blocks, AdamArgs a,
+                                                      const float* __restrict__ block_loss, float* __restrict__ loss) {
+    static_assert(kGParams % 4 == 0, "the partials are read in float4");
+    __shared__ __align__(16) float s_sum[kReduceGroups][64];
+    const uint32_t q = threadIdx.x >> 4, e4 = blockIdx.x * 64 + 4 * (threadIdx.x & 15);
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (e4 < (uint32_t)kGParams) {
+        const float* src = part + e4;
+#pragma unroll 8
+        for (uint32_t b = q; b < blocks; b += kReduceGroups) {
+            const float4 t = *reinterpret_cast<const float4*>(src + (size_t)b * kGParams);
+            v.x += t.x;
+            v.y += t.y;
+            v.z += t.z;
+            v.w += t.w;
+        }
+    }
+    *reinterpret_cast<float4*>(&s_sum[q][4 * (threadIdx.x & 15)]) = v;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const uint32_t e = blockIdx.x * 64 + threadIdx.x;
+    if (blockIdx.x == 0) {
+        float t = 0.0f;
+        for (uint32_t b = threadIdx.x; b < blocks; b += 64) t += block_loss[b];
+        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off);
+        if (threadIdx.x == 0) *loss = t;
+    }
+    if (e >= (uint32_t)kGParams) return;
+    float sum[kReduceGroups];
+#pragma unroll
+    for (int k = 0; k < kReduceGroups; k++) sum[k] = s_sum[k][threadIdx.x];
+#pragma unroll
+    for (int n = 1; n < kReduceGroups; n *= 2)
+#pragma unroll
+        for (int k = 0; k < kReduceGroups; k += 2 * n) sum[k] += sum[k + n];
+    const float gr = a.grad[e] + sum[0];
+    if (!a.apply) {
+        a.grad[e] = gr;
+        return;
+    }
+    const float mm = 0.9f * a.m[e] + 0.1f * gr;
+    const float vv = 0.999f * a.v[e] + 0.001f * gr * gr;
+    a.m[e] = mm;
+    a.v[e] = vv;
+    const float th = a.theta[e] - a.lr * (mm / a.c1) / (sqrtf(vv / a.c2) + 1e-8f);
+    a.theta[e] = th;
+    a.grad[e] = 0.0f;
+    refresh_param((int)e, th, a.w, a.w16, a.wt16, a.bias);
 }
 
 // Training weight of one render record: c = L_i(d) / p(d), the incident
@@ -415,18 +672,16 @@ __global__ void k_resample(const float* __restrict__ rec, uint32_t R, const floa
 // host side
 // ---------------------------------------------------------------------------
 // the device bytes the render service reserves for a guided render
-static_assert(kGuideBatch == dl_sizes::kGuideBatchRows && kChunk == (int)dl_sizes::kGuideChunkRows &&
-                  kScanTile == (int)dl_sizes::kGuideScanTile && kGParams == dl_sizes::kGuideParams &&
+static_assert(kGuideBatch == dl_sizes::kGuideBatchRows && kScanTile == (int)dl_sizes::kGuideScanTile && kGParams == dl_sizes::kGuideParams &&
                   kGWSlot == dl_sizes::kGuideWSlot,
               "guided render sizes");
 static_assert(dl_sizes::kGuideNetBytes == 4ull * kGParams * sizeof(float) + 5 * 64 * sizeof(float) +
-                                              2ull * 5 * kGWSlot * sizeof(uint16_t) + 4 * sizeof(float),
+                                              3ull * 5 * kGWSlot * sizeof(uint16_t) +
+                                              (4 + kSumBlocks + dl_sizes::kGuideTrainBlocks) * sizeof(float),
               "guide_init allocations");
-static_assert(dl_sizes::kGuideTrainBytes ==
-                  (uint64_t)kGuideBatch * ((glayer_in(0) + 4 * glayer_in(1)) * sizeof(uint16_t) +
-                                           (kGOut + 2 * 64) * sizeof(float) + (kGIn + 3 + 1) * sizeof(float)) +
-                      (uint64_t)(kGuideBatch / kChunk) * (64 * 96 + 64) * sizeof(float),
-              "ensure_train and training batch allocations");
+static_assert(dl_sizes::kGuideTrainBytes == (uint64_t)kGuideBatch * (kGIn + 3 + 1) * sizeof(float) +
+                                                (uint64_t)dl_sizes::kGuideTrainBlocks * kGParams * sizeof(float),
+              "training batch and partial gradients");
 
 struct GuideState {
     // training batch built from render records
@@ -436,14 +691,11 @@ struct GuideState {
     uint32_t rw_cap = 0;
     float *rw = nullptr, *tile_sum = nullptr, *tile_off = nullptr;
     float *theta = nullptr, *m = nullptr, *v = nullptr, *grad = nullptr, *bias = nullptr;
-    uint16_t *w = nullptr, *wt = nullptr;
+    uint16_t *w = nullptr, *w16 = nullptr, *wt16 = nullptr;
     int step = 0;
     float lr = 1e-2f;
-    // training buffers
-    uint32_t cap = 0;
-    uint16_t* act[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
-    float *out = nullptr, *g0 = nullptr, *g1 = nullptr, *scalars = nullptr;
-    float* part = nullptr;  // per-chunk partial weight/bias gradients of one layer
+    float* scalars = nullptr;  // [1]: the step's loss; then the partial sums of the weights, the blocks' losses
+    float* part = nullptr;     // per-block partial gradients of a training step
     std::vector<void*> allocs;
 };
 
@@ -464,7 +716,7 @@ dl_status galloc(Ctx* c, GuideState* g, T** p, size_t count) {
         if (s_ != DL_OK) return s_; \
     } while (0)
 
-Net net_of(const GuideState* g) { return Net{g->w, g->wt, g->bias}; }
+Net net_of(const GuideState* g) { return Net{g->w, g->w16, g->wt16, g->bias}; }
 
 // Deterministic initial weights: He-uniform (last layer x0.1), zero biases,
 // uniforms from splitmix64 (Steele et al. 2014).
@@ -482,28 +734,6 @@ void init_weights(uint64_t seed, std::vector<float>& th) {
         const float a = std::sqrt(6.0f / glayer_in(l)) * (l == 4 ? 0.1f : 1.0f);
         for (int k = 0; k < glayer_out(l) * glayer_in(l); k++) th[glayer_w(l) + k] = (2.0f * next() - 1.0f) * a;
     }
-}
-
-dl_status ensure_train(Ctx* c, GuideState* g, uint32_t n) {
-    if (g->cap >= n) return DL_OK;
-    for (int l = 0; l < 5; l++)
-        if (g->act[l]) {
-            dfree(c, g->act[l]);
-            g->allocs.erase(std::find(g->allocs.begin(), g->allocs.end(), (void*)g->act[l]));
-        }
-    for (float** p : {&g->out, &g->g0, &g->g1, &g->part})
-        if (*p) {
-            dfree(c, *p);
-            g->allocs.erase(std::find(g->allocs.begin(), g->allocs.end(), (void*)*p));
-        }
-    g->cap = n;
-    for (int l = 0; l < 5; l++) DL_TRY(galloc(c, g, &g->act[l], (size_t)n * glayer_in(l)));
-    DL_TRY(galloc(c, g, &g->out, (size_t)n * kGOut));
-    DL_TRY(galloc(c, g, &g->g0, (size_t)n * 64));
-    DL_TRY(galloc(c, g, &g->g1, (size_t)n * 64));
-    // largest layer: 64 x 96 weights + 64 biases per chunk
-    DL_TRY(galloc(c, g, &g->part, (size_t)((n + kChunk - 1) / kChunk) * (64 * 96 + 64)));
-    return DL_OK;
 }
 
 }  // namespace
@@ -531,8 +761,9 @@ dl_status guide_init(Ctx* c, uint64_t seed, float lr, const float* params) {
     DL_TRY(galloc(c, g, &g->grad, kGParams));
     DL_TRY(galloc(c, g, &g->bias, 5 * 64));
     DL_TRY(galloc(c, g, &g->w, 5 * kGWSlot));
-    DL_TRY(galloc(c, g, &g->wt, 5 * kGWSlot));
-    DL_TRY(galloc(c, g, &g->scalars, 4));
+    DL_TRY(galloc(c, g, &g->w16, 5 * kGWSlot));
+    DL_TRY(galloc(c, g, &g->wt16, 5 * kGWSlot));
+    DL_TRY(galloc(c, g, &g->scalars, 4 + kSumBlocks + dl_sizes::kGuideTrainBlocks));
     std::vector<float> th;
     if (params)
         th.assign(params, params + kGParams);
@@ -543,22 +774,21 @@ dl_status guide_init(Ctx* c, uint64_t seed, float lr, const float* params) {
     DL_HIP_CHECK(c, hipMemsetAsync(g->v, 0, kGParams * sizeof(float), c->stream));
     DL_HIP_CHECK(c, hipMemsetAsync(g->grad, 0, kGParams * sizeof(float), c->stream));
     DL_HIP_CHECK(c, hipMemsetAsync(g->w, 0, 5 * kGWSlot * sizeof(uint16_t), c->stream));
-    DL_HIP_CHECK(c, hipMemsetAsync(g->wt, 0, 5 * kGWSlot * sizeof(uint16_t), c->stream));
+    DL_HIP_CHECK(c, hipMemsetAsync(g->w16, 0, 5 * kGWSlot * sizeof(uint16_t), c->stream));
+    DL_HIP_CHECK(c, hipMemsetAsync(g->wt16, 0, 5 * kGWSlot * sizeof(uint16_t), c->stream));
     DL_HIP_CHECK(c, hipMemsetAsync(g->bias, 0, 5 * 64 * sizeof(float), c->stream));
-    k_adam<<<(kGParams + 255) / 256, 256, 0, c->stream>>>(g->theta, g->m, g->v, g->grad, 0.f, 1.f, 1.f, 0, g->w,
-                                                          g->wt, g->bias);
+    k_refresh<<<(kGParams + 255) / 256, 256, 0, c->stream>>>(g->theta, g->w, g->w16, g->wt16, g->bias);
     DL_HIP_CHECK(c, hipGetLastError());
     return DL_OK;
 }
 
 // Forward pass over n float32 input rows (device), raw outputs to out.
-dl_status guide_forward(Ctx* c, const float* x, uint32_t n, float* out, bool keep) {
+dl_status guide_forward(Ctx* c, const float* x, uint32_t n, float* out) {
     GuideState* g = (GuideState*)c->guide;
     if (n == 0) return DL_OK;
     const uint32_t tiles = (n + kGRowsPerWave - 1) / kGRowsPerWave;
     const int grid = (int)std::max<uint32_t>(1, std::min<uint32_t>((tiles + kGWaves - 1) / kGWaves, (uint32_t)c->num_cus * 4));
-    k_mlp_forward<<<grid, kGWaves * 64, 0, c->stream>>>(net_of(g), x, n, out, keep ? 1 : 0, g->act[0], g->act[1],
-                                                       g->act[2], g->act[3], g->act[4]);
+    k_mlp_forward<<<grid, kGWaves * 64, 0, c->stream>>>(net_of(g), x, n, out);
     DL_HIP_CHECK(c, hipGetLastError());
     return DL_OK;
 }
@@ -566,50 +796,24 @@ dl_status guide_forward(Ctx* c, const float* x, uint32_t n, float* out, bool kee
 // One training step on n records (device arrays): gradient, then Adam.
 dl_status guide_train(Ctx* c, const float* x, const float* dirs, const float* cw, uint32_t n, bool apply) {
     GuideState* g = (GuideState*)c->guide;
-    DL_TRY(ensure_train(c, g, n));
-    DL_HIP_CHECK(c, hipMemsetAsync(g->scalars, 0, 4 * sizeof(float), c->stream));
-    DL_TRY(guide_forward(c, x, n, g->out, true));
-    const int eg = std::max(1, std::min<int>((int)((n + 255) / 256), c->num_cus * 8));
-    k_sum<<<std::min(eg, 64), 256, 0, c->stream>>>(cw, n, g->scalars);
-    k_loss_grad<<<eg, 256, 0, c->stream>>>(g->out, dirs, cw, n, g->scalars, g->g0, g->scalars + 1);
-    float* gcur = g->g0;
-    float* gnext = g->g1;
-    int gw = kGOut;
-    const uint32_t chunks = (n + kChunk - 1) / kChunk;
-    for (int l = 4; l >= 0; l--) {
-        const int K = glayer_in(l);
-        const uint32_t cnt = (uint32_t)(gw * K + gw);
-        k_dw<<<dim3((gw + 31) / 32, K / 32, chunks), kDwWaves * 64, 0, c->stream>>>(gcur, gw, g->act[l], K, n,
-                                                                                    g->part);
-        k_dw_reduce<<<(cnt + 63) / 64, 256, 0, c->stream>>>(g->part, chunks, cnt, g->grad + glayer_w(l));
-        if (l > 0) {
-            const uint32_t tiles = (n + kGRowsPerWave - 1) / kGRowsPerWave;
-            const int grid = (int)std::max<uint32_t>(
-                1, std::min<uint32_t>((tiles + kGWaves - 1) / kGWaves, (uint32_t)c->num_cus * 4));
-            k_dact<<<grid, kGWaves * 64, 0, c->stream>>>(net_of(g), l, gcur, gw, g->act[l], n, gnext);
-            std::swap(gcur, gnext);
-            gw = 64;
-        }
-    }
+    if (!g->part) DL_TRY(galloc(c, g, &g->part, (size_t)dl_sizes::kGuideTrainBlocks * kGParams));
+    const uint32_t blocks = std::min<uint32_t>((uint32_t)std::min(std::max(1, 2 * c->num_cus), (int)dl_sizes::kGuideTrainBlocks),
+                                               (n + kTrainRows - 1) / kTrainRows);
+    float* const sums = g->scalars + 4;
+    float* const losses = sums + kSumBlocks;
+    k_sum<<<kSumBlocks, 256, 0, c->stream>>>(cw, n, sums);
+    k_train<<<blocks, kTrainWaves * 64, 0, c->stream>>>(net_of(g), x, dirs, cw, n, sums, g->part, losses);
+    if (apply) g->step++;
+    AdamArgs a{g->theta, g->m, g->v, g->grad, g->lr, 1.0f - std::pow(0.9f, (float)g->step),
+               1.0f - std::pow(0.999f, (float)g->step), apply ? 1 : 0, g->w, g->w16, g->wt16, g->bias};
+    k_train_reduce<<<(kGParams + 63) / 64, 256, 0, c->stream>>>(g->part, blocks, a, losses, g->scalars + 1);
     DL_HIP_CHECK(c, hipGetLastError());
-    if (apply) {
-        g->step++;
-        const float c1 = 1.0f - std::pow(0.9f, (float)g->step), c2 = 1.0f - std::pow(0.999f, (float)g->step);
-        k_adam<<<(kGParams + 255) / 256, 256, 0, c->stream>>>(g->theta, g->m, g->v, g->grad, g->lr, c1, c2, 1, g->w,
-                                                              g->wt, g->bias);
-        DL_HIP_CHECK(c, hipGetLastError());
-    }
     return DL_OK;
 }
 
 int guide_step_count(Ctx* c) { return c->guide ? ((GuideState*)c->guide)->step : 0; }
 
-void guide_net_ptrs(Ctx* c, const uint16_t** w, const uint16_t** wt, const float** bias) {
-    GuideState* g = (GuideState*)c->guide;
-    *w = g->w;
-    *wt = g->wt;
-    *bias = g->bias;
-}
+Net guide_net(Ctx* c) { return net_of((GuideState*)c->guide); }
 
 // `steps` Adam steps on batches of kGuideBatch records resampled from the R
 // render records in proportion to their weights; returns the steps taken.
@@ -700,7 +904,7 @@ dl_status dl_hip_guide_eval(void* h, const float* x, uint32_t n, float* out, flo
     if (!c || !x || !out) return DL_ERR_INVALID;
     if (!c->guide) return set_error(c, DL_ERR_STATE, "guide not initialised");
     (void)hipSetDevice(c->device);
-    DL_TRY(guide_forward(c, x, n, out, false));
+    DL_TRY(guide_forward(c, x, n, out));
     if (mix) DL_TRY(guide_decode_rows(c, out, n, mix));
     DL_HIP_CHECK(c, hipStreamSynchronize(c->stream));
     return DL_OK;

@@ -1220,7 +1220,7 @@ __global__ __launch_bounds__(kGWaves * 64) void k_guide_infer(PassParams pp, Sce
         // raw outputs overwrite the activation rows of their own 32-row block
         // after that block's last MFMA (byte ranges checked: 192 B per output
         // row vs 208 B per activation row)
-        forward_rows(net, sm, row0, n, false, nullptr, [&](int r, int c, float v) { smf[r * kGOut + c] = v; });
+        forward_rows(net, sm, [&](int r, int c, float v) { smf[r * kGOut + c] = v; });
         if (i < n) {
             float o[kGOut], mix[kGMix];
             for (int j = 0; j < kGOut; j++) o[j] = smf[lane * kGOut + j];
@@ -1793,7 +1793,7 @@ dl_status render(Ctx* c, const dl_render_params* prm, float* rgb_host, dl_render
     if (guided) {
         if (!c->guide) DL_TRY(guide_init(c, 0x5EEDull + prm->seed, 1e-2f, nullptr));
         DL_TRY(ensure_guide_bufs(c, rs, cap));
-        guide_net_ptrs(c, &net.w, &net.wt, &net.bias);
+        net = guide_net(c);
         gv.mix = rs->b.gmix;
         gv.frac = kGuideFraction;
         gv.rec = train ? rs->b.grec : nullptr;

@@ -25,29 +25,34 @@ constexpr int kGuideMixFloats = 40;          // decoded mixture per queued shadi
 constexpr int kGuideRecordFloats = 24;       // training record
 constexpr uint32_t kGuideRecordSlots = 1u << 23;
 constexpr uint32_t kGuideBatchRows = 1u << 18;  // records per Adam step
-constexpr uint32_t kGuideChunkRows = 1024;      // rows per partial weight gradient
+constexpr uint32_t kGuideTrainBlocks = 512;     // blocks of a training step (at most), a partial gradient each
+constexpr uint32_t kGuideSumBlocks = 64;        // partial sums of the training weights
 constexpr uint32_t kGuideScanTile = 1024;       // records per prefix-sum tile
 constexpr int kGuideParams = 21808;
-constexpr int kGuideWSlot = 64 * 96;            // bfloat16 elements per layer copy (W or W^T)
+constexpr int kGuideWSlot = 64 * 96;            // bfloat16 elements per layer copy
 
-// network parameters, Adam moments, gradient, biases, bfloat16 W and W^T,
-// scalars
-constexpr uint64_t kGuideNetBytes = 4ull * kGuideParams * 4 + 5 * 64 * 4 + 2ull * 5 * kGuideWSlot * 2 + 4 * 4;
-// one training batch: bfloat16 layer inputs (96 + 4 x 64 per row), outputs
-// (48), two gradient rows (64 each), per-chunk partial gradients of the
-// largest layer; the batch's features (96), directions (3) and weights (1)
+// network parameters, Adam moments, gradient, biases, bfloat16 copies
+// (W in two orders, W^T), scalars and partial sums
+constexpr uint64_t kGuideNetBytes = 4ull * kGuideParams * 4 + 5 * 64 * 4 + 3ull * 5 * kGuideWSlot * 2 +
+                                    (4 + kGuideSumBlocks + kGuideTrainBlocks) * 4;
+// one training batch: its features (96), directions (3) and weights (1); the
+// blocks' partial gradients
 constexpr uint64_t kGuideTrainBytes =
-    (uint64_t)kGuideBatchRows * ((96 + 4 * 64) * 2 + 48 * 4 + 2 * 64 * 4 + (96 + 3 + 1) * 4) +
-    (uint64_t)(kGuideBatchRows / kGuideChunkRows) * (64 * 96 + 64) * 4;
+    (uint64_t)kGuideBatchRows * (96 + 3 + 1) * 4 + (uint64_t)kGuideTrainBlocks * kGuideParams * 4;
 // record weights and the prefix-sum tiles over every record slot
 constexpr uint64_t kGuideResampleBytes =
     (uint64_t)kGuideRecordSlots * 4 + 2ull * (kGuideRecordSlots / kGuideScanTile + 1) * 4;
+
+// Headroom of a guided job's reservation, which stays more than 1 GiB above a
+// plain job's as budgets expect (a step's activations and gradients, 0.39 GB,
+// are no longer kept in memory).
+constexpr uint64_t kGuideHeadroomBytes = 128ull << 20;
 
 // Everything a guided render adds to a plain one whose passes hold `paths`
 // paths.
 constexpr uint64_t guide_bytes(uint64_t paths) {
     return paths * kGuideMixFloats * 4 + (uint64_t)kGuideRecordSlots * kGuideRecordFloats * 4 + kGuideNetBytes +
-           kGuideTrainBytes + kGuideResampleBytes;
+           kGuideTrainBytes + kGuideResampleBytes + kGuideHeadroomBytes;
 }
 
 }  // namespace dl_sizes

@@ -72,6 +72,33 @@ def test_gradient_matches_oracle(backend):
             k += size
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 127, 32767, 32769, 70001])
+def test_gradient_at_tile_edges(backend, n):
+    """Rows short of a wave's 16, of a block's 64 and of one tile per block,
+    and blocks with several tiles.  The matrix products read bfloat16 (2^-9
+    relative per operand): through ten of them the gradient of a layer keeps
+    its norm to 5 %, as for the batch above, and for the few rows whose
+    gradient is one sample's, to the 10 % that a single lobe's concentration
+    (exp of a rounded output) allows."""
+    th = _theta(41)
+    x, rng = _inputs(42, n)
+    d = rng.normal(size=(n, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    c = rng.random(n) + 0.1
+    backend.guide_init(params=th)
+    loss = backend.guide_train_step(x, d, c, apply=False)
+    _, g = backend.guide_params()
+    rl, rg = G.loss_and_grad(th, x, d, c)
+    assert loss == pytest.approx(rl, rel=2e-2 if n < 128 else 2e-3)
+    k = 0
+    for i, o in G.LAYERS:
+        for size in (o * i, o):
+            a, b = g[k:k + size], rg[k:k + size]
+            rel = np.linalg.norm(a - b) / (np.linalg.norm(b) + 1e-12)
+            assert rel < (0.10 if n < 128 else 0.05), (i, o, size, rel)
+            k += size
+
+
 def test_adam_step_matches_oracle(backend):
     th = _theta(31)
     x, rng = _inputs(32, 2048)

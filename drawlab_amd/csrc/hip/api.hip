@@ -66,6 +66,7 @@ void swap_scene(Ctx* c, SceneState& s) {
 
 void free_scene(Ctx* c) {
     free_scene_union(c);
+    trim_build(c, true);
     if (c->stream) hipStreamSynchronize(c->stream);
     // the acceleration structure is allocated by the builders, outside
     // scene_allocs
@@ -109,6 +110,7 @@ dl_status check_camera(Ctx* c, const dl_camera_desc& cam) {
 // under its key when it has one, freed otherwise.
 void release_current(Ctx* c) {
     invalidate_film(c);
+    trim_build(c, true);
     if (c->scene_key != 0 && c->has_scene) {
         SceneState s;
         swap_scene(c, s);
@@ -472,15 +474,17 @@ dl_status dl_hip_build_accel(void* h, int builder, dl_accel_stats* stats) {
     if (!c->has_scene) return set_error(c, DL_ERR_STATE, "build_accel before upload_scene");
     hipSetDevice(c->device);
     free_scene_union(c);  // it may hold this scene's previous BVH
-    if (c->ds.nodes) {
-        dfree(c, c->ds.nodes);
-        dfree(c, c->ds.tris);
-        c->ds.nodes = nullptr;
-        c->ds.tris = nullptr;
-    }
     dl_accel_stats st{};
     if (builder != DL_BUILD_GPU && builder != DL_BUILD_GPU_LBVH && builder != DL_BUILD_HOST_SAH)
         return set_error(c, DL_ERR_INVALID, "unknown builder");
+    // a previous structure's buffers are written again where their size still
+    // fits: nothing on any stream may be reading them
+    DL_HIP_CHECK(c, hipDeviceSynchronize());
+    c->has_accel = false;
+    struct Trim {
+        Ctx* c;
+        ~Trim() { trim_build(c, false); }
+    } trim{c};
     bool host = builder == DL_BUILD_HOST_SAH;
     if (!host) {
         c->bvh_too_deep = false;
@@ -489,10 +493,6 @@ dl_status dl_hip_build_accel(void* h, int builder, dl_accel_stats* stats) {
         if (s != DL_OK) {
             // a tree deeper than the traversal stack allows (pathological
             // geometry): rebuilt by the host builder, whose depth is bounded
-            dfree(c, c->ds.nodes);
-            dfree(c, c->ds.tris);
-            c->ds.nodes = nullptr;
-            c->ds.tris = nullptr;
             st = dl_accel_stats{};
             host = true;
             c->err.clear();
@@ -503,15 +503,7 @@ dl_status dl_hip_build_accel(void* h, int builder, dl_accel_stats* stats) {
         HostBvh bvh;
         build_bvh_host(c->tri_verts.data(), c->nprims, bvh);
         auto t1 = std::chrono::steady_clock::now();
-        void* pn = nullptr;
-        void* pt = nullptr;
-        DL_HIP_CHECK(c, dmalloc(c, &pn, bvh.nodes.size() * sizeof(BvhNodeH)));
-        DL_HIP_CHECK(c, dmalloc(c, &pt, std::max<size_t>(1, bvh.tris.size()) * sizeof(BvhTriH)));
-        DL_HIP_CHECK(c, hipMemcpy(pn, bvh.nodes.data(), bvh.nodes.size() * sizeof(BvhNodeH), hipMemcpyHostToDevice));
-        if (!bvh.tris.empty())
-            DL_HIP_CHECK(c, hipMemcpy(pt, bvh.tris.data(), bvh.tris.size() * sizeof(BvhTriH), hipMemcpyHostToDevice));
-        c->ds.nodes = (float4*)pn;
-        c->ds.tris = (float4*)pt;
+        DL_TRY(upload_host_bvh(c, bvh));
         st.num_nodes = (uint32_t)bvh.nodes.size();
         st.num_leaves = bvh.num_leaves;
         st.max_depth = bvh.max_depth;
@@ -519,7 +511,7 @@ dl_status dl_hip_build_accel(void* h, int builder, dl_accel_stats* stats) {
     }
     {
         const auto t0 = std::chrono::steady_clock::now();
-        DL_TRY(collapse_bvh4(c, st.num_nodes, &st));
+        DL_TRY(collapse_bvh4(c, &st));
         st.build_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
     st.num_prims = c->nprims;
@@ -710,6 +702,7 @@ dl_status dl_hip_scene_keep(void* h, uint64_t key) {
     if (!c->has_accel) return set_error(c, DL_ERR_STATE, "scene_keep before build_accel");
     (void)hipSetDevice(c->device);
     free_scene_union(c);  // members are named by key
+    trim_build(c, true);
     auto it = c->stash.find(key);
     if (it != c->stash.end()) {  // an older scene under the same key is replaced
         free_stashed(c, it->second);

@@ -184,6 +184,11 @@ struct SceneUnion {
     std::vector<void*> allocs;
 };
 
+struct DevBuf {
+    void* p = nullptr;
+    size_t bytes = 0;
+};
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -243,6 +248,10 @@ struct Ctx {
     // dmalloc / dfree): current and peak bytes
     std::unordered_map<void*, size_t> dev_allocs;
     size_t dev_bytes = 0, dev_peak = 0;
+    // build_accel's scratch and the binary nodes it collapses, kept for the
+    // current scene's next build (trim_build)
+    DevBuf build_scratch, build_nodes;
+    uint32_t num_binary = 0;  // nodes in build_nodes
 };
 
 // Tracked device allocation of a context.
@@ -266,6 +275,13 @@ inline hipError_t dfree(Ctx* c, void* p) {
 }
 
 dl_status set_error(Ctx* c, dl_status s, const std::string& msg);
+// Frees the kept buffers of build_accel: all of them, or only if they hold
+// more than kBuildKeepBytes.
+void trim_build(Ctx* c, bool all);
+// Grows b to at least `bytes` (its contents are lost when it grows).
+dl_status grow(Ctx* c, DevBuf& b, size_t bytes);
+// Gives *p (null or a dmalloc'd buffer of the scene) exactly `bytes`.
+dl_status resize_exact(Ctx* c, float4** p, size_t bytes);
 dl_status hip_fail(Ctx* c, hipError_t e, const char* what);
 
 #define DL_HIP_CHECK(ctx, call)                                    \
@@ -321,6 +337,9 @@ void free_scene_union(Ctx* c);
 // bvh_gpu.hip
 dl_status build_bvh_gpu(Ctx* c, dl_accel_stats* stats, int method);
 // Binary nodes of any builder -> the 4-wide nodes the traversal reads.
-dl_status collapse_bvh4(Ctx* c, uint32_t num_binary, dl_accel_stats* stats);
+dl_status collapse_bvh4(Ctx* c, dl_accel_stats* stats);
+// A host-built binary tree to build_nodes and the scene's triangles.
+struct HostBvh;
+dl_status upload_host_bvh(Ctx* c, const HostBvh& bvh);
 
 }  // namespace dl

@@ -30,10 +30,12 @@ namespace dl {
 
 namespace {
 
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // a caller's rows
+
 // Network evaluation on float32 inputs x (n x 96).
 __global__ __launch_bounds__(kGWaves * 64) void k_mlp_forward(Net net, const float* __restrict__ x, uint32_t n,
                                                              float* __restrict__ out) {
-    __shared__ uint16_t s_act[kGWaves][kGRowsPerWave * kGRowStride];
+    __shared__ __align__(16) uint16_t s_act[kGWaves][kGRowsPerWave * kGRowStride];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     uint16_t* s = s_act[wave];
     for (uint32_t tile = blockIdx.x * kGWaves + wave; (size_t)tile * kGRowsPerWave < n; tile += gridDim.x * kGWaves) {
@@ -44,8 +46,9 @@ __global__ __launch_bounds__(kGWaves * 64) void k_mlp_forward(Net net, const flo
             for (int j = 0; j < 8; j++) f[j] = row < n ? x[(size_t)row * kGIn + q * 8 + j] : 0.0f;
             *reinterpret_cast<bf16x8*>(s + lane * kGRowStride + q * 8) = pack8(f);
         }
-        forward_rows(net, s, [&](int r, int c, float v) {
-            if (row0 + r < n) out[(size_t)(row0 + r) * kGOut + c] = v;
+        forward_rows(net, s, [&](int r, int c, float4 v) {
+            if (row0 + r < n)
+                *reinterpret_cast<f32x4_any*>(out + (size_t)(row0 + r) * kGOut + c) = f32x4_any{v.x, v.y, v.z, v.w};
         });
     }
 }
@@ -112,25 +115,13 @@ static_assert(kTrainOutStride * 4 <= kGRowStride * 2, "outputs overlay the opera
 constexpr int train_col(int l) { return l == 0 ? 0 : kGIn + (l - 1) * kGHid; }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // a caller's rows
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
     // lane l holds A[l%16][(l/16)*8 + 0..7] and B[(l/16)*8 + 0..7][l%16];
     // register r of the result is D[4*(l/16) + r][l%16]
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
                                                    0, 0, 0);
 }
-// Two float32 to bfloat16, rounded to nearest even, a in the low half.
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-    const f32x2_t v = {a, b};
-    const bf16x2_t r = __builtin_convertvector(v, bf16x2_t);
-    return __builtin_bit_cast(uint32_t, r);
-}
-// Orders a wave's own LDS accesses, which are of several types.
-__device__ __forceinline__ void lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
-
 // Sums over the 16 rows of a wave (lanes of equal quad) of each of a lane's 16
 // values: lane rl returns the sum of value rl (v[rl / 4][rl % 4]).  Four
 // exchange steps, each halving the values: lanes l and l ^ 8, l ^ 7, l ^ 2,

@@ -1186,9 +1186,9 @@ __global__ __launch_bounds__(kStageBlock) void k_finish(PassParams pp, SceneView
 // the network on the matrix cores (64 points per wave), decoded mixtures
 // written per queue entry.
 template <int TYPE>
-__global__ __launch_bounds__(kGWaves * 64) void k_guide_infer(PassParams pp, SceneView s, RenderBufs rs, int cur,
+__global__ __launch_bounds__(kGWaves * 64, 3) void k_guide_infer(PassParams pp, SceneView s, RenderBufs rs, int cur,
                                                               GuideView gv, Net net) {
-    __shared__ uint16_t s_act[kGWaves][kGRowsPerWave * kGRowStride];
+    __shared__ __align__(16) uint16_t s_act[kGWaves][kGRowsPerWave * kGRowStride];
     const uint32_t n = rs.cnt->mat[cur][TYPE];
     const uint32_t* __restrict__ queue = rs.matq[cur] + (size_t)TYPE * pp.cap;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -1220,15 +1220,21 @@ __global__ __launch_bounds__(kGWaves * 64) void k_guide_infer(PassParams pp, Sce
         // raw outputs overwrite the activation rows of their own 32-row block
         // after that block's last MFMA (byte ranges checked: 192 B per output
         // row vs 208 B per activation row)
-        forward_rows(net, sm, [&](int r, int c, float v) { smf[r * kGOut + c] = v; });
+        forward_rows(net, sm, [&](int r, int c, float4 v) { *reinterpret_cast<float4*>(smf + r * kGOut + c) = v; });
         if (i < n) {
             float o[kGOut], mix[kGMix];
-            for (int j = 0; j < kGOut; j++) o[j] = smf[lane * kGOut + j];
+            for (int j = 0; j < kGOut; j += 4) {
+                const float4 v = *reinterpret_cast<const float4*>(smf + lane * kGOut + j);
+                o[j] = v.x;
+                o[j + 1] = v.y;
+                o[j + 2] = v.z;
+                o[j + 3] = v.w;
+            }
             guide_decode(o, mix);
             float4* dst = reinterpret_cast<float4*>(rs.gmix + (size_t)i * kGMix);
             for (int j = 0; j < kGMix / 4; j++) dst[j] = make_float4(mix[4 * j], mix[4 * j + 1], mix[4 * j + 2], mix[4 * j + 3]);
         }
-        __builtin_amdgcn_wave_barrier();  // the next tile overwrites these LDS rows
+        lds_order();  // the next tile overwrites these LDS rows
     }
 }
 

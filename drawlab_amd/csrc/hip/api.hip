@@ -66,7 +66,6 @@ void swap_scene(Ctx* c, SceneState& s) {
 
 void free_scene(Ctx* c) {
     free_scene_union(c);
-    trim_build(c, true);
     if (c->stream) hipStreamSynchronize(c->stream);
     // the acceleration structure is allocated by the builders, outside
     // scene_allocs
@@ -110,7 +109,6 @@ dl_status check_camera(Ctx* c, const dl_camera_desc& cam) {
 // under its key when it has one, freed otherwise.
 void release_current(Ctx* c) {
     invalidate_film(c);
-    trim_build(c, true);
     if (c->scene_key != 0 && c->has_scene) {
         SceneState s;
         swap_scene(c, s);
@@ -122,6 +120,7 @@ void release_current(Ctx* c) {
 }
 
 void free_all_scenes(Ctx* c) {
+    trim_build(c, true);
     free_scene(c);
     for (auto& kv : c->stash) free_stashed(c, kv.second);
     c->stash.clear();

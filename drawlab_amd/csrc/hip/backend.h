@@ -249,7 +249,7 @@ struct Ctx {
     std::unordered_map<void*, size_t> dev_allocs;
     size_t dev_bytes = 0, dev_peak = 0;
     // build_accel's scratch and the binary nodes it collapses, kept for the
-    // current scene's next build (trim_build)
+    // context's next build (trim_build)
     DevBuf build_scratch, build_nodes;
     uint32_t num_binary = 0;  // nodes in build_nodes
 };

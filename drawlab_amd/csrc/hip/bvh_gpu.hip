@@ -387,8 +387,9 @@ struct Scratch {
 }  // namespace
 
 // Kept by a context between builds at most: the scratch and binary nodes of
-// 3.5 million triangles.  They are given back when the scene is replaced, put
-// aside or freed.
+// 3.5 million triangles.  They serve the builds of the scenes that replace each
+// other on the context, and are given back when a scene is put aside
+// (dl_hip_scene_keep), with dl_hip_trim and with the context.
 constexpr size_t kBuildKeepBytes = 1ull << 30;
 
 void trim_build(Ctx* c, bool all) {

@@ -89,14 +89,18 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_trace_queue_%s_traffic.json" % 
 
 
 def traffic_from_profiles():
-    """HBM bytes per closest-hit traversal launch of this workload, measured
-    by two rocprofv3 PMC runs (FETCH_SIZE, WRITE_SIZE) scaled by a copy
-    kernel of known size; None when the summary is absent."""
+    """(HBM bytes, milliseconds) per launch of the closest-hit traversal
+    kernel of this workload, measured by two rocprofv3 PMC runs (FETCH_SIZE,
+    WRITE_SIZE) scaled by a copy kernel of known size; (None, None) when the
+    summary is absent.  Only the bounces of many paths are launches of this
+    kernel (the others share a launch with the shadow queries), so both are
+    larger than the run's averages per closest-hit launch."""
     try:
         with open(TRAFFIC_FILE) as f:
-            return float(json.load(f)["hbm_bytes_per_launch"])
+            d = json.load(f)
+            return float(d["hbm_bytes_per_launch"]), d["ms_per_launch"]
     except (OSError, KeyError, ValueError):
-        return None
+        return None, None
 
 
 def host_cpus():
@@ -198,7 +202,7 @@ def limiter_from_profiles(kernel, traffic, ms_per_launch):
     c = counters_from_profiles(kernel)
     if c is None:
         return None
-    actual = traffic / (ms_per_launch * 1e-3) / 1e9 if traffic else None
+    actual = traffic / (ms_per_launch * 1e-3) / 1e9 if traffic and ms_per_launch else None
     if actual is not None and actual > 0.8 * HBM_PEAK_GBS:
         what = "HBM bandwidth"
     elif c["valu_busy_pct"] >= 50:
@@ -244,6 +248,13 @@ def _pmc_means(d, counter):
     return {k: (sum(v) / len(v), len(v)) for k, v in acc.items()}
 
 
+def _pmc_ms(d, kernel):
+    path = sorted(glob.glob(os.path.join(d, "**", "*counter_collection.csv"), recursive=True))[0]
+    t = {r["Dispatch_Id"]: (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) * 1e-6
+         for r in csv.DictReader(open(path)) if short_name(r["Kernel_Name"]) == kernel and "Dispatch_Id" in r}
+    return sum(t.values()) / len(t) if t else None
+
+
 def summarize_pmc(fetch_dir, write_dir, out_json, copy_bytes, commands):
     f = _pmc_means(fetch_dir, "FETCH_SIZE")
     w = _pmc_means(write_dir, "WRITE_SIZE")
@@ -263,6 +274,7 @@ def summarize_pmc(fetch_dir, write_dir, out_json, copy_bytes, commands):
         "fetch_scale": cf,
         "write_scale": cw,
         "hbm_bytes_per_launch": fetch + write,
+        "ms_per_launch": _pmc_ms(fetch_dir, TRACE_KERNEL),
         "commands": commands,
         "other_kernels_fetch_kib": {k: v[0] for k, v in f.items()},
         "other_kernels_write_kib": {k: v[0] for k, v in w.items()},
@@ -935,7 +947,7 @@ def main():
     achieved = bytes_per_launch / (ms_per_launch * 1e-3) / 1e9
     # counter profiles exist for the headline workload only
     headline = args.scene == "displaced_sphere"
-    traffic = traffic_from_profiles() if headline else None
+    traffic, traffic_ms = traffic_from_profiles() if headline else (None, None)
     sh_launches = max(1.0, agg["launches_shadow"])
     sh_bytes_per_launch = agg["shadow_rays"] * bytes_per_shadow / sh_launches
     sh_ms_per_launch = agg["ms_shadow"] / sh_launches
@@ -999,13 +1011,16 @@ def main():
                             "frac": round(value / (HBM_PEAK_GBS * 1e3 / bpath["total"]), 4)},
         "roofline": {
             "bound": "hbm",
-            "limiter": limiter_from_profiles(TRACE_KERNEL, traffic, ms_per_launch) if headline else None,
+            "limiter": limiter_from_profiles(TRACE_KERNEL, traffic, traffic_ms) if headline else None,
             "kernel": TRACE_KERNEL + " (closest hit)",
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": traffic,
+            "traffic_launch_ms": traffic_ms,
+            # every node and triangle a ray reads, wherever from: above the
+            # peak the caches supply the difference to `traffic`
             "algorithmic_bytes_per_launch": round(bytes_per_launch),
             "bytes_per_ray": round(bytes_per_ray, 1),
             "node_visits_per_ray": round(nodes_per_ray, 2),

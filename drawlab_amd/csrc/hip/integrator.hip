@@ -77,7 +77,7 @@ struct RenderBufs {
     uint32_t* rayq;
     uint32_t* shq;
     Counters* cnt;
-    uint32_t* work;  // work counters of the closest-hit, then of the shadow traversal (trace.h)
+    uint32_t* work;  // work counters of the closest-hit, then of the shadow traversal (trace.h), and count_sums
     float4* film;
     float* rgb;
     float* gmix;  // guided rendering: mixture (40 floats) per entry of the queue being shaded
@@ -202,9 +202,33 @@ __global__ __launch_bounds__(kStageBlock) void k_reset(Counters* cnt, uint32_t* 
     if (t < 2 * (int)kWorkGroups) work[t * kWorkStride] = 0;
 }
 
-__global__ __launch_bounds__(kStageBlock) void k_reset_all(Counters* cnt) {
+__global__ __launch_bounds__(kStageBlock) void k_reset_all(Counters* cnt, uint32_t* work) {
     uint32_t* w = reinterpret_cast<uint32_t*>(cnt);
     for (uint32_t i = threadIdx.x; i < sizeof(Counters) / 4; i += blockDim.x) w[i] = 0;
+    for (uint32_t i = threadIdx.x; i < 2 * kWorkGroups * kWorkStride; i += blockDim.x) work[i] = 0;
+}
+
+// Node visits and triangle tests of a counting render, summed per line of
+// work counters (line l: closest-hit groups, then shadow groups) in words the
+// claims and k_reset leave alone.  All on one line, the two atomics of every
+// wave of every launch took longer than the traversal: a counting render of
+// the 640x480x4 Cornell box 3.66 ms, now 1.78 (plain: 1.43).
+__device__ __forceinline__ unsigned long long* count_sums(uint32_t* work, uint32_t l) {
+    return reinterpret_cast<unsigned long long*>(work + l * kWorkStride + 8);
+}
+__global__ __launch_bounds__(64) void k_sum_counts(Counters* cnt, uint32_t* work) {
+    static_assert(kWorkGroups == 64, "one line per lane");
+    unsigned long long v[4];
+    for (int q = 0; q < 4; q++) {
+        v[q] = count_sums(work, (q >> 1) * kWorkGroups + threadIdx.x)[q & 1];
+        for (int off = 32; off > 0; off >>= 1) v[q] += __shfl_xor(v[q], off);
+    }
+    if (threadIdx.x == 0) {
+        cnt->nodes = v[0];
+        cnt->tris = v[1];
+        cnt->nodes_sh = v[2];
+        cnt->tris_sh = v[3];
+    }
 }
 
 __global__ __launch_bounds__(kStageBlock) void k_clear_film(float4* film, uint32_t n) {
@@ -344,8 +368,9 @@ __global__ __launch_bounds__(kTraceBlock, COUNT ? 4 : 8) void k_trace_queue(BvhV
     TraceCounters cnt;
     traverse_persistent<false, COUNT>(bvh, trace_work(rs.work, n, grid_wave(), grid_waves()), stk, io, cnt);
     if (COUNT) {
-        wave_add(&rs.cnt->nodes, cnt.nodes);
-        wave_add(&rs.cnt->tris, cnt.tris);
+        unsigned long long* sums = count_sums(rs.work, blockIdx.x % kWorkGroups);
+        wave_add(sums, cnt.nodes);
+        wave_add(sums + 1, cnt.tris);
     }
 }
 
@@ -359,8 +384,9 @@ __global__ __launch_bounds__(kTraceBlock, COUNT ? 4 : 8) void k_shadow_queue(Bvh
     TraceCounters cnt;
     traverse_persistent<true, COUNT>(bvh, trace_work(rs.work + kWorkGroups * kWorkStride, n, grid_wave(), grid_waves()), stk, io, cnt);
     if (COUNT) {
-        wave_add(&rs.cnt->nodes_sh, cnt.nodes);
-        wave_add(&rs.cnt->tris_sh, cnt.tris);
+        unsigned long long* sums = count_sums(rs.work, kWorkGroups + blockIdx.x % kWorkGroups);
+        wave_add(sums, cnt.nodes);
+        wave_add(sums + 1, cnt.tris);
     }
 }
 
@@ -1818,7 +1844,7 @@ dl_status render(Ctx* c, const dl_render_params* prm, float* rgb_host, dl_render
     double closest = 0, shadow = 0, paths = 0;
 
     DL_HIP_CHECK(c, hipEventRecord(c->ev0, c->stream));
-    k_reset_all<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt);
+    k_reset_all<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, rs->b.work);
     if (!(prm->flags & DL_RENDER_ACCUMULATE) || !rs->film_valid)
         k_clear_film<<<stage_grid, kStageBlock, 0, c->stream>>>(rs->b.film, WH);
     rs->film_valid = paths_sample < 0;
@@ -1875,6 +1901,7 @@ dl_status render(Ctx* c, const dl_render_params* prm, float* rgb_host, dl_render
         DL_TRY(tm.stop());
         done += kk;
     }
+    if (count) k_sum_counts<<<1, 64, 0, c->stream>>>(rs->b.cnt, rs->b.work);
     if (paths_sample < 0 && rgb_host) k_resolve<<<stage_grid, kStageBlock, 0, c->stream>>>(rs->b.film, rs->b.rgb, WH);
     DL_HIP_CHECK(c, hipGetLastError());
     DL_HIP_CHECK(c, hipEventRecord(c->ev1, c->stream));
@@ -2044,7 +2071,7 @@ dl_status render_batch(Ctx* c, const dl_render_params* prm, const dl_batch_item*
     std::vector<PassParams> ipp(n);
     std::vector<uint32_t> base(n);
     DL_HIP_CHECK(c, hipEventRecord(c->ev0, c->stream));
-    k_reset_all<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt);
+    k_reset_all<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, rs->b.work);
     k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, rs->b.work, 0);
     k_reset<<<1, kStageBlock, 0, c->stream>>>(rs->b.cnt, rs->b.work, 1);
     DL_TRY(tm.start(kTagOther));
@@ -2085,6 +2112,7 @@ dl_status render_batch(Ctx* c, const dl_render_params* prm, const dl_batch_item*
                                                                   c->film_slots[it.film].rgb, q.W * q.H);
     }
     DL_TRY(tm.stop());
+    if (count) k_sum_counts<<<1, 64, 0, c->stream>>>(rs->b.cnt, rs->b.work);
     DL_HIP_CHECK(c, hipGetLastError());
     DL_HIP_CHECK(c, hipEventRecord(c->ev1, c->stream));
     DL_HIP_CHECK(c, hipEventSynchronize(c->ev1));

@@ -68,3 +68,21 @@ def test_paths_finished_in_one_launch_equal_the_bounce_by_bounce_ones(backend, n
             img, st = backend.render(spp=spp, seed=3, max_depth=depth, rr_depth=rr, spp_per_pass=per_pass)
             assert np.array_equal(img.view(np.uint32), ref.view(np.uint32)), (depth, rr, per_pass)
             assert st["closest_rays"] == rs["closest_rays"] and st["shadow_rays"] == rs["shadow_rays"]
+
+
+def test_traversal_counts_add_up_over_passes_and_images(backend):
+    """Node visits and triangle tests are summed per block group and over the
+    passes of a render: the sums of two renders of half the samples, and of a
+    shared pass of the same samples (whole numbers, exact)."""
+    keys = ("closest_rays", "shadow_rays", "nodes_closest", "tris_closest", "nodes_shadow", "tris_shadow")
+    d = scenes.material_zoo(96, 72)
+    backend.upload_scene(d)
+    backend.build_accel(drawlab_amd.BUILD_GPU)
+    _, whole = backend.render(spp=4, seed=2, count_traversal=True)
+    _, passes = backend.render(spp=4, seed=2, count_traversal=True, spp_per_pass=1)
+    halves = [backend.render(spp=2, seed=2, first_sample=k, count_traversal=True)[1] for k in (0, 2)]
+    _, shared = backend.render_batch([{"camera": d.camera, "spp": 2, "seed": 2, "first_sample": k, "film": k}
+                                      for k in (0, 2)], count_traversal=True)
+    for k in keys:
+        assert whole[k] > 0
+        assert whole[k] == passes[k] == halves[0][k] + halves[1][k] == shared[k], k

@@ -213,7 +213,7 @@ dl_status dl_hip_create(int device, void** out) {
     c->trace_grid = cus * (uint32_t)std::min(render_trace_blocks_per_cu(false), batch_trace_blocks_per_cu(false));
     c->trace_grid_count = cus * (uint32_t)std::min(render_trace_blocks_per_cu(true), batch_trace_blocks_per_cu(true));
     e = dmalloc(c, (void**)&c->stack_ovf, sizeof(int) * (size_t)c->trace_blocks * kTraceBlockHost * (kMaxStack - kLdsStack));
-    if (e == hipSuccess) e = dmalloc(c, (void**)&c->work, kWorkGroupsHost * kWorkStride * sizeof(uint32_t));
+    if (e == hipSuccess) e = dmalloc(c, (void**)&c->work, kWorkGroups * kWorkStride * sizeof(uint32_t));
     if (e != hipSuccess) {
         dl_hip_destroy(c);
         return DL_ERR_OOM;

@@ -9,15 +9,15 @@
 #include <vector>
 
 #include "../../../include/dl_hip.h"
+#include "../work_split.h"
 #include "../bvh_layout.h"
 
 namespace dl {
 
 constexpr int kTraceBlockHost = 128;  // threads per traversal block (trace.h kTraceBlock)
 constexpr int kTraceBlocksPerCu = 16;  // at most: 8 waves per SIMD
-// Work counters of a persistent traversal (trace.h): one per group of blocks,
+// Work counters of a persistent traversal (kWorkGroups of them, work_split.h):
 // each in a 128-byte line of its own.
-constexpr uint32_t kWorkGroupsHost = 64;
 constexpr uint32_t kWorkStride = 32;  // uint32 words
 
 // Device copy of the scene in the layouts the kernels read.  All arrays are

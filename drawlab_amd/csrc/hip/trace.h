@@ -14,6 +14,7 @@
 // accepted triangle (src/tracer/accel/octree.cpp:112-133).
 #pragma once
 #include "../bvh_layout.h"
+#include "../work_split.h"
 #include "backend.h"
 #include "dl_math.h"
 
@@ -151,43 +152,22 @@ __device__ __forceinline__ void wave_add(unsigned long long* dst, uint32_t v) {
 // 4 : 5 measure within 0.5% of it).
 constexpr uint32_t kTriCost = 2, kNodeCost = 5;
 
-// How a persistent grid's waves share n work slots: slots [0, base) are
-// spread evenly over them, the others handed out in chunks of `unit` slots.
-// The chunks are dealt in turn to kWorkGroups groups of blocks, and a wave
-// claims its group's next chunk with one atomic on the group's counter (zero
-// at launch).  One counter for all waves would serialise: its atomics pass at
-// about 55 per microsecond (measured), so the 8192 waves of a full grid
-// claiming once each would already take 150 us.  The blocks of a group run on
-// one XCD (block b runs on XCD b mod 8), whose L2 holds their counter.
-constexpr uint32_t kWorkGroups = kWorkGroupsHost;
-struct TraceWork {
+// How a persistent grid's waves share n work slots (work_split.h): slots
+// [0, base) are spread evenly over them, the others handed out in chunks of
+// `unit` slots.  The chunks are dealt in turn to kWorkGroups groups of blocks
+// (one per block in a smaller grid), and a wave claims its group's next chunk
+// with one atomic on the group's counter (zero at launch).  One counter for
+// all waves would serialise: its atomics pass at about 55 per microsecond
+// (measured), so the 8192 waves of a full grid claiming once each would
+// already take 150 us.  The blocks of a group run on one XCD (block b runs on
+// XCD b mod 8), whose L2 holds their counter.
+struct TraceWork : WorkSplit {
     uint32_t* counter;  // of this wave's group
-    uint32_t n;         // slots in all
-    uint32_t first;     // this wave's first slots: [first, first + count)
-    uint32_t count;
-    uint32_t base;
-    uint32_t unit;
-    uint32_t group;
 };
-// wave / waves: this wave's index among those that start with slots of their
-// own, and their number; a wave beyond them only claims.
 __device__ __forceinline__ TraceWork trace_work(uint32_t* counters, uint32_t n, uint32_t wave, uint32_t waves) {
-    // (n is at most 2^31 and a grid has at most 2^13 waves)
-    const uint32_t share = (n + waves - 1) / waves;
-    // Few slots: a few lanes of every wave rather than all lanes of some, as
-    // a wave takes as long as the slowest of its lanes.  From 16 per wave on
-    // half of them, at most 64, are given out at once, the rest in chunks of
-    // a quarter of a wave's share, 8 to 64 slots, so the waves end together
-    // (1M shadow rays take 231 us, with a sixteenth 242 us).
-    const uint32_t per = share < 16u ? share : min(64u, share / 2u);
     TraceWork w;
-    w.group = blockIdx.x % kWorkGroups;
+    static_cast<WorkSplit&>(w) = split_work(n, wave, waves, blockIdx.x, gridDim.x);
     w.counter = counters + w.group * kWorkStride;
-    w.n = n;
-    w.base = min(n, per * waves);
-    w.first = min(min(wave, waves) * per, w.base);
-    w.count = wave < waves ? min(per, w.base - w.first) : 0u;
-    w.unit = share >= 256u ? 64u : share >= 128u ? 32u : share >= 64u ? 16u : 8u;
     return w;
 }
 
@@ -408,8 +388,7 @@ __device__ __forceinline__ void traverse_persistent(const BvhView& bvh, const Tr
     TraceCounters cnt;
     for (;;) {
         if (pos == len && more) {
-            const uint32_t chunk = (uint32_t)__builtin_amdgcn_readfirstlane((int)claim) * kWorkGroups + work.group;
-            const uint32_t b = work.base + chunk * work.unit;
+            const uint32_t b = chunk_start(work, (uint32_t)__builtin_amdgcn_readfirstlane((int)claim));
             if (b < n) {
                 pos = 0;
                 len = min(work.unit, n - b);

@@ -102,10 +102,9 @@ uint32_t batch_blocks(uint32_t grid, uint32_t n) {
 }
 
 // Whether trace_work leaves rays to claim, so that the counters have to be
-// cleared first: from 16 rays per wave on.
+// cleared first.
 bool claims_work(uint32_t blocks, uint32_t n) {
-    const uint32_t waves = blocks * (uint32_t)(kTraceBlock / 64);
-    return (n + waves - 1) / waves >= 16u;
+    return wave_share(n, blocks * (uint32_t)(kTraceBlock / 64)) >= kClaimShare;
 }
 
 dl_status launch_trace_closest(Ctx* c, const float* rays, uint32_t n, uint32_t* prim, float* t, float* u, float* v,

@@ -106,6 +106,7 @@ __global__ __launch_bounds__(256) void k_sum(const float* __restrict__ c, uint32
 // reduction and dAct per layer, 700 bytes of activations and gradients per row
 // through memory) and takes 208 us as three.
 constexpr int kTrainWaves = 4, kTrainRows = 16 * kTrainWaves;
+static_assert(kTrainRows == (int)dl_sizes::kGuideTrainRows, "rows of a training tile");
 constexpr int kTrainStride = kTrainRows + 8;         // bf16 per transposed column
 constexpr int kTrainCols = kGIn + 4 * kGHid;         // the inputs of the five layers
 constexpr int kTrainOutStride = kGOut + 1;           // float32 outputs of a row
@@ -788,8 +789,7 @@ dl_status guide_forward(Ctx* c, const float* x, uint32_t n, float* out) {
 dl_status guide_train(Ctx* c, const float* x, const float* dirs, const float* cw, uint32_t n, bool apply) {
     GuideState* g = (GuideState*)c->guide;
     if (!g->part) DL_TRY(galloc(c, g, &g->part, (size_t)dl_sizes::kGuideTrainBlocks * kGParams));
-    const uint32_t blocks = std::min<uint32_t>((uint32_t)std::min(std::max(1, 2 * c->num_cus), (int)dl_sizes::kGuideTrainBlocks),
-                                               (n + kTrainRows - 1) / kTrainRows);
+    const uint32_t blocks = dl_sizes::guide_train_blocks(n);
     float* const sums = g->scalars + 4;
     float* const losses = sums + kSumBlocks;
     k_sum<<<kSumBlocks, 256, 0, c->stream>>>(cw, n, sums);

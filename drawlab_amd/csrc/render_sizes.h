@@ -25,7 +25,16 @@ constexpr int kGuideMixFloats = 40;          // decoded mixture per queued shadi
 constexpr int kGuideRecordFloats = 24;       // training record
 constexpr uint32_t kGuideRecordSlots = 1u << 23;
 constexpr uint32_t kGuideBatchRows = 1u << 18;  // records per Adam step
+constexpr uint32_t kGuideTrainRows = 64;        // rows of a training tile
 constexpr uint32_t kGuideTrainBlocks = 512;     // blocks of a training step (at most), a partial gradient each
+// Blocks of a training step on n rows: a tile each until there are
+// kGuideTrainBlocks, two for each of the MI355X's 256 CUs.  They depend on the
+// rows alone, not on the device's CUs: the blocks' shares of the rows are the
+// order of the gradient's sums, so a trained network is the same everywhere.
+constexpr uint32_t guide_train_blocks(uint32_t n) {
+    const uint32_t tiles = n / kGuideTrainRows + (n % kGuideTrainRows != 0 ? 1 : 0);
+    return tiles < kGuideTrainBlocks ? tiles : kGuideTrainBlocks;
+}
 constexpr uint32_t kGuideSumBlocks = 64;        // partial sums of the training weights
 constexpr uint32_t kGuideScanTile = 1024;       // records per prefix-sum tile
 constexpr int kGuideParams = 21808;

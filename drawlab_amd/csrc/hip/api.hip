@@ -480,10 +480,14 @@ dl_status dl_hip_build_accel(void* h, int builder, dl_accel_stats* stats) {
     // fits: nothing on any stream may be reading them
     DL_HIP_CHECK(c, hipDeviceSynchronize());
     c->has_accel = false;
-    struct Trim {
+    struct Building {
         Ctx* c;
-        ~Trim() { trim_build(c, false); }
-    } trim{c};
+        explicit Building(Ctx* ctx) : c(ctx) { c->building = true; }
+        ~Building() {
+            c->building = false;
+            trim_build(c, false);
+        }
+    } building(c);
     bool host = builder == DL_BUILD_HOST_SAH;
     if (!host) {
         c->bvh_too_deep = false;

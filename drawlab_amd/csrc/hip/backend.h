@@ -251,12 +251,23 @@ struct Ctx {
     // build_accel's scratch and the binary nodes it collapses, kept for the
     // context's next build (trim_build)
     DevBuf build_scratch, build_nodes;
+    bool building = false;  // a build is using them
     uint32_t num_binary = 0;  // nodes in build_nodes
 };
 
-// Tracked device allocation of a context.
+// Frees the kept buffers of build_accel: all of them, or only if they hold
+// more than kBuildKeepBytes.
+void trim_build(Ctx* c, bool all);
+
+// Tracked device allocation of a context.  What a finished build left for the
+// next one is given back before an allocation is refused.
 inline hipError_t dmalloc(Ctx* c, void** p, size_t bytes) {
-    const hipError_t e = hipMalloc(p, bytes);
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && !c->building && (c->build_scratch.p || c->build_nodes.p)) {
+        (void)hipGetLastError();
+        trim_build(c, true);
+        e = hipMalloc(p, bytes);
+    }
     if (e == hipSuccess) {
         c->dev_allocs[*p] = bytes;
         c->dev_bytes += bytes;
@@ -275,9 +286,6 @@ inline hipError_t dfree(Ctx* c, void* p) {
 }
 
 dl_status set_error(Ctx* c, dl_status s, const std::string& msg);
-// Frees the kept buffers of build_accel: all of them, or only if they hold
-// more than kBuildKeepBytes.
-void trim_build(Ctx* c, bool all);
 // Grows b to at least `bytes` (its contents are lost when it grows).
 dl_status grow(Ctx* c, DevBuf& b, size_t bytes);
 // Gives *p (null or a dmalloc'd buffer of the scene) exactly `bytes`.

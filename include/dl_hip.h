@@ -241,6 +241,11 @@ const char* dl_hip_device_name(void* ctx);
 
 /* ---- scene and acceleration structure ---------------------------------- */
 dl_status dl_hip_upload_scene(void* ctx, const dl_scene_desc* scene);
+/* Builds the current scene's acceleration structure (again, if it has one).
+ * The build's scratch memory, about 284 bytes per triangle, stays with the
+ * context for its next build if it is at most 1 GiB (it counts in
+ * dl_hip_memory_usage); dl_hip_scene_keep, dl_hip_trim and any allocation of
+ * the context that would not fit beside it give it back. */
 dl_status dl_hip_build_accel(void* ctx, int builder, dl_accel_stats* stats);
 
 /* ---- traversal on device-resident batches ------------------------------

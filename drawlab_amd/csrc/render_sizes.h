@@ -52,16 +52,11 @@ constexpr uint64_t kGuideTrainBytes =
 constexpr uint64_t kGuideResampleBytes =
     (uint64_t)kGuideRecordSlots * 4 + 2ull * (kGuideRecordSlots / kGuideScanTile + 1) * 4;
 
-// Headroom of a guided job's reservation, which stays more than 1 GiB above a
-// plain job's as budgets expect (a step's activations and gradients, 0.39 GB,
-// are no longer kept in memory).
-constexpr uint64_t kGuideHeadroomBytes = 128ull << 20;
-
 // Everything a guided render adds to a plain one whose passes hold `paths`
 // paths.
 constexpr uint64_t guide_bytes(uint64_t paths) {
     return paths * kGuideMixFloats * 4 + (uint64_t)kGuideRecordSlots * kGuideRecordFloats * 4 + kGuideNetBytes +
-           kGuideTrainBytes + kGuideResampleBytes + kGuideHeadroomBytes;
+           kGuideTrainBytes + kGuideResampleBytes;
 }
 
 }  // namespace dl_sizes

@@ -269,4 +269,8 @@ def test_guided_job_within_its_reservation():
     assert ig["state"] == drawlab_amd.JOB_DONE and ip["state"] == drawlab_amd.JOB_DONE
     assert ig["peak_bytes"] <= ig["reserved_bytes"] and ip["peak_bytes"] <= ip["reserved_bytes"]
     assert st["estimate_misses"] == 0
-    assert ig["reserved_bytes"] > ip["reserved_bytes"] + (1 << 30)  # records + training batch
+    # records, training batch, blocks' partial gradients, record weights and
+    # mixtures; the network, its copies and the tiles' sums are less than a MiB
+    adds = (1 << 23) * 96 + (1 << 18) * (96 + 3 + 1) * 4 + 512 * 21808 * 4 + (1 << 23) * 4 + 64 * 64 * 16 * 40 * 4
+    assert adds < ig["reserved_bytes"] - ip["reserved_bytes"] < adds + (1 << 20)
+    assert ig["peak_bytes"] - ip["peak_bytes"] > adds - (1 << 20)

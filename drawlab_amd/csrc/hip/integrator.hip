@@ -990,9 +990,11 @@ constexpr uint32_t kFinishLanes = 32;
 // from the camera: Cornell box 0.65, 0.34, MIS plates 0.60, 0.38, zoo 0.79,
 // 0.75; of 262,144: 0.75, 0.50, 0.70, 0.59, 0.96, 1.07, sphere 1.72, 2.02.
 constexpr uint32_t kFinishPaths = 1u << 18, kFinishCamera = 1u << 17;
-// A path ends after this many bounces in k_finish: Russian roulette leaves
-// 0.99^4096 = 1e-18 of the paths that long, and a throughput of NaN, which
-// roulette never ends, must not keep the kernel running.
+// A path ends after this many bounces in k_finish.  A throughput of NaN, which
+// Russian roulette never ends, must not keep the kernel running; roulette, which
+// sets in by bounce kFinishRoulette where the depth is not capped by it, leaves
+// at most 0.99^3072 = 4e-14 of the paths that long.
+constexpr int kFinishRoulette = 1024;
 constexpr int kFinishBounces = 4096;
 // Bounces of at most this many paths trace both queries in one launch (the
 // 1080p frame takes 5.43, 5.22 and 5.04 ms with 2^20, 2^22 and 2^24, the
@@ -1638,7 +1640,7 @@ dl_status run_bounces(Ctx* c, RenderState* rs, const PassParams& pp, const Scene
     // k_finish follows the plain paths only, and only where their number of
     // bounces is bounded
     const bool finish = !count && !normals && !hide && !guided &&
-                        (pp.rr_depth <= 1024 || (pp.max_depth >= 0 && pp.max_depth <= 1024));
+                        (pp.rr_depth <= kFinishRoulette || (pp.max_depth >= 0 && pp.max_depth <= kFinishRoulette));
     // (its time counts as closest-hit time, which it mostly is)
     auto finish_grid = [&](uint32_t paths) {
         return (int)std::min<uint32_t>((uint32_t)std::max(1, c->num_cus) * 2u, (paths + 15u) / 16u);

@@ -86,3 +86,33 @@ def test_traversal_counts_add_up_over_passes_and_images(backend):
     for k in keys:
         assert whole[k] > 0
         assert whole[k] == passes[k] == halves[0][k] + halves[1][k] == shared[k], k
+
+
+@pytest.mark.parametrize("size", [(8, 8, 1), (75, 64, 2)], ids=lambda s: "%dx%dx%d" % s)
+def test_paths_that_roulette_never_ends_are_cut_off(backend, size):
+    """A throughput of NaN survives every roulette (no comparison with NaN
+    ends it), so in a closed room such paths would go on for good: the launch
+    that carries few paths to their end gives each 4,097 vertices past the
+    camera's ray (bounces 0 to 4,096), and the film drops what they return.
+    A ray gets out of the room of 8 units if it leaves within its offset of
+    1e-4 from an edge (at most 4e-4 / 8 of a wall's area), or if rounding put
+    its origin behind the wall (1e-6) and it leaves at a cosine below 1e-2
+    (1e-4 of the directions): less than 1.5e-4 of the bounces, so the paths
+    average more than (1 - exp(-.61)) / .61 = 0.75 of the 4,097."""
+    W, H, spp = size
+    d = scenes.chimney_room(W, H)
+    for b in d.bsdfs:
+        b.params = (float("nan"),) * 3
+    walls = [m for m in d.meshes if m.name == "wall"]
+    assert len(walls) == 6
+    for m in walls:
+        m.V = np.ascontiguousarray(m.V * np.float32(8.0))
+    cam = dataclasses.replace(d.camera, eye=(4.0, 4.0, 0.16), lookat=(4.0, 2.4, 8.0))
+    d = dataclasses.replace(d, meshes=walls, camera=cam, point_lights=[((4.0, 7.2, 4.0), (1.0, 1.0, 1.0))])
+    backend.upload_scene(d)
+    backend.build_accel(drawlab_amd.BUILD_GPU)
+    img, st = backend.render(spp=spp, seed=1, max_depth=-1, rr_depth=4)
+    paths = W * H * spp
+    print("queries per path", st["closest_rays"] / paths, "invalid", st["invalid_samples"], flush=True)
+    assert 0.5 * 4098 * paths < st["closest_rays"] <= 4098 * paths
+    assert st["invalid_samples"] == paths and not img.any()

@@ -26,8 +26,8 @@ one-at-a-time rendering, and both saturated throughputs (jobs/s).
 `--workload trace`: the traversal micro-bench on the same geometry -- three
 ray sets (2,073,600 primary rays, 2^22 diffuse-bounce rays and 2^22 shadow
 rays toward the sky and sun, both from the points the primary rays hit)
-through the batch traversal kernels, each with its own HBM roofline
-fraction in algorithmic bytes.
+through the batch traversal kernels, each with the bytes its rays touch
+(nodes, triangles, rays and results, wherever the caches serve them from).
 
 `--workload guided`: the learned proposal against plain rendering at equal
 wall time on the same scene at 480x270 -- a 65,536-spp plain reference, then
@@ -84,22 +84,23 @@ PATH_STATE_BYTES = {"raygen": 2 * 16 + 8 + 4 + 8 + 1 + 4,                     # 
                     "film": 8 + 16 + 16 / 64.0,
                     "first_vertex_skip": 16}                                   # per path: an undercount
 TRACE_KERNEL = "k_trace_queue<false>"
+SHADOW_KERNEL = "k_shadow_queue<false>"
 COPY_KERNEL = "k_copy"
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_trace_queue_%s_traffic.json" % WORKLOAD)
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "bench_%s_traffic.json" % WORKLOAD)
 
 
-def traffic_from_profiles():
-    """(HBM bytes, milliseconds) per launch of the closest-hit traversal
-    kernel of this workload, measured by two rocprofv3 PMC runs (FETCH_SIZE,
-    WRITE_SIZE) scaled by a copy kernel of known size; (None, None) when the
-    summary is absent.  Only the bounces of many paths are launches of this
-    kernel (the others share a launch with the shadow queries), so both are
-    larger than the run's averages per closest-hit launch."""
+def traffic_from_profiles(kernel):
+    """(bytes beyond L2, milliseconds) per launch of `kernel` in this
+    workload, measured by two rocprofv3 PMC runs (read requests of each size,
+    WRITE_SIZE); (None, None) when the summary is absent.  Only the bounces of
+    many paths are launches of the traversal kernels (the others share one
+    launch for both queries), so both are larger than the run's averages per
+    closest-hit launch."""
     try:
         with open(TRAFFIC_FILE) as f:
-            d = json.load(f)
-            return float(d["hbm_bytes_per_launch"]), d["ms_per_launch"]
-    except (OSError, KeyError, ValueError):
+            d = json.load(f)["kernels"][kernel]
+            return float(d["fetch_bytes"] + d["write_bytes"]), d["ms"]
+    except (OSError, KeyError, ValueError, TypeError):
         return None, None
 
 
@@ -151,6 +152,33 @@ def cpu_baseline(desc, target_s, threads):
     }
 
 
+def roofline(kernel, query, traffic, traffic_ms, rays, bytes_per_ray, nodes_per_ray, tris_per_ray, ms, launches,
+             profiled):
+    """`kernel` against the HBM roofline: what its launches move beyond L2 per
+    second, from the profile of the same workload (null without one).  Beside
+    it the run's own queries of this kind, whichever kernel traced them (the
+    bounces of many rays `kernel`, the others a launch of both queries, and the
+    last paths one launch): the bytes of every node, triangle, ray and result
+    they touch, wherever from -- the caches serve most of them, so their rate
+    is no fraction of the HBM peak."""
+    got = rate_gbs(traffic, traffic_ms)
+    return {
+        "bound": "hbm",
+        "limiter": limiter_from_profiles(kernel, traffic, traffic_ms) if profiled else None,
+        "kernel": "%s (%s)" % (kernel, query),
+        "achieved": round(got, 1) if got else None,
+        "peak": HBM_PEAK_GBS,
+        "unit": "GB/s",
+        "frac": round(got / HBM_PEAK_GBS, 4) if got else None,
+        "traffic": traffic,
+        "traffic_launch_ms": traffic_ms,
+        "queries": {"rays": int(rays), "bytes_per_ray": round(bytes_per_ray, 1),
+                    "node_visits_per_ray": round(nodes_per_ray, 2), "tri_tests_per_ray": round(tris_per_ray, 2),
+                    "launches": int(launches), "avg_launch_ms": round(ms / launches, 4),
+                    "touched_gbs": round(rays * bytes_per_ray / (ms * 1e-3) / 1e9, 1) if ms > 0 else None},
+    }
+
+
 def path_bytes(agg, bytes_closest, bytes_shadow):
     """Algorithmic bytes per path: its traversal queries (closest-hit and
     shadow, at their measured bytes per query) plus the path state its
@@ -194,6 +222,10 @@ def counters_from_profiles(kernel):
     return None
 
 
+def rate_gbs(nbytes, ms):
+    return nbytes / (ms * 1e-3) / 1e9 if nbytes and ms else None
+
+
 def limiter_from_profiles(kernel, traffic, ms_per_launch):
     """What limits the kernel below the HBM roofline, from its counters:
     actual HBM traffic near the peak means bandwidth; otherwise a busy VALU
@@ -202,7 +234,7 @@ def limiter_from_profiles(kernel, traffic, ms_per_launch):
     c = counters_from_profiles(kernel)
     if c is None:
         return None
-    actual = traffic / (ms_per_launch * 1e-3) / 1e9 if traffic and ms_per_launch else None
+    actual = rate_gbs(traffic, ms_per_launch)
     if actual is not None and actual > 0.8 * HBM_PEAK_GBS:
         what = "HBM bandwidth"
     elif c["valu_busy_pct"] >= 50:
@@ -248,40 +280,48 @@ def _pmc_means(d, counter):
     return {k: (sum(v) / len(v), len(v)) for k, v in acc.items()}
 
 
-def _pmc_ms(d, kernel):
+def _pmc_ms(d):
     path = sorted(glob.glob(os.path.join(d, "**", "*counter_collection.csv"), recursive=True))[0]
-    t = {r["Dispatch_Id"]: (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) * 1e-6
-         for r in csv.DictReader(open(path)) if short_name(r["Kernel_Name"]) == kernel and "Dispatch_Id" in r}
-    return sum(t.values()) / len(t) if t else None
+    t = {}
+    for r in csv.DictReader(open(path)):
+        t.setdefault(short_name(r["Kernel_Name"]), {})[r.get("Dispatch_Id", len(t))] = (
+            int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) * 1e-6
+    return {k: sum(v.values()) / len(v) for k, v in t.items()}
+
+
+# read requests an XCD's L2 sends, by size in bytes
+FETCH_COUNTERS = {"TCC_EA0_RDREQ_32B_sum": 32, "TCC_EA0_RDREQ_64B_sum": 64, "TCC_EA0_RDREQ_128B_sum": 128}
 
 
 def summarize_pmc(fetch_dir, write_dir, out_json, copy_bytes, commands):
-    f = _pmc_means(fetch_dir, "FETCH_SIZE")
+    """Bytes each kernel's launches move beyond L2 (HBM and the memory-side
+    cache before it), means per launch.  Reads are counted by request size:
+    FETCH_SIZE takes a 128-byte request for 64 bytes, so it reports half of a
+    streaming kernel's reads and a gather's as they are, and no one factor
+    corrects both.  The copy kernel, whose reads and writes are known, shows
+    that the counts are whole (copy_fetch, copy_write: counted over known)."""
+    sizes = [(_pmc_means(fetch_dir, c), b) for c, b in FETCH_COUNTERS.items()]
     w = _pmc_means(write_dir, "WRITE_SIZE")
-    cf = copy_bytes / (f[COPY_KERNEL][0] * 1024.0)
-    cw = copy_bytes / (w[COPY_KERNEL][0] * 1024.0)
-    fetch = f[TRACE_KERNEL][0] * 1024.0 * cf
-    write = w[TRACE_KERNEL][0] * 1024.0 * cw
+    ms = _pmc_ms(fetch_dir)
+    kernels = {}
+    for k, (_, n) in sizes[0][0].items():
+        req = {"%dB" % b: m[k][0] for m, b in sizes}
+        fetch = sum(m[k][0] * b for m, b in sizes)
+        write = w[k][0] * 1024.0 if k in w else 0.0
+        kernels[k] = {"launches": n, "ms": ms[k], "fetch_bytes": fetch, "write_bytes": write,
+                      "gbs": (fetch + write) / (ms[k] * 1e-3) / 1e9 if ms[k] > 0 else None, "read_requests": req}
     out = {
-        "kernel": TRACE_KERNEL,
         "workload": WORKLOAD + " (256 spp per pass)",
-        "dispatches": f[TRACE_KERNEL][1],
-        "fetch_kib_per_dispatch": f[TRACE_KERNEL][0],
-        "write_kib_per_dispatch": w[TRACE_KERNEL][0],
         "copy_kernel_bytes": copy_bytes,
-        "copy_fetch_kib": f[COPY_KERNEL][0],
-        "copy_write_kib": w[COPY_KERNEL][0],
-        "fetch_scale": cf,
-        "write_scale": cw,
-        "hbm_bytes_per_launch": fetch + write,
-        "ms_per_launch": _pmc_ms(fetch_dir, TRACE_KERNEL),
+        "copy_fetch": kernels[COPY_KERNEL]["fetch_bytes"] / copy_bytes,
+        "copy_write": kernels[COPY_KERNEL]["write_bytes"] / copy_bytes,
         "commands": commands,
-        "other_kernels_fetch_kib": {k: v[0] for k, v in f.items()},
-        "other_kernels_write_kib": {k: v[0] for k, v in w.items()},
+        "kernels": dict(sorted(kernels.items(), key=lambda kv: -kv[1]["launches"] * kv[1]["ms"])),
     }
     with open(out_json, "w") as fo:
         json.dump(out, fo, indent=1)
-    print(json.dumps({k: out[k] for k in list(out)[:12]}, indent=1))
+    print(json.dumps({"copy_fetch": out["copy_fetch"], "copy_write": out["copy_write"],
+                      TRACE_KERNEL: kernels.get(TRACE_KERNEL)}, indent=1))
 
 
 def summarize_counters(dirs, out_md, command, kernels):
@@ -786,13 +826,12 @@ def trace_bench(args):
         res[name] = {"rays": n, "kernel": "k_trace_shadow" if any_hit else "k_trace_closest<false>",
                      "ms": round(med, 4), "mrays_per_s": round(n / (med * 1e-3) / 1e6, 1),
                      "node_visits_per_ray": round(nodes, 3), "tri_tests_per_ray": round(tris, 3),
-                     "bytes_per_ray": round(bpr, 1), "achieved_gbs": round(gbs, 1),
-                     "frac": round(gbs / HBM_PEAK_GBS, 4), ("occluded" if any_hit else "hit") + "_fraction":
-                         round(hit_frac, 4)}
+                     "bytes_per_ray": round(bpr, 1), "touched_gbs": round(gbs, 1),
+                     ("occluded" if any_hit else "hit") + "_fraction": round(hit_frac, 4)}
         total_rays += n
         total_ms += med
-        print("%-8s %9d rays  %8.3f ms  %8.1f Mrays/s  %6.1f B/ray  %7.1f GB/s (%.3f of HBM peak)" % (
-            name, n, med, res[name]["mrays_per_s"], bpr, gbs, gbs / HBM_PEAK_GBS), file=sys.stderr, flush=True)
+        print("%-8s %9d rays  %8.3f ms  %8.1f Mrays/s  %6.1f B/ray  %7.1f GB/s touched, caches included" % (
+            name, n, med, res[name]["mrays_per_s"], bpr, gbs), file=sys.stderr, flush=True)
     value = total_rays / (total_ms * 1e-3) / 1e6
     dom = max(res, key=lambda k: res[k]["ms"])
     out = {
@@ -812,9 +851,11 @@ def trace_bench(args):
                    "bvh": "gpu-ploc, quantised 4-wide nodes", "bvh_build_ms": round(accel["build_ms"], 2),
                    "ray_generation_s": round(gen_s, 1)},
         "ray_sets": res,
-        "roofline": {"bound": "hbm", "kernel": res[dom]["kernel"] + " (%s rays)" % dom,
-                     "achieved": res[dom]["achieved_gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": res[dom]["frac"], "traffic": None},
+        # (this workload has no traffic profile, and the bytes its rays touch
+        # come mostly from the caches)
+        "roofline": {"bound": "hbm", "kernel": res[dom]["kernel"] + " (%s rays)" % dom, "achieved": None,
+                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": None, "traffic": None,
+                     "touched_gbs": res[dom]["touched_gbs"]},
         "cpu_baseline": None,
     }
     print(json.dumps(out), flush=True)
@@ -942,16 +983,11 @@ def main():
     paths = agg["paths"]
     value = paths / seconds / 1e6
     launches = max(1.0, agg["launches_closest"])
-    bytes_per_launch = agg["closest_rays"] * bytes_per_ray / launches
-    ms_per_launch = agg["ms_closest"] / launches
-    achieved = bytes_per_launch / (ms_per_launch * 1e-3) / 1e9
     # counter profiles exist for the headline workload only
     headline = args.scene == "displaced_sphere"
-    traffic, traffic_ms = traffic_from_profiles() if headline else (None, None)
+    traffic, traffic_ms = traffic_from_profiles(TRACE_KERNEL) if headline else (None, None)
+    sh_traffic, sh_traffic_ms = traffic_from_profiles(SHADOW_KERNEL) if headline else (None, None)
     sh_launches = max(1.0, agg["launches_shadow"])
-    sh_bytes_per_launch = agg["shadow_rays"] * bytes_per_shadow / sh_launches
-    sh_ms_per_launch = agg["ms_shadow"] / sh_launches
-    sh_achieved = sh_bytes_per_launch / (sh_ms_per_launch * 1e-3) / 1e9
     # rays: average algorithmic bytes per traversal query; paths: per path
     rays = agg["closest_rays"] + agg["shadow_rays"]
     bytes_per_query = (agg["closest_rays"] * bytes_per_ray + agg["shadow_rays"] * bytes_per_shadow) / rays
@@ -1001,48 +1037,20 @@ def main():
             "bvh_build_ms": round(accel["build_ms"], 2),
         },
         "mrays_per_s": round(mrays, 2),
-        # Mrays/s and Mpaths/s against the rates the HBM roofline allows at
-        # the algorithmic bytes of a query and of a path
+        # Mrays/s and Mpaths/s against the rates HBM would allow if every
+        # byte of a query and of a path came from it (caches serve part, so
+        # these may exceed 1)
         "mrays_roofline": {"bytes_per_query": round(bytes_per_query, 1),
                            "roofline_mrays_per_s": round(HBM_PEAK_GBS * 1e3 / bytes_per_query, 1),
                            "frac": round(mrays / (HBM_PEAK_GBS * 1e3 / bytes_per_query), 4)},
         "mpaths_roofline": {"bytes_per_path": round(bpath["total"], 1), "breakdown": bpath,
                             "roofline_mpaths_per_s": round(HBM_PEAK_GBS * 1e3 / bpath["total"], 1),
                             "frac": round(value / (HBM_PEAK_GBS * 1e3 / bpath["total"]), 4)},
-        "roofline": {
-            "bound": "hbm",
-            "limiter": limiter_from_profiles(TRACE_KERNEL, traffic, traffic_ms) if headline else None,
-            "kernel": TRACE_KERNEL + " (closest hit)",
-            "achieved": round(achieved, 1),
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "traffic": traffic,
-            "traffic_launch_ms": traffic_ms,
-            # every node and triangle a ray reads, wherever from: above the
-            # peak the caches supply the difference to `traffic`
-            "algorithmic_bytes_per_launch": round(bytes_per_launch),
-            "bytes_per_ray": round(bytes_per_ray, 1),
-            "node_visits_per_ray": round(nodes_per_ray, 2),
-            "tri_tests_per_ray": round(tris_per_ray, 2),
-            "launches": int(launches),
-            "avg_launch_ms": round(ms_per_launch, 4),
-        },
-        "roofline_shadow": {
-            "bound": "hbm",
-            "limiter": limiter_from_profiles("k_shadow_queue<false>", None, sh_ms_per_launch) if headline else None,
-            "kernel": "k_shadow_queue<false> (any hit)",
-            "achieved": round(sh_achieved, 1),
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": round(sh_achieved / HBM_PEAK_GBS, 4),
-            "algorithmic_bytes_per_launch": round(sh_bytes_per_launch),
-            "bytes_per_ray": round(bytes_per_shadow, 1),
-            "node_visits_per_ray": round(nodes_per_shadow, 2),
-            "tri_tests_per_ray": round(tris_per_shadow, 2),
-            "launches": int(sh_launches),
-            "avg_launch_ms": round(sh_ms_per_launch, 4),
-        },
+        "roofline": roofline(TRACE_KERNEL, "closest hit", traffic, traffic_ms, agg["closest_rays"], bytes_per_ray,
+                             nodes_per_ray, tris_per_ray, agg["ms_closest"], launches, headline),
+        "roofline_shadow": roofline(SHADOW_KERNEL, "any hit", sh_traffic, sh_traffic_ms, agg["shadow_rays"],
+                                    bytes_per_shadow, nodes_per_shadow, tris_per_shadow, agg["ms_shadow"],
+                                    sh_launches, headline),
         "stage_ms": {k: round(agg[k], 1) for k in ("ms_closest", "ms_shadow", "ms_shade", "ms_film", "ms_other")},
         "cpu_baseline": cpu,
     }

@@ -21,32 +21,47 @@ def test_more_than_one_gpu_is_refused_with_a_message():
     assert "single MI355X" in r.stderr and r.stdout == ""
 
 
-def _write_pmc(d, counter, rows):
+def _write_pmc(d, rows):
     os.makedirs(d, exist_ok=True)
     with open(os.path.join(d, "x_counter_collection.csv"), "w", newline="") as f:
-        w = csv.DictWriter(f, fieldnames=["Kernel_Name", "Counter_Name", "Counter_Value", "Start_Timestamp",
-                                          "End_Timestamp"])
+        w = csv.DictWriter(f, fieldnames=["Dispatch_Id", "Kernel_Name", "Counter_Name", "Counter_Value",
+                                          "Start_Timestamp", "End_Timestamp"])
         w.writeheader()
-        for name, value in rows:
-            w.writerow({"Kernel_Name": name, "Counter_Name": counter, "Counter_Value": value,
-                        "Start_Timestamp": 0, "End_Timestamp": 1000})
+        for k, (name, counter, value, ns) in enumerate(rows):
+            w.writerow({"Dispatch_Id": k, "Kernel_Name": name, "Counter_Name": counter, "Counter_Value": value,
+                        "Start_Timestamp": 1000, "End_Timestamp": 1000 + ns})
 
 
-def test_traffic_summary_scales_by_the_copy_kernel(tmp_path):
-    """FETCH_SIZE / WRITE_SIZE are KiB per dispatch; each is scaled by what
-    the plain copy of known size reads or writes, so a copy that reports
-    half its bytes (fetch) doubles the traversal's fetch."""
+def test_traffic_summary_counts_requests_by_size(tmp_path):
+    """Reads are the requests of each size times that size -- a streaming
+    copy's 128-byte requests and a gather's 64-byte ones alike, with no factor
+    of one applied to the other; WRITE_SIZE is KiB per dispatch."""
     copy = 1 << 30
     trace = "void dl::k_trace_queue<false>(dl::BvhView, dl::RenderBufs, int*)"
-    _write_pmc(str(tmp_path / "f"), "FETCH_SIZE", [(trace, 1000.0), (trace, 3000.0), ("k_copy", copy / 2048.0)])
-    _write_pmc(str(tmp_path / "w"), "WRITE_SIZE", [(trace, 500.0), ("k_copy", copy / 1024.0)])
+    rows = []
+    for name, per_dispatch in ((trace, [(10, 300, 40), (30, 100, 80)]), ("k_copy", [(0, 0, copy // 128)])):
+        for ns, r in zip((2_000_000, 4_000_000), per_dispatch):
+            rows += [(name, "TCC_EA0_RDREQ_%dB_sum" % b, v, ns) for b, v in zip((32, 64, 128), r)]
+    _write_pmc(str(tmp_path / "f"), rows)
+    _write_pmc(str(tmp_path / "w"), [(trace, "WRITE_SIZE", 2.0, 1), ("k_copy", "WRITE_SIZE", copy / 1024.0, 1)])
     out = tmp_path / "traffic.json"
     bench.summarize_pmc(str(tmp_path / "f"), str(tmp_path / "w"), str(out), copy_bytes=copy, commands="cmd")
     t = json.loads(out.read_text())
-    assert t["dispatches"] == 2
-    assert t["fetch_scale"] == pytest.approx(2.0) and t["write_scale"] == pytest.approx(1.0)
-    # mean fetch 2000 KiB x 2, write 500 KiB x 1
-    assert t["hbm_bytes_per_launch"] == pytest.approx(2000 * 1024 * 2.0 + 500 * 1024 * 1.0)
+    assert t["copy_fetch"] == 1.0 and t["copy_write"] == 1.0
+    k = t["kernels"]["k_trace_queue<false>"]
+    assert k["launches"] == 2 and k["ms"] == pytest.approx(3.0)
+    assert k["fetch_bytes"] == 20 * 32 + 200 * 64 + 60 * 128 and k["write_bytes"] == 2048
+    assert k["gbs"] == pytest.approx((k["fetch_bytes"] + 2048) / 3e-3 / 1e9)
+
+
+def test_roofline_fraction_is_of_measured_traffic():
+    """The fraction of the HBM peak comes from the profiled launches' traffic;
+    bytes that caches may have served (here 9 TB/s of them) are only listed."""
+    r = bench.roofline("k_x", "closest hit", 4e9, 1.0, 9e9, 1000.0, 8.0, 3.0, 1000.0, 10, False)
+    assert r["achieved"] == 4000.0 and r["frac"] == 0.5
+    assert r["queries"]["touched_gbs"] == 9000.0 and r["queries"]["launches"] == 10
+    r = bench.roofline("k_x", "closest hit", None, None, 9e9, 1000.0, 8.0, 3.0, 1000.0, 10, False)
+    assert r["achieved"] is None and r["frac"] is None
 
 
 def test_kernel_time_table(tmp_path):

@@ -50,13 +50,29 @@ SCENES = {
 }
 
 
+# paths of a pass against 2^17 (from the camera on in one launch), 2^18 (the
+# rest in one launch) and 2^24 (both queries of a bounce in one launch): the
+# least launches of closest-hit queries a plain render at the scene's depth
+# takes -- the camera rays', one per bounce, the last paths' -- says that its
+# paths went the intended way
+SIZES = {
+    (1, 1, 3): 1, (31, 1, 2): 1, (43, 33, 5): 1,
+    (362, 362, 1): 1, (363, 361, 1): 1,   # 131,044 and 131,043: from the camera on
+    (363, 362, 1): 2,                     # 131,406: from the first vertices on
+    (362, 362, 2): 2, (363, 361, 2): 2,   # 262,088 and 262,086
+    (513, 512, 2): 3,                     # 525,312: from a later bounce on
+    (1024, 768, 4): 4,                    # 3,145,728: after two bounces that claim chunks
+    (1024, 1024, 17): 5,                  # 17,825,792: the first bounce's queries apart
+}
+
+
 @pytest.mark.parametrize("name", sorted(SCENES))
-@pytest.mark.parametrize("size", [(1, 1, 3), (31, 1, 2), (43, 33, 5), (362, 362, 2), (363, 361, 2)],
-                         ids=lambda s: "%dx%dx%d" % s)
+@pytest.mark.parametrize("size", sorted(SIZES, key=lambda s: s[0] * s[1] * s[2]), ids=lambda s: "%dx%dx%d" % s)
 def test_paths_finished_in_one_launch_equal_the_bounce_by_bounce_ones(backend, name, size):
-    """A counting render goes bounce by bounce to the end; a plain one hands
-    the paths over when few are left, or from the camera on when its passes
-    are small (131,072 paths): same images and same ray counts."""
+    """A counting render goes bounce by bounce to the end, each query in a
+    launch of its own; a plain one traces both queries of a bounce in one
+    launch, and hands the paths over when few are left, or from the camera on
+    when its passes are small: same images and same ray counts."""
     W, H, spp = size
     d = SCENES[name]()
     d = dataclasses.replace(d, camera=dataclasses.replace(d.camera, width=W, height=H))
@@ -68,6 +84,11 @@ def test_paths_finished_in_one_launch_equal_the_bounce_by_bounce_ones(backend, n
             img, st = backend.render(spp=spp, seed=3, max_depth=depth, rr_depth=rr, spp_per_pass=per_pass)
             assert np.array_equal(img.view(np.uint32), ref.view(np.uint32)), (depth, rr, per_pass)
             assert st["closest_rays"] == rs["closest_rays"] and st["shadow_rays"] == rs["shadow_rays"]
+            if depth == d.max_depth and per_pass == 0:
+                print(name, size, "launches", st["launches_closest"], "rays per path",
+                      st["closest_rays"] / (W * H * spp), flush=True)
+                least = SIZES[size]
+                assert st["launches_closest"] == 1 if least == 1 else st["launches_closest"] >= least
 
 
 def test_traversal_counts_add_up_over_passes_and_images(backend):

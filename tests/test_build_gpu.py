@@ -3,6 +3,7 @@ change hands: one chunk and several (256 clusters), the last steps in one block
 (2048 clusters), chunks of more than 256 (beyond 2048 * 256 clusters), a
 frontier of several chunks, and degenerate inputs whose areas all tie."""
 import dataclasses
+import hashlib
 
 import numpy as np
 import pytest
@@ -78,3 +79,38 @@ def test_tree_structure(backend, kind, n, builder):
         bhi[parent[at, 0], parent[at, 1]] = bhi[at].max(axis=1)
     used = inner | leaf
     assert (lo.transpose(0, 2, 1)[used] <= blo[used]).all() and (hi.transpose(0, 2, 1)[used] >= bhi[used]).all()
+
+
+# SHA-256 (first 16 digits) of the exported nodes and triangles, PLOC and LBVH,
+# of the builders whose steps the host launched one by one with library scans
+# between them: fewer and larger launches leave every byte as it was.
+TREES = {
+    "soup-9": ("0c4a1dc73e0aa9d8", "18ba1b4e7e996ac3"),
+    "soup-255": ("4c08e36d1f0fba62", "ca0021fad5de6453"),
+    "soup-257": ("685b9e4603452a56", "75fa0e0e8b6003de"),
+    "soup-2048": ("b327bc6147fda240", "262c22878552a715"),
+    "soup-2049": ("421529b5f4997111", "ddab6fd3cdb1d2c7"),
+    "soup-70001": ("c670f20bdedaacb2", "853c65a496d8fcb3"),
+    "soup-524289": ("f1edc21f0cc43ede", "4dadf7eea0295b00"),
+    "same-3000": ("cfa0f083ca4491e5", "33ce0d44838c222f"),
+    "line-2500": ("67d339405b4521f5", "828f32602ca334b6"),
+    "sphere-8": ("0276451afcb8e95f", "08e188fd80ee6b6a"),
+    "sphere-37": ("b4321f7103d3b854", "d1c520ee51a1eb00"),
+    "sphere-200": ("20988c3307dcccff", "f27e261f7e5c5583"),
+    "sphere-1024": ("6f8b5b153eed15fe", "5c1bfa94b567bfc7"),
+    "zoo": ("5c172e9ced3fefc9", "3238c7d90a93664e"),
+}
+
+
+@pytest.mark.parametrize("name", sorted(TREES))
+def test_trees_are_byte_for_byte_the_same(backend, name):
+    kind, _, size = name.partition("-")
+    if kind == "sphere":
+        d = scenes.displaced_sphere(width=16, height=9, grid=int(size), glass_level=2, env_size=(8, 4))
+    else:
+        d = scenes.material_zoo() if kind == "zoo" else _scene(int(size), kind)[0]
+    for builder, want in zip((drawlab_amd.BUILD_GPU, drawlab_amd.BUILD_GPU_LBVH), TREES[name]):
+        backend.upload_scene(d)
+        backend.build_accel(builder)
+        nodes, tris = backend.accel_export()
+        assert hashlib.sha256(nodes.tobytes() + tris.tobytes()).hexdigest()[:16] == want, builder

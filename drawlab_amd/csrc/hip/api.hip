@@ -155,14 +155,13 @@ __global__ __launch_bounds__(256) void k_prim_recs(const float* __restrict__ pos
             const float* q = pos + 3 * (size_t)idx[3 * i + k];
             p[k] = v3(q[0], q[1], q[2]);
         }
-        const uint32_t m = prim_mesh[i];
-        const MeshRec& r = meshes[m];
+        const MeshRec& r = meshes[prim_mesh[i]];
         const dl_material_desc& md = mats[r.material];
         uint32_t flags = (r.has_normals ? kRecNormals : 0u) | (r.has_tangents ? kRecTangents : 0u) |
                          (r.has_texcoords ? kRecTexcoords : 0u);
         for (int k = 0; k < DL_TEX_SLOTS; k++) flags |= md.tex[k] ? kRecTextured : 0u;
         const vec3 nrm = normalized(cross(sub(p[1], p[0]), sub(p[2], p[0])));
-        recs[4 * i] = make_float4(p[0].x, p[0].y, p[0].z, __uint_as_float(m));
+        recs[4 * i] = make_float4(p[0].x, p[0].y, p[0].z, 0.0f);
         recs[4 * i + 1] = make_float4(p[1].x, p[1].y, p[1].z, __int_as_float(r.material));
         recs[4 * i + 2] = make_float4(p[2].x, p[2].y, p[2].z, __uint_as_float(flags));
         recs[4 * i + 3] = make_float4(nrm.x, nrm.y, nrm.z, __int_as_float(r.light));

@@ -75,10 +75,10 @@ struct MeshRec {
 };
 
 // What the shading kernels read of one primitive, 64 bytes in one cache line
-// (k_prim_recs gathers it at upload): the three vertices, and in the fourth
-// components the mesh, the material, the flags below and the area light (-1:
-// none); the last record also holds the face normal.
-//   r0 = p0, mesh   r1 = p1, material   r2 = p2, flags   r3 = normal, light
+// (k_prim_recs gathers it at upload): the three vertices and the face normal,
+// and in fourth components the material, the flags below and the area light
+// (-1: none).
+//   r0 = p0, 0   r1 = p1, material   r2 = p2, flags   r3 = normal, light
 // One gather of four 16-byte loads instead of about sixteen dependent ones
 // (mesh, mesh record, vertex indices, vertices).
 enum : uint32_t { kRecNormals = 1u, kRecTangents = 2u, kRecTexcoords = 4u, kRecTextured = 8u };

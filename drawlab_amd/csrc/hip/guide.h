@@ -45,7 +45,6 @@ __host__ __device__ __forceinline__ uint16_t f2bf(float f) {
     u += 0x7FFFu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
 }
-__device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
 // Training record layout (floats): position (normalised) 0..2, wo 3..5,
 // shading normal 6..8, roughness 9, sampled direction 10..12, sampling pdf

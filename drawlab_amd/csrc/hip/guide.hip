@@ -10,7 +10,7 @@
 //   forward     a wave takes 64 rows (two 32-row blocks); activations live
 //               in the wave's LDS rows (bfloat16, in place layer by layer);
 //               weights are read from global memory (43 KB, L2-resident) as
-//               B operands, 1 KB in a row per tile
+//               A operands, 1 KB in a row per tile
 //   training    one kernel per step for forward, loss and backward (16x16x32
 //               and 32x32x16 tiles): a block keeps its rows' activations in LDS
 //               and its share of dW in registers; per-block partial gradients are then summed in a
@@ -669,7 +669,7 @@ static_assert(kGuideBatch == dl_sizes::kGuideBatchRows && kScanTile == (int)dl_s
               "guided render sizes");
 static_assert(dl_sizes::kGuideNetBytes == 4ull * kGParams * sizeof(float) + 5 * 64 * sizeof(float) +
                                               3ull * 5 * kGWSlot * sizeof(uint16_t) +
-                                              (4 + kSumBlocks + dl_sizes::kGuideTrainBlocks) * sizeof(float),
+                                              (1 + kSumBlocks + dl_sizes::kGuideTrainBlocks) * sizeof(float),
               "guide_init allocations");
 static_assert(dl_sizes::kGuideTrainBytes == (uint64_t)kGuideBatch * (kGIn + 3 + 1) * sizeof(float) +
                                                 (uint64_t)dl_sizes::kGuideTrainBlocks * kGParams * sizeof(float),
@@ -686,7 +686,7 @@ struct GuideState {
     uint16_t *w = nullptr, *w16 = nullptr, *wt16 = nullptr;
     int step = 0;
     float lr = 1e-2f;
-    float* scalars = nullptr;  // [1]: the step's loss; then the partial sums of the weights, the blocks' losses
+    float* scalars = nullptr;  // the step's loss, the partial sums of the weights, the blocks' losses
     float* part = nullptr;     // per-block partial gradients of a training step
     std::vector<void*> allocs;
 };
@@ -739,9 +739,6 @@ void free_guide(Ctx* c) {
     c->guide = nullptr;
 }
 
-GuideState* guide_state(Ctx* c) { return (GuideState*)c->guide; }
-const float* guide_bias(GuideState* g) { return g->bias; }
-
 dl_status guide_init(Ctx* c, uint64_t seed, float lr, const float* params) {
     free_guide(c);
     GuideState* g = new GuideState();
@@ -755,7 +752,7 @@ dl_status guide_init(Ctx* c, uint64_t seed, float lr, const float* params) {
     DL_TRY(galloc(c, g, &g->w, 5 * kGWSlot));
     DL_TRY(galloc(c, g, &g->w16, 5 * kGWSlot));
     DL_TRY(galloc(c, g, &g->wt16, 5 * kGWSlot));
-    DL_TRY(galloc(c, g, &g->scalars, 4 + kSumBlocks + dl_sizes::kGuideTrainBlocks));
+    DL_TRY(galloc(c, g, &g->scalars, 1 + kSumBlocks + dl_sizes::kGuideTrainBlocks));
     std::vector<float> th;
     if (params)
         th.assign(params, params + kGParams);
@@ -790,14 +787,14 @@ dl_status guide_train(Ctx* c, const float* x, const float* dirs, const float* cw
     GuideState* g = (GuideState*)c->guide;
     if (!g->part) DL_TRY(galloc(c, g, &g->part, (size_t)dl_sizes::kGuideTrainBlocks * kGParams));
     const uint32_t blocks = dl_sizes::guide_train_blocks(n);
-    float* const sums = g->scalars + 4;
+    float* const sums = g->scalars + 1;
     float* const losses = sums + kSumBlocks;
     k_sum<<<kSumBlocks, 256, 0, c->stream>>>(cw, n, sums);
     k_train<<<blocks, kTrainWaves * 64, 0, c->stream>>>(net_of(g), x, dirs, cw, n, sums, g->part, losses);
     if (apply) g->step++;
     AdamArgs a{g->theta, g->m, g->v, g->grad, g->lr, 1.0f - std::pow(0.9f, (float)g->step),
                1.0f - std::pow(0.999f, (float)g->step), apply ? 1 : 0, g->w, g->w16, g->wt16, g->bias};
-    k_train_reduce<<<(kGParams + 63) / 64, 256, 0, c->stream>>>(g->part, blocks, a, losses, g->scalars + 1);
+    k_train_reduce<<<(kGParams + 63) / 64, 256, 0, c->stream>>>(g->part, blocks, a, losses, g->scalars);
     DL_HIP_CHECK(c, hipGetLastError());
     return DL_OK;
 }
@@ -910,7 +907,7 @@ dl_status dl_hip_guide_train_step(void* h, const float* x, const float* dirs, co
     if (n == 0) return set_error(c, DL_ERR_INVALID, "empty batch");
     (void)hipSetDevice(c->device);
     DL_TRY(guide_train(c, x, dirs, weights, n, apply != 0));
-    if (loss) DL_HIP_CHECK(c, hipMemcpyAsync(loss, g->scalars + 1, sizeof(float), hipMemcpyDeviceToHost, c->stream));
+    if (loss) DL_HIP_CHECK(c, hipMemcpyAsync(loss, g->scalars, sizeof(float), hipMemcpyDeviceToHost, c->stream));
     DL_HIP_CHECK(c, hipStreamSynchronize(c->stream));
     return DL_OK;
 }

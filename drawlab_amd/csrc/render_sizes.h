@@ -41,9 +41,9 @@ constexpr int kGuideParams = 21808;
 constexpr int kGuideWSlot = 64 * 96;            // bfloat16 elements per layer copy
 
 // network parameters, Adam moments, gradient, biases, bfloat16 copies
-// (W in two orders, W^T), scalars and partial sums
+// (W in two orders, W^T), the step's loss and the partial sums
 constexpr uint64_t kGuideNetBytes = 4ull * kGuideParams * 4 + 5 * 64 * 4 + 3ull * 5 * kGuideWSlot * 2 +
-                                    (4 + kGuideSumBlocks + kGuideTrainBlocks) * 4;
+                                    (1 + kGuideSumBlocks + kGuideTrainBlocks) * 4;
 // one training batch: its features (96), directions (3) and weights (1); the
 // blocks' partial gradients
 constexpr uint64_t kGuideTrainBytes =

@@ -12,10 +12,15 @@
 //   loop:
 //     shade         per path, material-sorted: emitter sampling (NEE) with
 //                   a shadow ray, BSDF sampling, continuation ray
-//     trace_closest + trace_shadow
-//     post          NEE resolution, emitter hit with MIS, miss with the
-//                   environment, Russian roulette, depth cap; survivors are
-//                   appended to the next material queues
+//     trace_closest + trace_shadow (one launch for bounces of at most
+//                   kBothPaths paths); an unoccluded shadow ray adds its
+//                   emitter sample to the path's radiance
+//     post          miss with the environment, Russian roulette, depth cap;
+//                   survivors are appended to the next material queues,
+//                   emitter hits to post_emit's
+//     post_emit     MIS-weighted emission of the emitter hits
+//   finish          takes over from the loop once few paths are left, or from
+//                   the camera rays on in a small pass
 //   film            deterministic gather of the pass's samples through the
 //                   reconstruction filter (ImageBlock::put, block.cpp:81-113)
 //
@@ -790,8 +795,6 @@ __global__ __launch_bounds__(kStageBlock) void k_shade(PassParams pp, SceneView 
     }
 }
 
-// NEE resolution, emitter hit / miss with MIS, Russian roulette
-// (path.cpp:46-56, 71-97; miss.cu:31-42).
 // A continuation that hit an area light: its MIS-weighted emission
 // (path.cpp:72-84) is added by k_post_emit, after the rest of k_post, from
 // the throughput before Russian roulette, kept in the path's NEE slot (the
@@ -844,6 +847,7 @@ __global__ __launch_bounds__(kStageBlock) void k_post_emit(PassParams pp, SceneV
 // hits one collects its emission as usual, unless it is still the camera
 // ray, and passes through (queue kPassQ) without a bounce; a camera ray that
 // passed through is treated as the camera ray at its next hit or miss.
+// (path.cpp:71-97; miss.cu:31-42)
 template <bool HIDE>
 __global__ __launch_bounds__(kStageBlock) void k_post(PassParams pp, SceneView s, RenderBufs rs, int next, int depth,
                                                       float* __restrict__ grec) {
@@ -996,10 +1000,12 @@ constexpr uint32_t kFinishPaths = 1u << 18, kFinishCamera = 1u << 17;
 // at most 0.99^3072 = 4e-14 of the paths that long.
 constexpr int kFinishRoulette = 1024;
 constexpr int kFinishBounces = 4096;
-// Bounces of at most this many paths trace both queries in one launch (the
-// 1080p frame takes 5.43, 5.22 and 5.04 ms with 2^20, 2^22 and 2^24, the
-// 64-spp sphere 67.3, 66.6 and 65.8); larger ones keep a launch and a time of
-// their own for each.
+// Bounces of at most this many paths trace both queries in one launch, whose
+// waves end together instead of twice (the 1080p frame takes 5.43, 5.22 and
+// 5.04 ms with 2^20, 2^22 and 2^24, the 64-spp sphere 67.3, 66.6 and 65.8).
+// In larger ones the tail no longer counts: against 2^24, 2^26 takes 0.996 of
+// the sphere's time and no limit at all 1.012, with 1.5 to 3 % between runs
+// of one side, and the 256-spp frame runs at 2362, 2401 and 2333 Mpaths/s.
 constexpr uint32_t kBothPaths = 1u << 24;
 
 // A vertex's results in registers.

@@ -19,8 +19,8 @@ struct BatchIO {
     uint32_t *__restrict__ cn, *__restrict__ ct;
     uint8_t* __restrict__ occ;
     // (4.19M diffuse-bounce rays against 2M triangles take 0.821, 0.801 and
-    // 0.782 ms with 4, 8 and 16; 1M shadow rays against 0.5M triangles 242 us
-    // with 1, 4 or 8)
+    // 0.782 ms with 4, 8 and 16; 1M shadow rays against 0.5M triangles the same
+    // with 1, 4 and 8)
     static constexpr uint32_t kRefillMin = 16, kRefillMinAny = 8;
     __device__ __forceinline__ uint32_t entry(uint32_t slot) const { return slot; }
     __device__ __forceinline__ void load(uint32_t i, vec3& o, vec3& d, float& tmin, float& tmax) const {
@@ -89,8 +89,8 @@ int batch_trace_blocks_per_cu(bool counting) {
 
 __global__ void k_zero_work(uint32_t* w) { w[threadIdx.x * kWorkStride] = 0; }
 
-// Lanes of a persistent grid step through ray indices by the grid size; a
-// 32-bit index must not wrap past n.
+// Ray indices are 32-bit, and the waves that find nothing left to claim ask for
+// chunks beyond n: for less than 2^20 rays (2^13 waves, chunks of 64).
 constexpr uint32_t kMaxBatchRays = 1u << 31;
 
 // Blocks that trace n rays: a few rays per wave until every block of the
@@ -156,7 +156,7 @@ dl_status launch_trace_shadow(Ctx* c, const float* rays, uint32_t n, uint8_t* oc
 
 // ---- allocation-free closest hits (dl_hip_trace_closest_noalloc) ---------
 // The closest-hit traversal's scratch -- the per-lane stack overflow of a
-// persistent grid of kNoAllocBlocks blocks, then its work counter -- in a
+// persistent grid of kNoAllocBlocks blocks, then its work counters -- in a
 // static array that each device holds until the process ends (92.3 MB)
 // instead of the context's buffers.  Host code never passes the array's
 // name to a kernel: it stands for a host-side shadow there.  Its device

@@ -259,7 +259,7 @@ dl_status dl_hip_trace_shadow(void* ctx, const float* rays, uint32_t n, uint8_t*
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): dl_hip_trace_closest with the traversal's scratch (the
  * stack overflow of a fixed persistent grid of 1024 blocks and its work
- * counter) in a static per-device array of 92.3 MB, held until the process
+ * counters) in a static per-device array of 92.3 MB, held until the process
  * ends, instead of the context's buffers.  The call allocates nothing;
  * inputs and outputs are the caller's device pointers, as for
  * dl_hip_trace_closest, and the results are identical.  n is at most 2^31

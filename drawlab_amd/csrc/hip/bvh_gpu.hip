@@ -355,9 +355,9 @@ dl_status read_slots(Ctx* c, const uint32_t* red, uint32_t* depth, uint32_t* lea
 // Scratch arrays of a build: want() names them, alloc() lays them out in the
 // context's kept build scratch.  (A hipMalloc and hipFree per array, 27 of
 // each, cost more than a build's kernels: 18 ms of a build of 2,097,152
-// triangles were 5 ms of kernels.  One allocation per build instead made a
-// context's first build 5.5 ms and a repeated one 19, after half a gigabyte had
-// been given back.  So it is kept, see kBuildKeepBytes: 3.0 ms.)
+// triangles and a query were 5 ms of kernels.  With one allocation, given back
+// after every build, it takes 3.7 ms; kept for the next one, see
+// kBuildKeepBytes, 2.9.  A process's first build also loads the kernels: 12 ms.)
 struct Scratch {
     Ctx* c;
     size_t bytes = 0;
